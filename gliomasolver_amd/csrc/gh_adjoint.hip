@@ -49,12 +49,16 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     // forward sweep with checkpoints every K steps; two steps per launch from
     // a clamped state (k >= 1) when no checkpoint falls in between
     const bool pairs = c.fast_ok && c.topo.uniform_bpd > 0;
+    // the two-step schedule (tile 0) leaves out the groups of blocks without
+    // diffusion that u_1 leaves at zero, in both directions
+    const bool skip = pairs && c.rd_bpw == 0 && c.nGrp > 0;
     for (int64_t k = 0; k < N;) {
+        if (k == 1 && skip && (rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p))) return rc;
         if (k % K == 0)
             GH_HIP_CHECK(hipMemcpyAsync(ck + (size_t)(k / K) * nb, c.phi[c.cur].p, nb, hipMemcpyDeviceToDevice,
                                         c.stream));
         if (pairs && k >= 1 && k + 2 <= N && (k + 1) % K != 0) {
-            if ((rc = rd_step2_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, nullptr, dt))) return rc;
+            if ((rc = rd_step2_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, nullptr, dt, skip))) return rc;
             k += 2;
         } else {
             if ((rc = rd_step_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt))) return rc;
@@ -71,10 +75,13 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     hipLaunchKernelGGL(adj_mask_kernel<Real>, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, c.stream, nc,
                        c.adjLam[lc].as<double>(), (const Real*)c.phi[c.cur].p);
     GH_HIP_CHECK(hipGetLastError());
+    const bool still = skip && N > 1;  // (marked before step 1)
+    if (still) {  // what the launches leave out: zero states, the seed in both adjoint buffers
+        if ((rc = rd_zero_still(c, seg, K + 1))) return rc;
+        GH_HIP_CHECK(hipMemcpyAsync(c.adjLam[1 - lc].p, c.adjLam[lc].p, nc * 8, hipMemcpyDeviceToDevice, c.stream));
+    }
     // reverse sweep
     const int ns = c.topo.nblocks();
-    const int per_xcd = (ns + 7) / 8;
-    const unsigned grid = 8 * per_xcd;
     if ((rc = c.adjPart.ensure(sizeof(double) * ADJ_PART * ns))) return rc;
     GH_HIP_CHECK(hipMemsetAsync(c.adjPart.p, 0, sizeof(double) * ADJ_PART * ns, c.stream));
     const double h = block_h_of(c);
@@ -82,15 +89,17 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     const UniformAdjParams prm{c.rho, ih2, dt, 1.0 / (double)N, 1.0 / c.Dw, c.topo.uniform_bpd,
                                 bpd_magic(c.topo.uniform_bpd)};
     // blocks without diffusion take the reverse step's short path under the
-    // two-step schedule (tile 0), whose plan holds their flags
-    const unsigned char* zflux = (c.nItems2f > 0 && c.rd_bpw == 0) ? c.zeroFlux.as<unsigned char>() : nullptr;
+    // two-step schedule (tile 0); step 0 reads the caller's state and leaves
+    // nothing out
+    const StepWork all = c.rd_bpw == 0 ? rd_step_work(c, false) : step_work(ns, nullptr, 0, nullptr, nullptr);
+    const StepWork moving = still ? rd_step_work(c, true) : all;
     for (int64_t sgi = nck - 1; sgi >= 0; --sgi) {
         const int64_t k0 = sgi * K, k1 = std::min<int64_t>(N, k0 + K);
         GH_HIP_CHECK(hipMemcpyAsync(seg, ck + (size_t)sgi * nb, nb, hipMemcpyDeviceToDevice, c.stream));
         for (int64_t j = 0; j < k1 - k0;) {  // the segment's states, pairs from clamped states
             if (pairs && k0 + j >= 1 && j + 2 <= k1 - k0) {
                 if ((rc = rd_step2_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 2) * nb,
-                                           seg + (size_t)(j + 1) * nb, dt)))
+                                           seg + (size_t)(j + 1) * nb, dt, still)))
                     return rc;
                 j += 2;
             } else {
@@ -101,16 +110,16 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
         for (int64_t k = k1 - 1; k >= k0; --k) {
             const Real* uk = (const Real*)(seg + (size_t)(k - k0) * nb);
             const int mask_out = k >= 1;
+            const StepWork& wk = k >= 1 ? moving : all;
             if (c.fast_ok && k >= 1)  // u_k is a clamped state: the clamped-state records
-                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams, true>), dim3(grid), dim3(512), 0,
-                                   c.stream, ns, per_xcd, uk, mask_out, c.adjLam[lc].as<double>(),
+                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams, true>), dim3(wk.grid()), dim3(512), 0,
+                                   c.stream, wk, uk, mask_out, c.adjLam[lc].as<double>(),
                                    c.adjLam[1 - lc].as<double>(), c.statF.as<Stat4<Real>>(), (const Real*)nullptr,
-                                   prm, c.adjPart.as<double>(), zflux);
+                                   prm, c.adjPart.as<double>());
             else
-                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams>), dim3(grid), dim3(512), 0, c.stream,
-                                   ns, per_xcd, uk, mask_out, c.adjLam[lc].as<double>(), c.adjLam[1 - lc].as<double>(),
-                                   c.statD.as<Stat4<Real>>(), c.statSig.as<Real>(), prm, c.adjPart.as<double>(),
-                                   zflux);
+                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams>), dim3(wk.grid()), dim3(512), 0, c.stream,
+                                   wk, uk, mask_out, c.adjLam[lc].as<double>(), c.adjLam[1 - lc].as<double>(),
+                                   c.statD.as<Stat4<Real>>(), c.statSig.as<Real>(), prm, c.adjPart.as<double>());
             GH_HIP_CHECK(hipGetLastError());
             lc = 1 - lc;
         }

@@ -90,6 +90,7 @@ template <typename Real>
 struct AdjJob {
     const Real* u;        // final state (seed) or initial state (IC gradient)
     double* lam;          // the sample's adjoint range
+    double* lam2;         // the same range of the other buffer, or null
     const unsigned char* t1;
     const unsigned char* fl;
     const double* pet;
@@ -113,7 +114,9 @@ template <typename Real>
 __global__ __launch_bounds__(256) void batch_mask_kernel(const AdjJob<Real>* __restrict__ jobs) {
     const AdjJob<Real>& j = jobs[blockIdx.y];
     const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < j.ncells) adj_mask_cell(c, j.lam, j.u);
+    if (c >= j.ncells) return;
+    adj_mask_cell(c, j.lam, j.u);
+    if (j.lam2) j.lam2[c] = j.lam[c];  // still groups are left out by every launch
 }
 
 template <typename Real>
@@ -253,7 +256,18 @@ struct Batch {
     DevBuf phi[2], statD, statSig, nbr, slotPos, range, apw, apg, likPart, likOut, likJobs;
     DevBuf statF, flag;  // rd_step2f_kernel records (valid iff fast_ok), count scratch
     bool fast_ok = false;
-    DevBuf zeroFlux;                 // per slot: 1 = block without diffusion (zero_flux_kernel)
+    DevBuf zeroFlux;                 // per slot: != 0 a block without diffusion (zero_flux_kernel)
+    // StepWork lists of all slots and their lengths per count of positions (index p: positions 0..p)
+    DevBuf fullList, grpList, stillGrp;
+    std::vector<int> nFull, nGrp;
+    bool skip_still = false;  // stillGrp holds the marks of the current states
+    // the work of the slots of positions [0, active)
+    StepWork work(int active) const {
+        const int p = active - 1;
+        if (nGrp.empty() || nGrp.back() == 0) return step_work((int)slot0[active], nullptr, 0, nullptr, nullptr);
+        return step_work(nFull[p], fullList.as<int32_t>(), nGrp[p], grpList.as<int2>(),
+                         skip_still ? stillGrp.as<unsigned char>() : nullptr);
+    }
     DevBuf ck, tape, lam[2], apart, icpart, adjJobs;  // adjoint
     double ic_is2 = 1.0;                                 // adjoint: 1 / sigma^2 of the Gaussian IC
     std::vector<int> final_buf;                          // per position: phi buffer of the final state
@@ -355,12 +369,33 @@ int build_layout_t(Batch& b) {
     if ((rc = build_stat_fast(b.stream, sizeof(Real) == 4 ? GH_REAL_F32 : GH_REAL_F64, nc, b.statD.p, b.statSig.p,
                               b.statF, b.flag, &b.fast_ok)))
         return rc;
+    b.nFull.clear();
+    b.nGrp.clear();
+    b.skip_still = false;
     if (b.fast_ok && nsl > 0) {  // blocks without diffusion
         if ((rc = b.zeroFlux.ensure_grow(nsl))) return rc;
         const BatchStepParams<Real> prm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
         hipLaunchKernelGGL((zero_flux_kernel<Real, BatchStepParams<Real>>), dim3((unsigned)nsl), dim3(256), 0,
                            b.stream, (int)nsl, b.statF.as<Stat4<Real>>(), prm, b.zeroFlux.as<unsigned char>());
         GH_HIP_CHECK(hipGetLastError());
+        std::vector<unsigned char> z(nsl);
+        GH_HIP_CHECK(hipMemcpyAsync(z.data(), b.zeroFlux.p, nsl, hipMemcpyDeviceToHost, b.stream));
+        GH_HIP_CHECK(hipStreamSynchronize(b.stream));
+        std::vector<int32_t> full;
+        std::vector<int2> grp;
+        const std::vector<size_t> cut(b.slot0.begin() + 1, b.slot0.end());
+        build_step_work(z.data(), cut, full, grp, &b.nFull, &b.nGrp);
+        if (!grp.empty()) {
+            if ((rc = b.fullList.ensure_grow(std::max<size_t>(1, full.size()) * sizeof(int32_t))) ||
+                (rc = b.grpList.ensure_grow(grp.size() * sizeof(int2))) || (rc = b.stillGrp.ensure_grow(grp.size())))
+                return rc;
+            if (!full.empty())
+                GH_HIP_CHECK(hipMemcpyAsync(b.fullList.p, full.data(), full.size() * sizeof(int32_t),
+                                            hipMemcpyHostToDevice, b.stream));
+            GH_HIP_CHECK(hipMemcpyAsync(b.grpList.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice,
+                                        b.stream));
+            GH_HIP_CHECK(hipStreamSynchronize(b.stream));  // the lists are read by the copies
+        }
     }
     GH_HIP_CHECK(hipMemsetAsync(b.phi[0].p, 0, nc * sizeof(Real), b.stream));
     GH_HIP_CHECK(hipStreamSynchronize(b.stream));
@@ -496,6 +531,16 @@ struct ForwardSweep {
         active = ns;
         b.final_buf.assign(ns, 0);
     }
+    // marks the groups that the initial states leave at zero for good
+    int mark() {
+        if (b.nGrp.empty() || b.nGrp.back() == 0) return GH_OK;
+        hipLaunchKernelGGL(still_kernel<Real>, dim3(b.nGrp.back()), dim3(256), 0, b.stream, b.nGrp.back(),
+                           b.grpList.as<int2>(), b.zeroFlux.as<unsigned char>(), b.phi[cur].as<Real>(),
+                           b.phi[1 - cur].as<Real>(), b.stillGrp.as<unsigned char>());
+        GH_HIP_CHECK(hipGetLastError());
+        b.skip_still = true;
+        return GH_OK;
+    }
     // retire the samples that have reached step k
     void retire(int64_t k) {
         while (active > 0 && npos[active - 1] <= k) b.final_buf[--active] = cur;
@@ -510,10 +555,10 @@ struct ForwardSweep {
         Real* out = b.phi[1 - cur].as<Real>();
         if (two) {
             const int per_xcd = (nsl + 7) / 8;
+            const StepWork wk = b.work(active);
             if (b.fast_ok)
-                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
-                                   b.stream, even_split(nsl), (const int2*)nullptr, in, out, (Real*)nullptr,
-                                   b.statF.as<Stat4<Real>>(), b.zeroFlux.as<unsigned char>(), prm);
+                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(wk.grid()), dim3(512), 0,
+                                   b.stream, wk, in, out, (Real*)nullptr, b.statF.as<Stat4<Real>>(), prm);
             else
                 hipLaunchKernelGGL((rd_step2_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
                                    b.stream, nsl, per_xcd, in, out, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
@@ -534,6 +579,7 @@ int run_t(Batch& b, double* elapsed_ms) {
     ForwardSweep<Real> fw(b);
     const int64_t maxsteps = fw.npos.empty() ? 0 : fw.npos[0];
     GH_HIP_CHECK(hipEventRecord(b.ev0, b.stream));
+    if (int rc = fw.mark()) return rc;
     int64_t k = 0;
     while (true) {
         fw.retire(k);
@@ -625,8 +671,6 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         return rc;
     const BatchStepParams<Real> fprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
-    // blocks without diffusion take the reverse step's short path (flags exist when fast_ok)
-    const unsigned char* zflux = b.fast_ok ? b.zeroFlux.as<unsigned char>() : nullptr;
     auto step = [&](const void* in, void* out, int nslots) {  // one Euler step (tape recompute)
         const int per_xcd = ((nslots + 1) / 2 + 7) / 8;
         hipLaunchKernelGGL((rd_step_kernel<Real, true, 2, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
@@ -638,6 +682,7 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     GH_HIP_CHECK(hipEventRecord(b.ev0, b.stream));
     // forward, with a checkpoint of the running samples every K steps
     ForwardSweep<Real> fw(b);
+    if ((rc = fw.mark())) return rc;
     for (int64_t k = 0;;) {
         fw.retire(k);
         if (k >= Nmax) break;
@@ -660,6 +705,8 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         LikParams lp;
         if ((rc = check_params(lik + 5 * i, stepPET, stepTi, lp))) return rc;
         jobs[p] = AdjJob<Real>{final_phi<Real>(b, p), b.lam[b.smp[i].nsteps & 1].as<double>() + b.slot0[p] * BCELLS,
+                               b.skip_still ? b.lam[1 - (b.smp[i].nsteps & 1)].as<double>() + b.slot0[p] * BCELLS
+                                            : nullptr,
                                a.t1.as<unsigned char>(), a.fl.as<unsigned char>(), a.pet.as<double>(),
                                a.nslots * BCELLS, a.bpd, lp, 0, 0, 0, 0};
         maxc = std::max(maxc, a.nslots * BCELLS);
@@ -686,6 +733,11 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     GH_HIP_CHECK(hipGetLastError());
     // reverse
     GH_HIP_CHECK(hipMemsetAsync(b.apart.p, 0, ADJ_PART * nsl * 8, b.stream));
+    if (b.skip_still) {  // the tape's zeros that no launch writes
+        hipLaunchKernelGGL(still_zero_kernel<Real>, dim3(b.nGrp.back(), K + 1), dim3(256), 0, b.stream, b.nGrp.back(),
+                           b.grpList.as<int2>(), b.stillGrp.as<unsigned char>(), b.tape.as<Real>(), nc);
+        GH_HIP_CHECK(hipGetLastError());
+    }
     for (int64_t j = J - 1; j >= 0; --j) {
         const int64_t k0 = j * K, k1 = std::min<int64_t>(Nmax, k0 + K);
         GH_HIP_CHECK(hipMemcpyAsync(tape, ck + ckoff[j] * slot_bytes, b.slot0[active(k0)] * slot_bytes,
@@ -698,11 +750,10 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
             char* in = tape + (size_t)(k - k0) * nsl * slot_bytes;
             const int nslots = (int)b.slot0[active(k)];
             if (b.fast_ok && k >= 1 && k + 2 <= k1) {
-                const int per_xcd = (nslots + 7) / 8;
-                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
-                                   b.stream, even_split(nslots), (const int2*)nullptr, (const Real*)in,
-                                   (Real*)(in + 2 * (size_t)nsl * slot_bytes), (Real*)(in + (size_t)nsl * slot_bytes),
-                                   b.statF.as<Stat4<Real>>(), b.zeroFlux.as<unsigned char>(), fprm);
+                const StepWork wk = b.work(active(k));
+                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(wk.grid()), dim3(512), 0,
+                                   b.stream, wk, (const Real*)in, (Real*)(in + 2 * (size_t)nsl * slot_bytes),
+                                   (Real*)(in + (size_t)nsl * slot_bytes), b.statF.as<Stat4<Real>>(), fprm);
                 k += 2;
             } else {
                 step(in, in + (size_t)nsl * slot_bytes, nslots);
@@ -710,22 +761,22 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
             }
         }
         for (int64_t k = k1 - 1; k >= k0; --k) {
-            const int nslots = (int)b.slot0[active(k)];
-            const int per_xcd = (nslots + 7) / 8;
+            StepWork wk = b.work(active(k));
+            if (k == 0) wk.still = nullptr;  // u_0 is the given state
             const Real* uk = (const Real*)(tape + (size_t)(k - k0) * nsl * slot_bytes);
             const int mask_out = k >= 1;
             if (b.fast_ok && k >= 1)  // clamped states: the clamped-state records
-                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>, true>), dim3(8 * per_xcd), dim3(512),
-                                   0, b.stream, nslots, per_xcd, uk, mask_out,
+                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>, true>), dim3(wk.grid()), dim3(512),
+                                   0, b.stream, wk, uk, mask_out,
                                    b.lam[(k + 1) & 1].as<double>(),
                                    b.lam[k & 1].as<double>(), b.statF.as<Stat4<Real>>(), (const Real*)nullptr, aprm,
-                                   b.apart.as<double>(), zflux);
+                                   b.apart.as<double>());
             else
-                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
-                                   b.stream, nslots, per_xcd, uk, mask_out,
+                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>>), dim3(wk.grid()), dim3(512), 0,
+                                   b.stream, wk, uk, mask_out,
                                    b.lam[(k + 1) & 1].as<double>(),
                                    b.lam[k & 1].as<double>(), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(), aprm,
-                                   b.apart.as<double>(), zflux);
+                                   b.apart.as<double>());
         }
         GH_HIP_CHECK(hipGetLastError());
     }
@@ -808,7 +859,8 @@ int gh_batch_destroy(gh_batch* bh) {
     }
     DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->nbr,    &b->slotPos, &b->range,
                       &b->apw,    &b->apg,    &b->likPart, &b->likOut, &b->likJobs, &b->ck,     &b->tape,
-                      &b->lam[0], &b->lam[1], &b->apart,   &b->icpart, &b->adjJobs, &b->statF,  &b->flag};
+                      &b->lam[0], &b->lam[1], &b->apart,   &b->icpart, &b->adjJobs, &b->statF,  &b->flag,
+                      &b->zeroFlux, &b->fullList, &b->grpList, &b->stillGrp};
     for (DevBuf* d : bufs) d->release();
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);

@@ -142,9 +142,11 @@ struct Ctx {
     bool fast_ok = false;  // every cell has p_w + p_g >= 0: clamped states may take rd_step2f_kernel
     DevBuf zeroFlux;       // per slot: 1 = block without diffusion (zero_flux_kernel), uniform grids
     int nZeroFlux = 0;     // blocks without diffusion
-    DevBuf items2f;        // rd_step2f_kernel's work items {slot, blocks without diffusion} (plan_step2f)
-    int nItems2f = 0;      // 0: one item per slot
-    int split2f[9] = {0};  // per-XCD item ranges, balanced by estimated cost
+    // work list of the two-step and reverse-step kernels (StepWork, plan_step2f):
+    // slots of the blocks with diffusion, groups of blocks without (nGrp = 0:
+    // every slot an item), and per group whether a solve leaves it at zero
+    DevBuf fullList, grpList, stillGrp;
+    int nFull = 0, nGrp = 0;
     DevBuf nbr;         // 6 * nblocks int32
     std::vector<DevBuf> ckpt;  // device-side copies of phi (gh_checkpoint_*)
     std::vector<uint64_t> ckptVersion;  // tree_version each checkpoint was saved on
@@ -185,7 +187,17 @@ int rd_steps(Ctx& c, int64_t nsteps, double dt);
 int rd_step_buffers(Ctx& c, const void* in, void* out, double dt);
 // two fused steps from a clamped state (every value >= +0, as written by the
 // fused update) when c.fast_ok; mid (may be null) gets the state in between
-int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt);
+// skip_still: leave out the groups that rd_mark_still marked, whose zeros
+// stand in out and mid
+int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool skip_still = false);
+// marks the groups of blocks without diffusion that the clamped state `in`
+// leaves at zero for good, and writes their zeros into out
+int rd_mark_still(Ctx& c, const void* in, void* out);
+// the marked groups' zeros in n states, one after another from `states` on
+int rd_zero_still(Ctx& c, void* states, int n);
+// the work list of the current constants
+struct StepWork;
+StepWork rd_step_work(const Ctx& c, bool skip_still);
 double block_h_of(const Ctx& c);
 // the rd_step2f_kernel records of n cells from {D+, tau} and sigma into out;
 // *ok = every cell has sigma <= 0 (p_w + p_g >= 0).  Synchronizes the stream.

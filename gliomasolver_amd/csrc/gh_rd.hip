@@ -68,22 +68,21 @@ __global__ __launch_bounds__(256) void rd_update_kernel(size_t nc, Real* __restr
     phi[i] = rd_update(phi[i], dphidt[i], dt);
 }
 
+constexpr int64_t kStillMinSteps = 9;  // shortest call that marks the still groups
+
 inline double block_h(const Ctx& c) {
     // info.h[0] = 2^-level / 8 as Real (MRAGrid.inl:200-206); exact in float
     return std::ldexp(1.0, -c.topo.blocks[0].level) / BS;
 }
 
-// Work items of rd_step2f_kernel on a uniform grid: each block with diffusion
-// is an item; runs of consecutive blocks without diffusion (zero_flux_kernel)
-// are items of up to ZF_GROUP blocks, so those workgroups keep several blocks'
-// loads in flight.  The eight XCDs get contiguous item ranges (halos stay in
-// one L2) of equal estimated cost: a full block 1, a block without diffusion
-// kZeroFluxCost.
+// The work list of the two-step and reverse-step kernels on a uniform grid
+// (StepWork): zero_flux_kernel's flags decide.
 template <typename Real>
 int plan_step2f(Ctx& c) {
     const int ns = c.topo.nblocks();
     c.nZeroFlux = 0;
-    c.nItems2f = 0;
+    c.nFull = ns;
+    c.nGrp = 0;
     if (!c.fast_ok || c.topo.uniform_bpd <= 0 || ns == 0) return GH_OK;
     int rc;
     if ((rc = c.zeroFlux.ensure_grow(ns))) return rc;
@@ -94,45 +93,32 @@ int plan_step2f(Ctx& c) {
     std::vector<unsigned char> z(ns);
     GH_HIP_CHECK(hipMemcpyAsync(z.data(), c.zeroFlux.p, ns, hipMemcpyDeviceToHost, c.stream));
     GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    std::vector<int2> items;
-    std::vector<double> cost;
-    for (int s = 0; s < ns;) {
-        if (!z[s]) {
-            items.push_back(make_int2(s, 0));
-            cost.push_back(1.0);
-            ++s;
-            continue;
-        }
-        int k = 0;
-        while (s + k < ns && z[s + k] && k < ZF_GROUP) ++k;
-        items.push_back(make_int2(s, k));
-        cost.push_back(kZeroFluxCost * k);
-        c.nZeroFlux += k;
-        s += k;
-    }
-    const int ni = (int)items.size();
-    double total = 0;
-    for (double v : cost) total += v;
-    // split point x: the first item whose prefix cost reaches x/8 of the total
-    double acc = 0;
-    int x = 1;
-    c.split2f[0] = 0;
-    for (int i = 0; i < ni && x < 8; ++i) {
-        acc += cost[i];
-        while (x < 8 && acc >= total * x / 8) c.split2f[x++] = i + 1;
-    }
-    for (; x <= 8; ++x) c.split2f[x] = ni;
-    // within each XCD's range the blocks with diffusion go first (in slot
-    // order, so neighbouring blocks still run close in time) and the short
-    // groups of blocks without diffusion last, where they fill the tail
-    for (int r = 0; r < 8; ++r)
-        std::stable_partition(items.begin() + c.split2f[r], items.begin() + c.split2f[r + 1],
-                              [](const int2& v) { return v.y == 0; });
-    if ((rc = c.items2f.ensure_grow((size_t)ni * sizeof(int2)))) return rc;
-    GH_HIP_CHECK(hipMemcpyAsync(c.items2f.p, items.data(), (size_t)ni * sizeof(int2), hipMemcpyHostToDevice,
-                                c.stream));
+    std::vector<int32_t> full;
+    std::vector<int2> grp;
+    build_step_work(z.data(), {(size_t)ns}, full, grp, nullptr, nullptr);
+    for (const int2& g : grp) c.nZeroFlux += g.y;
+    if (grp.empty()) return GH_OK;  // item i is slot i
+    if ((rc = c.fullList.ensure_grow(std::max<size_t>(1, full.size()) * sizeof(int32_t))) ||
+        (rc = c.grpList.ensure_grow(grp.size() * sizeof(int2))) || (rc = c.stillGrp.ensure_grow(grp.size())))
+        return rc;
+    if (!full.empty())
+        GH_HIP_CHECK(hipMemcpyAsync(c.fullList.p, full.data(), full.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                                    c.stream));
+    GH_HIP_CHECK(hipMemcpyAsync(c.grpList.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice, c.stream));
     GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    c.nItems2f = ni;
+    c.nFull = (int)full.size();
+    c.nGrp = (int)grp.size();
+    return GH_OK;
+}
+
+// marks the still groups from the state in `in` (clamped: written by the fused
+// update) and writes their zeros into `out`
+template <typename Real>
+int mark_still(Ctx& c, const Real* in, Real* out) {
+    if (c.nGrp == 0) return GH_OK;
+    hipLaunchKernelGGL(still_kernel<Real>, dim3(c.nGrp), dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
+                       c.zeroFlux.as<unsigned char>(), in, out, c.stillGrp.as<unsigned char>());
+    GH_HIP_CHECK(hipGetLastError());
     return GH_OK;
 }
 
@@ -184,25 +170,16 @@ int launch_step2(Ctx& c, const Real* in, Real* out, double dt) {
 }
 
 // two fused steps per launch on a clamped state (rd_step2f_kernel); mid, when
-// not null, receives the state after the first step
+// not null, receives the state after the first step; skip_still: the still
+// groups are marked and their zeros stand in out (and mid)
 template <typename Real>
-int launch_step2f(Ctx& c, const Real* in, Real* out, double dt, Real* mid = nullptr) {
-    const int ns = c.topo.nblocks();
-    const int per_xcd = (ns + 7) / 8;
+int launch_step2f(Ctx& c, const Real* in, Real* out, double dt, bool skip_still, Real* mid = nullptr) {
     const double h = block_h(c);
     const double ih2 = 1. / (h * h);
     const UniformStepParams<Real> prm{(Real)c.rho, ih2, dt, c.topo.uniform_bpd, bpd_magic(c.topo.uniform_bpd)};
-    (void)per_xcd;
-    XcdSplit split = even_split(ns);
-    const int2* items = nullptr;
-    if (c.nItems2f > 0) {  // work items of the current prepare (plan_step2f)
-        for (int i = 0; i <= 8; ++i) split.start[i] = c.split2f[i];
-        items = c.items2f.as<int2>();
-    }
-    int widest = 0;
-    for (int i = 0; i < 8; ++i) widest = std::max(widest, split.start[i + 1] - split.start[i]);
-    hipLaunchKernelGGL((rd_step2f_kernel<Real, UniformStepParams<Real>>), dim3(8 * widest), dim3(512), 0, c.stream,
-                       split, items, in, out, mid, c.statF.as<Stat4<Real>>(), (const unsigned char*)nullptr, prm);
+    const StepWork wk = rd_step_work(c, skip_still);
+    hipLaunchKernelGGL((rd_step2f_kernel<Real, UniformStepParams<Real>>), dim3(wk.grid()), dim3(512), 0, c.stream, wk,
+                       in, out, mid, c.statF.as<Stat4<Real>>(), prm);
     GH_HIP_CHECK(hipGetLastError());
     return GH_OK;
 }
@@ -279,7 +256,7 @@ int rd_autotune(Ctx& c, double dt, int trial_steps, int* best_out) {
     int best = c.rd_bpw;
     for (int k = 0; k < 4; ++k) {
         c.rd_bpw = cand[k];
-        int rc = rd_steps(c, 2, dt);  // warm
+        int rc = rd_steps(c, cand[k] == 0 ? kStillMinSteps : 2, dt);  // warm: every kernel of the trial
         if (rc) return rc;
         GH_HIP_CHECK(hipEventRecord(c.ev0, c.stream));
         if ((rc = rd_steps(c, trial_steps, dt))) return rc;
@@ -298,6 +275,12 @@ int rd_autotune(Ctx& c, double dt, int trial_steps, int* best_out) {
 }
 
 double block_h_of(const Ctx& c) { return block_h(c); }
+
+StepWork rd_step_work(const Ctx& c, bool skip_still) {
+    if (c.nGrp == 0) return step_work(c.nFull, nullptr, 0, nullptr, nullptr);
+    return step_work(c.nFull, c.fullList.as<int32_t>(), c.nGrp, c.grpList.as<int2>(),
+                     skip_still ? c.stillGrp.as<unsigned char>() : nullptr);
+}
 
 int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st, const void* sig, DevBuf& out,
                     DevBuf& flag, bool* ok) {
@@ -322,11 +305,30 @@ int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st,
     return GH_OK;
 }
 
-int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt) {
+int rd_mark_still(Ctx& c, const void* in, void* out) {
+    return c.real_kind == GH_REAL_F32 ? mark_still<float>(c, (const float*)in, (float*)out)
+                                      : mark_still<double>(c, (const double*)in, (double*)out);
+}
+
+int rd_zero_still(Ctx& c, void* states, int n) {
+    if (c.nGrp == 0 || n <= 0) return GH_OK;
+    const dim3 g((unsigned)c.nGrp, (unsigned)n);
+    if (c.real_kind == GH_REAL_F32)
+        hipLaunchKernelGGL(still_zero_kernel<float>, g, dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
+                           c.stillGrp.as<unsigned char>(), (float*)states, c.ncells());
+    else
+        hipLaunchKernelGGL(still_zero_kernel<double>, g, dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
+                           c.stillGrp.as<unsigned char>(), (double*)states, c.ncells());
+    GH_HIP_CHECK(hipGetLastError());
+    return GH_OK;
+}
+
+int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool skip_still) {
     if (!c.fast_ok || c.topo.uniform_bpd <= 0)
         return set_error(GH_ESTATE, "two-step launch: needs a uniform grid with p_w + p_g >= 0");
-    return c.real_kind == GH_REAL_F32 ? launch_step2f<float>(c, (const float*)in, (float*)out, dt, (float*)mid)
-                                      : launch_step2f<double>(c, (const double*)in, (double*)out, dt, (double*)mid);
+    return c.real_kind == GH_REAL_F32
+               ? launch_step2f<float>(c, (const float*)in, (float*)out, dt, skip_still, (float*)mid)
+               : launch_step2f<double>(c, (const double*)in, (double*)out, dt, skip_still, (double*)mid);
 }
 
 int rd_step_buffers(Ctx& c, const void* in, void* out, double dt) {
@@ -336,7 +338,9 @@ int rd_step_buffers(Ctx& c, const void* in, void* out, double dt) {
 
 // Tile 0 takes two steps per launch.  A state written by the fused update is
 // clamped, so after one single step from whatever state the call starts with,
-// the pairs run rd_step2f_kernel when the anatomy allows it (fast_ok).
+// the pairs run rd_step2f_kernel when the anatomy allows it (fast_ok).  The
+// still groups are marked after that step: one launch of 4-6 us, worth it from
+// a few pairs on.
 int rd_steps(Ctx& c, int64_t nsteps, double dt) {
     c.dt_last = dt;
     const bool ghosted = c.topo.uniform_bpd <= 0;
@@ -351,10 +355,12 @@ int rd_steps(Ctx& c, int64_t nsteps, double dt) {
             c.cur = 1 - c.cur;
             k = 1;
         }
+        const bool skip = fast && c.nGrp > 0 && nsteps >= kStillMinSteps;
+        if (skip)
+            if (int rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p)) return rc;
         for (; k + 1 < nsteps; k += 2) {
             const int cur = c.cur;
-            int rc = fast ? (f32 ? launch_step2f<float>(c, c.phi[cur].as<float>(), c.phi[1 - cur].as<float>(), dt)
-                                 : launch_step2f<double>(c, c.phi[cur].as<double>(), c.phi[1 - cur].as<double>(), dt))
+            int rc = fast ? rd_step2_buffers(c, c.phi[cur].p, c.phi[1 - cur].p, nullptr, dt, skip)
                           : (f32 ? launch_step2<float>(c, c.phi[cur].as<float>(), c.phi[1 - cur].as<float>(), dt)
                                  : launch_step2<double>(c, c.phi[cur].as<double>(), c.phi[1 - cur].as<double>(), dt));
             if (rc) return rc;

@@ -12,6 +12,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdint>
+#include <vector>
 
 #include "gh_internal.h"
 
@@ -492,16 +493,20 @@ __global__ __launch_bounds__(256) void stat_fast_kernel(size_t n, const Stat4<Re
 // marks such blocks from the clamped-pair records: the three plus-face
 // coefficients of all 512 cells and the minus-face coefficients across the
 // block's -x, -y, -z faces (the neighbours' plus-face values) must all be +0.
+// out[s]: 0 a block with diffusion, 1 without, 2 without and with no cell that
+// is in the domain at phi = 0 (p_w + p_g = 0 in every cell): still_kernel.
 template <typename Real, typename Params>
 __global__ __launch_bounds__(256) void zero_flux_kernel(int nslots, const Stat4<Real>* __restrict__ stf, Params prm,
                                                         unsigned char* __restrict__ out) {
     const int s = blockIdx.x;
     if (s >= nslots) return;
     const Stat4<Real>* r = stf + (size_t)s * BCELLS;
-    bool nz = false;
-    for (int c = threadIdx.x; c < BCELLS; c += 256)
+    bool nz = false, dom = false;
+    for (int c = threadIdx.x; c < BCELLS; c += 256) {
+        dom |= sign_of(r[c].tau) != 0;
         nz |= (r[c].dx != (Real)0 || sign_of(r[c].dx)) || (r[c].dy != (Real)0 || sign_of(r[c].dy)) ||
               (r[c].dz != (Real)0 || sign_of(r[c].dz));
+    }
     if (threadIdx.x < 64) {
         const BlockPos bp = prm.pos(s);
         const int a = threadIdx.x & 7, b = threadIdx.x >> 3;
@@ -511,7 +516,8 @@ __global__ __launch_bounds__(256) void zero_flux_kernel(int nslots, const Stat4<
         nz |= (mx != (Real)0 || sign_of(mx)) || (my != (Real)0 || sign_of(my)) || (mz != (Real)0 || sign_of(mz));
     }
     nz = __syncthreads_or(nz);
-    if (threadIdx.x == 0) out[s] = nz ? 0 : 1;
+    dom = __syncthreads_or(dom);
+    if (threadIdx.x == 0) out[s] = nz ? 0 : (dom ? 1 : 2);
 }
 
 // dphidt of a cell of a block without diffusion (see zero_flux_kernel)
@@ -523,24 +529,118 @@ __device__ inline Real rd_rhs_reaction_only(Real pc, bool dom, Real rho) {
     return dom ? dphidt : (Real)0.;
 }
 
-// Relative cost of a block without diffusion in rd_step2f_kernel (its own
-// 24 B per cell, no halo, no LDS) against a full block (about 2.75 stencil
-// evaluations per cell): the weight the XCD split gives it.
-constexpr double kZeroFluxCost = 0.3;
-
-// Work split of the two-step kernel over the eight XCDs: workgroup w runs on
-// XCD w % 8 and serves block start[w % 8] + w / 8 while that is below
-// start[w % 8 + 1]; contiguous slot ranges keep halos in one L2, and the split
-// points balance the ranges' work when blocks differ in cost.
+// Work list of the two-step and the reverse-step kernels.  Blocks with
+// diffusion are one item each (full: their slots, ascending; null: item i is
+// slot i), runs of up to ZF_GROUP consecutive blocks without diffusion one item
+// of grp {slot, blocks}.  Workgroup w runs on XCD w % 8 and takes item w / 8 of
+// that XCD's contiguous share of full -- neighbours' halos stay in one L2 --
+// and after these its share of grp, which fill the tail.
+// still (may be null) marks the grp items that need nothing (still_kernel).
 struct XcdSplit {
     int start[9];
 };
-// equal contiguous ranges of ceil(n / 8) blocks (grid: 8 * ceil(n / 8))
 inline XcdSplit even_split(int n) {
     XcdSplit x{};
-    const int per = (n + 7) / 8;
-    for (int i = 0; i <= 8; ++i) x.start[i] = std::min(i * per, n);
+    for (int i = 0; i <= 8; ++i) x.start[i] = (int)((int64_t)n * i / 8);
     return x;
+}
+struct StepWork {
+    XcdSplit fs, gs;
+    const int32_t* __restrict__ full;
+    const int2* __restrict__ grp;
+    const unsigned char* __restrict__ still;
+    // this workgroup's item: its first slot, *nzf = 0 for a block with
+    // diffusion, else the blocks without diffusion; -1: nothing to do
+    __device__ inline int item(int* nzf) const {
+        const int x = (int)(blockIdx.x % 8), nf = fs.start[x + 1] - fs.start[x];
+        int i = (int)(blockIdx.x / 8);
+        *nzf = 0;
+        if (i < nf) {
+            i += fs.start[x];
+            return full ? full[i] : i;
+        }
+        i += gs.start[x] - nf;
+        if (i >= gs.start[x + 1] || (still && still[i])) return -1;
+        const int2 v = grp[i];
+        *nzf = v.y;
+        return v.x;
+    }
+    unsigned grid() const {
+        int w = 0;
+        for (int x = 0; x < 8; ++x)
+            w = std::max(w, fs.start[x + 1] - fs.start[x] + gs.start[x + 1] - gs.start[x]);
+        return 8u * (unsigned)w;
+    }
+};
+constexpr int ZF_GROUP = 8;  // blocks without diffusion per workgroup
+// the first nfull blocks and ngrp groups of a list
+inline StepWork step_work(int nfull, const int32_t* full, int ngrp, const int2* grp, const unsigned char* still) {
+    return StepWork{even_split(nfull), even_split(ngrp), full, grp, still};
+}
+
+// Zero is a fixed point of a block without diffusion: the reaction of 0 is 0.
+// A group whose blocks have no cell in the domain at 0 (zflux = 2) and whose
+// state is +0 in every cell keeps it for the rest of the solve, and its adjoint
+// keeps its value (adj_cell's factor is 1 out of the domain, its sums are
+// zeros).  Marks these groups once per solve and writes the zeros of the other
+// state buffer; the launches that follow leave them out, 24 B per cell and pair
+// of steps of a brain's surroundings (62-77 % of the blocks of a uniform head
+// grid).  FP32, us per launch before and after: pair of steps 128^3 11.96 /
+// 6.98, 256^3 84.7 / 26.8; reverse step 128^3 23.8 / 7.8.
+template <typename Real>
+__global__ __launch_bounds__(256) void still_kernel(int ngrp, const int2* __restrict__ grp,
+                                                    const unsigned char* __restrict__ zflux,
+                                                    const Real* __restrict__ phi, Real* __restrict__ out,
+                                                    unsigned char* __restrict__ still) {
+    const int i = blockIdx.x;
+    if (i >= ngrp) return;
+    const int2 v = grp[i];
+    const size_t c0 = (size_t)v.x * BCELLS;
+    bool moves = zflux[v.x] != 2;  // a group's blocks have one flag
+    if (!moves)
+        for (int c = threadIdx.x; c < v.y * BCELLS; c += 256) {
+            const Real u = phi[c0 + c];
+            moves |= u != (Real)0 || sign_of(u) != 0;
+        }
+    moves = __syncthreads_or(moves);
+    if (threadIdx.x == 0) still[i] = moves ? 0 : 1;
+    if (!moves)
+        for (int c = threadIdx.x; c < v.y * BCELLS; c += 256) out[c0 + c] = (Real)0;
+}
+// the zeros of the still groups in the state buffers out + k * stride, k <
+// gridDim.y (a segment's states, which no later launch writes there)
+template <typename Real>
+__global__ __launch_bounds__(256) void still_zero_kernel(int ngrp, const int2* __restrict__ grp,
+                                                         const unsigned char* __restrict__ still,
+                                                         Real* __restrict__ out, size_t stride) {
+    const int i = blockIdx.x;
+    if (i >= ngrp || !still[i]) return;
+    const int2 v = grp[i];
+    Real* o = out + (size_t)blockIdx.y * stride + (size_t)v.x * BCELLS;
+    for (int c = threadIdx.x; c < v.y * BCELLS; c += 256) o[c] = (Real)0;
+}
+// the work list of slots [0, cut.back()) from their zflux flags; nfull / ngrp (may be
+// null) receive the list lengths after each of the slot counts in cut
+// (ascending), at which groups end
+inline void build_step_work(const unsigned char* z, const std::vector<size_t>& cut, std::vector<int32_t>& full,
+                            std::vector<int2>& grp, std::vector<int>* nfull, std::vector<int>* ngrp) {
+    full.clear();
+    grp.clear();
+    int s = 0;
+    for (size_t e : cut) {
+        while (s < (int)e) {
+            if (!z[s]) {
+                full.push_back(s++);
+                continue;
+            }
+            int k = 1;
+            while (s + k < (int)e && z[s + k] == z[s] && k < ZF_GROUP) ++k;
+            grp.push_back(make_int2(s, k));
+            s += k;
+        }
+        if (nfull) nfull->push_back((int)full.size());
+        if (ngrp) ngrp->push_back((int)grp.size());
+    }
 }
 
 // Where cell (a, b) of face f at depth d (1 or 2) outside the block sits:
@@ -565,28 +665,13 @@ __device__ inline FaceMap face_map(int f, int d) {
 }
 __device__ inline int mad24(int a, int b, int c) { return (int)__umul24((unsigned)a, (unsigned)b) + c; }
 
-// Work items: with items (may be null), workgroup item i is {slot, k}: k = 0
-// a full block, k >= 1 the k consecutive blocks from slot on, all without
-// diffusion (their two steps are each cell's reaction update alone: same
-// bits, no halo).  Without items, item i is slot i, and zflux (may be null)
-// marks the blocks without diffusion (k = 1).
-constexpr int ZF_GROUP = 8;  // blocks without diffusion per workgroup
 template <typename Real, typename Params>
-__global__ __launch_bounds__(512) void rd_step2f_kernel(XcdSplit split, const int2* __restrict__ items,
-                                                        const Real* __restrict__ phi, Real* __restrict__ out,
-                                                        Real* __restrict__ mid, const Stat4<Real>* __restrict__ stf,
-                                                        const unsigned char* __restrict__ zflux, Params prm) {
-    const int x = (int)(blockIdx.x % 8);
-    const int it = split.start[x] + (int)(blockIdx.x / 8);
-    if (it >= split.start[x + 1]) return;
-    int s = it, nzf = 0;
-    if (items) {
-        const int2 v = items[it];
-        s = v.x;
-        nzf = v.y;
-    } else if (zflux && zflux[s]) {
-        nzf = 1;
-    }
+__global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real* __restrict__ phi,
+                                                        Real* __restrict__ out, Real* __restrict__ mid,
+                                                        const Stat4<Real>* __restrict__ stf, Params prm) {
+    int nzf;
+    const int s = wk.item(&nzf);
+    if (s < 0) return;
     __shared__ Real s_uu[UU_SIZE];
     __shared__ Real s_dmx[1000], s_dmy[1000], s_dmz[1000];
 
