@@ -167,7 +167,11 @@ struct Ctx {
     bool faces_stale = false, constants_stale = false;
     double Dw = 0, Dg = 0, rho = 0;
     double dt_last = 0;  // dt of the running gh_rd_steps call
-    int rd_bpw = 2;      // blocks per workgroup of the step kernel (1, 2 or 4)
+    // schedule of gh_rd_set_tile: blocks per workgroup of the step kernel (1, 2
+    // or 4, one step per launch) or 0, two steps per launch -- the faster one at
+    // every size (us per step, 2 vs 0: 32^3 FP32 4.1 / 2.3, 64^3 FP64 4.7 / 2.8,
+    // 128^3 FP32 12.7 / 3.2)
+    int rd_bpw = 0;
 
     size_t ncells() const { return (size_t)topo.nblocks() * BCELLS; }
     int alloc_fields();
