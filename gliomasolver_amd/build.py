@@ -24,8 +24,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # every HIP translation unit.
 COMMON = ["-O3", "-fPIC", "-pthread", "-std=c++17", "-ffp-contract=off", "-Wall", "-Wno-unused-function",
           "-I" + os.path.join(ROOT, "include")]
+# kernarg preload: a kernel's first 14 argument registers are filled before its
+# waves start instead of by their first scalar loads.
 HIP_FLAGS = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-             "-fno-gpu-rdc"]
+             "-fno-gpu-rdc", "-mllvm", "-amdgpu-kernarg-preload-count=14"]
 
 
 def sources():

@@ -61,7 +61,9 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
             if ((rc = rd_step2_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, nullptr, dt, skip))) return rc;
             k += 2;
         } else {
-            if ((rc = rd_step_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt))) return rc;
+            if ((rc = pairs && k >= 1 ? rd_step1_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt, skip)
+                                      : rd_step_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt)))
+                return rc;
             k += 1;
         }
         c.cur = 1 - c.cur;
@@ -103,7 +105,10 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
                     return rc;
                 j += 2;
             } else {
-                if ((rc = rd_step_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 1) * nb, dt))) return rc;
+                if ((rc = pairs && k0 + j >= 1
+                              ? rd_step1_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 1) * nb, dt, still)
+                              : rd_step_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 1) * nb, dt)))
+                    return rc;
                 j += 1;
             }
         }

@@ -131,6 +131,12 @@ template <typename Real>
 struct BatchStepParams {
     const int32_t* __restrict__ slot_pos;
     const SlotRange<Real>* __restrict__ range;
+    static constexpr bool kPow2 = false;  // any number of blocks per side
+    __host__ __device__ static inline BatchStepParams make(Real, double, double, int, uint32_t, const int32_t* sp,
+                                                           const void* r) {
+        return {sp, (const SlotRange<Real>*)r};
+    }
+    StepArgs<Real> args() const { return {(Real)0, 0., 0., 0, 0u, slot_pos, range}; }
     __device__ inline void get(int s, Real& r, double& i, double& d) const {
         const SlotRange<Real>& q = range[slot_pos[s]];
         r = q.rho;
@@ -151,7 +157,8 @@ __global__ __launch_bounds__(256) void batch_statics_kernel(size_t nslots, const
                                                             const SlotRange<Real>* __restrict__ range,
                                                             const Real* const* __restrict__ apw,
                                                             const Real* const* __restrict__ apg,
-                                                            Stat4<Real>* __restrict__ st, Real* __restrict__ sig) {
+                                                            Stat4<Real>* __restrict__ st, Real* __restrict__ sig,
+                                                            unsigned int* __restrict__ flags) {
     const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= nslots * BCELLS) return;
     const size_t s = gid / BCELLS;
@@ -175,6 +182,7 @@ __global__ __launch_bounds__(256) void batch_statics_kernel(size_t nslots, const
     r.tau = chf_threshold(pwc, pgc);
     st[gid] = r;
     sig[gid] = domain_threshold(pwc, pgc);
+    if (cancels(pwc, pgc)) atomicOr(flags + 1, 1u);
 }
 
 template <typename Real>
@@ -255,7 +263,7 @@ struct Batch {
     std::vector<size_t> slot0;      // per position, plus the total
     DevBuf phi[2], statD, statSig, nbr, slotPos, range, apw, apg, likPart, likOut, likJobs;
     DevBuf statF, flag;  // rd_step2f_kernel records (valid iff fast_ok), count scratch
-    bool fast_ok = false;
+    bool fast_ok = false, plain_dom = false;
     DevBuf zeroFlux;                 // per slot: != 0 a block without diffusion (zero_flux_kernel)
     // StepWork lists of all slots and their lengths per count of positions (index p: positions 0..p)
     DevBuf fullList, grpList, stillGrp;
@@ -362,12 +370,14 @@ int build_layout_t(Batch& b) {
     GH_HIP_CHECK(hipMemcpyAsync(b.apw.p, apw.data(), ns * sizeof(void*), hipMemcpyHostToDevice, b.stream));
     GH_HIP_CHECK(hipMemcpyAsync(b.apg.p, apg.data(), ns * sizeof(void*), hipMemcpyHostToDevice, b.stream));
     const unsigned g = (unsigned)((nc + 255) / 256);
+    if ((rc = clear_stat_flags(b.stream, b.flag))) return rc;
     hipLaunchKernelGGL(batch_statics_kernel<Real>, dim3(g), dim3(256), 0, b.stream, nsl, b.nbr.as<int32_t>(),
                        b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>(), b.apw.as<const Real* const>(),
-                       b.apg.as<const Real* const>(), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>());
+                       b.apg.as<const Real* const>(), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
+                       b.flag.as<unsigned int>());
     GH_HIP_CHECK(hipGetLastError());
     if ((rc = build_stat_fast(b.stream, sizeof(Real) == 4 ? GH_REAL_F32 : GH_REAL_F64, nc, b.statD.p, b.statSig.p,
-                              b.statF, b.flag, &b.fast_ok)))
+                              b.statF, b.flag, &b.fast_ok, &b.plain_dom)))
         return rc;
     b.nFull.clear();
     b.nGrp.clear();
@@ -553,16 +563,13 @@ struct ForwardSweep {
         const bool two = npos[active - 1] >= k + 2 && (K <= 0 || (k + 1) % K != 0) && (k >= 1 || !b.fast_ok);
         const Real* in = b.phi[cur].as<Real>();
         Real* out = b.phi[1 - cur].as<Real>();
-        if (two) {
+        if (b.fast_ok && k >= 1) {
+            launch_step2f_kernel<Real>(b.stream, b.work(active), b.plain_dom, two, in, out, (Real*)nullptr,
+                                       b.statF.as<Stat4<Real>>(), prm);
+        } else if (two) {
             const int per_xcd = (nsl + 7) / 8;
-            const StepWork wk = b.work(active);
-            if (b.fast_ok)
-                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(wk.grid()), dim3(512), 0,
-                                   b.stream, wk, in, out, (Real*)nullptr, b.statF.as<Stat4<Real>>(), prm);
-            else
-                hipLaunchKernelGGL((rd_step2_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
-                                   b.stream, nsl, per_xcd, in, out, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
-                                   prm);
+            hipLaunchKernelGGL((rd_step2_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
+                               b.stream, nsl, per_xcd, in, out, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(), prm);
         } else {
             const int per_xcd = ((nsl + 1) / 2 + 7) / 8;  // two blocks per workgroup
             hipLaunchKernelGGL((rd_step_kernel<Real, true, 2, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512),
@@ -749,12 +756,13 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         for (int64_t k = k0; k < k1;) {
             char* in = tape + (size_t)(k - k0) * nsl * slot_bytes;
             const int nslots = (int)b.slot0[active(k)];
-            if (b.fast_ok && k >= 1 && k + 2 <= k1) {
-                const StepWork wk = b.work(active(k));
-                hipLaunchKernelGGL((rd_step2f_kernel<Real, BatchStepParams<Real>>), dim3(wk.grid()), dim3(512), 0,
-                                   b.stream, wk, (const Real*)in, (Real*)(in + 2 * (size_t)nsl * slot_bytes),
-                                   (Real*)(in + (size_t)nsl * slot_bytes), b.statF.as<Stat4<Real>>(), fprm);
-                k += 2;
+            if (b.fast_ok && k >= 1) {
+                const bool two = k + 2 <= k1;
+                Real* next = (Real*)(in + (size_t)nsl * slot_bytes);
+                launch_step2f_kernel<Real>(b.stream, b.work(active(k)), b.plain_dom, two, (const Real*)in,
+                                           two ? (Real*)(in + 2 * (size_t)nsl * slot_bytes) : next,
+                                           two ? next : (Real*)nullptr, b.statF.as<Stat4<Real>>(), fprm);
+                k += two ? 2 : 1;
             } else {
                 step(in, in + (size_t)nsl * slot_bytes, nslots);
                 k += 1;

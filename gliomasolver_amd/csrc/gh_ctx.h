@@ -140,7 +140,8 @@ struct Ctx {
     DevBuf statF;       // 4 * ncells: {D+x, D+y, D+z, tau_enc} of rd_step2f_kernel (valid iff fast_ok)
     DevBuf flag;        // small scratch word for device-side counts
     bool fast_ok = false;  // every cell has p_w + p_g >= 0: clamped states may take rd_step2f_kernel
-    DevBuf zeroFlux;       // per slot: 1 = block without diffusion (zero_flux_kernel), uniform grids
+    bool plain_dom = false;  // no cell has p_w = -p_g != 0: rd_step2f_kernel needs no domain test
+    DevBuf zeroFlux;       // per slot: != 0 a block without diffusion (zero_flux_kernel), uniform grids
     int nZeroFlux = 0;     // blocks without diffusion
     // work list of the two-step and reverse-step kernels (StepWork, plan_step2f):
     // slots of the blocks with diffusion, groups of blocks without (nGrp = 0:
@@ -194,6 +195,8 @@ int rd_step_buffers(Ctx& c, const void* in, void* out, double dt);
 // skip_still: leave out the groups that rd_mark_still marked, whose zeros
 // stand in out and mid
 int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool skip_still = false);
+// one fused step from a clamped state when c.fast_ok
+int rd_step1_buffers(Ctx& c, const void* in, void* out, double dt, bool skip_still);
 // marks the groups of blocks without diffusion that the clamped state `in`
 // leaves at zero for good, and writes their zeros into out
 int rd_mark_still(Ctx& c, const void* in, void* out);
@@ -204,9 +207,12 @@ struct StepWork;
 StepWork rd_step_work(const Ctx& c, bool skip_still);
 double block_h_of(const Ctx& c);
 // the rd_step2f_kernel records of n cells from {D+, tau} and sigma into out;
-// *ok = every cell has sigma <= 0 (p_w + p_g >= 0).  Synchronizes the stream.
+// *ok = every cell has sigma <= 0 (p_w + p_g >= 0); *plain = flag's second word
+// is 0 (no cell cancels).  Synchronizes the stream.
 int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st, const void* sig, DevBuf& out,
-                    DevBuf& flag, bool* ok);
+                    DevBuf& flag, bool* ok, bool* plain);
+// zeroes flag's two words, before the kernel that fills st and sig
+int clear_stat_flags(hipStream_t stream, DevBuf& flag);
 int rd_autotune(Ctx& c, double dt, int trial_steps, int* best);
 
 // adaptive grid (gh_adapt.hip)

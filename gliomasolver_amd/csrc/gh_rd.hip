@@ -38,7 +38,7 @@ template <typename Real>
 __global__ __launch_bounds__(256) void rd_statics_kernel(int nslots, const int32_t* __restrict__ nbr,
                                                          const Real* __restrict__ pw, const Real* __restrict__ pg,
                                                          Real Dw, Real Dg, Stat4<Real>* __restrict__ st,
-                                                         Real* __restrict__ sig) {
+                                                         Real* __restrict__ sig, unsigned int* __restrict__ flags) {
     const size_t nc = (size_t)nslots * BCELLS;
     const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= nc) return;
@@ -58,6 +58,7 @@ __global__ __launch_bounds__(256) void rd_statics_kernel(int nslots, const int32
     r.tau = chf_threshold(pwc, pgc);
     st[gid] = r;
     sig[gid] = domain_threshold(pwc, pgc);
+    if (cancels(pwc, pgc)) atomicOr(flags + 1, 1u);
 }
 
 template <typename Real>
@@ -127,12 +128,14 @@ int prepare_t(Ctx& c, double Dw, double Dg, double rho) {
     const int ns = c.topo.nblocks();
     const size_t nc = c.ncells();
     const unsigned grid = (unsigned)((nc + 255) / 256);
+    int rc;
+    if ((rc = clear_stat_flags(c.stream, c.flag))) return rc;
     hipLaunchKernelGGL(rd_statics_kernel<Real>, dim3(grid), dim3(256), 0, c.stream, ns, c.nbr.as<int32_t>(),
                        c.pw.as<Real>(), c.pg.as<Real>(), (Real)Dw, (Real)Dg, c.statD.as<Stat4<Real>>(),
-                       c.statSig.as<Real>());
+                       c.statSig.as<Real>(), c.flag.as<unsigned int>());
     GH_HIP_CHECK(hipGetLastError());
-    int rc;
-    if ((rc = build_stat_fast(c.stream, c.real_kind, nc, c.statD.p, c.statSig.p, c.statF, c.flag, &c.fast_ok)))
+    if ((rc = build_stat_fast(c.stream, c.real_kind, nc, c.statD.p, c.statSig.p, c.statF, c.flag, &c.fast_ok,
+                              &c.plain_dom)))
         return rc;
     if ((rc = plan_step2f<Real>(c))) return rc;
     c.Dw = Dw;
@@ -169,17 +172,16 @@ int launch_step2(Ctx& c, const Real* in, Real* out, double dt) {
     return GH_OK;
 }
 
-// two fused steps per launch on a clamped state (rd_step2f_kernel); mid, when
-// not null, receives the state after the first step; skip_still: the still
-// groups are marked and their zeros stand in out (and mid)
+// two fused steps (or one) per launch on a clamped state (rd_step2f_kernel);
+// mid, when not null, receives the state after the first of two; skip_still:
+// the still groups are marked and their zeros stand in out (and mid)
 template <typename Real>
-int launch_step2f(Ctx& c, const Real* in, Real* out, double dt, bool skip_still, Real* mid = nullptr) {
+int launch_step2f(Ctx& c, const Real* in, Real* out, double dt, bool two, bool skip_still, Real* mid = nullptr) {
     const double h = block_h(c);
     const double ih2 = 1. / (h * h);
     const UniformStepParams<Real> prm{(Real)c.rho, ih2, dt, c.topo.uniform_bpd, bpd_magic(c.topo.uniform_bpd)};
     const StepWork wk = rd_step_work(c, skip_still);
-    hipLaunchKernelGGL((rd_step2f_kernel<Real, UniformStepParams<Real>>), dim3(wk.grid()), dim3(512), 0, c.stream, wk,
-                       in, out, mid, c.statF.as<Stat4<Real>>(), prm);
+    launch_step2f_kernel<Real>(c.stream, wk, c.plain_dom, two, in, out, mid, c.statF.as<Stat4<Real>>(), prm);
     GH_HIP_CHECK(hipGetLastError());
     return GH_OK;
 }
@@ -282,12 +284,17 @@ StepWork rd_step_work(const Ctx& c, bool skip_still) {
                      skip_still ? c.stillGrp.as<unsigned char>() : nullptr);
 }
 
+int clear_stat_flags(hipStream_t stream, DevBuf& flag) {
+    if (int rc = flag.ensure(2 * sizeof(unsigned int))) return rc;
+    GH_HIP_CHECK(hipMemsetAsync(flag.p, 0, 2 * sizeof(unsigned int), stream));
+    return GH_OK;
+}
+
 int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st, const void* sig, DevBuf& out,
-                    DevBuf& flag, bool* ok) {
+                    DevBuf& flag, bool* ok, bool* plain) {
     const size_t rs = real_kind == GH_REAL_F32 ? 4 : 8;
     int rc;
-    if ((rc = out.ensure_grow(std::max<size_t>(1, n) * 4 * rs)) || (rc = flag.ensure(sizeof(unsigned int)))) return rc;
-    GH_HIP_CHECK(hipMemsetAsync(flag.p, 0, sizeof(unsigned int), stream));
+    if ((rc = out.ensure_grow(std::max<size_t>(1, n) * 4 * rs))) return rc;
     const unsigned grid = (unsigned)((n + 255) / 256);
     if (n > 0) {
         if (real_kind == GH_REAL_F32)
@@ -298,10 +305,11 @@ int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st,
                                (const double*)sig, out.as<Stat4<double>>(), flag.as<unsigned int>());
         GH_HIP_CHECK(hipGetLastError());
     }
-    unsigned int bad = 0;
-    GH_HIP_CHECK(hipMemcpyAsync(&bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost, stream));
+    unsigned int bad[2] = {1, 1};
+    GH_HIP_CHECK(hipMemcpyAsync(bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost, stream));
     GH_HIP_CHECK(hipStreamSynchronize(stream));
-    *ok = bad == 0;
+    *ok = bad[0] == 0;
+    *plain = bad[1] == 0;
     return GH_OK;
 }
 
@@ -323,12 +331,20 @@ int rd_zero_still(Ctx& c, void* states, int n) {
     return GH_OK;
 }
 
-int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool skip_still) {
+static int step2f_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool two, bool skip_still) {
     if (!c.fast_ok || c.topo.uniform_bpd <= 0)
         return set_error(GH_ESTATE, "two-step launch: needs a uniform grid with p_w + p_g >= 0");
     return c.real_kind == GH_REAL_F32
-               ? launch_step2f<float>(c, (const float*)in, (float*)out, dt, skip_still, (float*)mid)
-               : launch_step2f<double>(c, (const double*)in, (double*)out, dt, skip_still, (double*)mid);
+               ? launch_step2f<float>(c, (const float*)in, (float*)out, dt, two, skip_still, (float*)mid)
+               : launch_step2f<double>(c, (const double*)in, (double*)out, dt, two, skip_still, (double*)mid);
+}
+
+int rd_step2_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool skip_still) {
+    return step2f_buffers(c, in, out, mid, dt, true, skip_still);
+}
+
+int rd_step1_buffers(Ctx& c, const void* in, void* out, double dt, bool skip_still) {
+    return step2f_buffers(c, in, out, nullptr, dt, false, skip_still);
 }
 
 int rd_step_buffers(Ctx& c, const void* in, void* out, double dt) {
@@ -360,11 +376,16 @@ int rd_steps(Ctx& c, int64_t nsteps, double dt) {
             if (int rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p)) return rc;
         for (; k + 1 < nsteps; k += 2) {
             const int cur = c.cur;
-            int rc = fast ? rd_step2_buffers(c, c.phi[cur].p, c.phi[1 - cur].p, nullptr, dt, skip)
+            int rc = fast ? step2f_buffers(c, c.phi[cur].p, c.phi[1 - cur].p, nullptr, dt, true, skip)
                           : (f32 ? launch_step2<float>(c, c.phi[cur].as<float>(), c.phi[1 - cur].as<float>(), dt)
                                  : launch_step2<double>(c, c.phi[cur].as<double>(), c.phi[1 - cur].as<double>(), dt));
             if (rc) return rc;
             c.cur = 1 - c.cur;
+        }
+        if (fast && k < nsteps) {  // the odd step
+            if (int rc = rd_step1_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt, skip)) return rc;
+            c.cur = 1 - c.cur;
+            ++k;
         }
     }
     for (; k < nsteps; ++k) {

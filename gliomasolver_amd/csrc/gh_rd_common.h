@@ -101,6 +101,13 @@ __host__ __device__ inline Real domain_threshold(Real pw, Real pg) {
     return -s;
 }
 
+// p_w + p_g = 0 with p_w = -p_g != 0: a cell outside the domain (at phi = 0)
+// whose face coefficients need not be zeros
+template <typename Real>
+__host__ __device__ inline bool cancels(Real pw, Real pg) {
+    return pw != (Real)0 && pw + pg == (Real)0;
+}
+
 // LDS index of cell (x, y, z) in a 10^3 block tile with a one-cell halo
 __device__ inline int P(int x, int y, int z) { return (z + 1) * 100 + (y + 1) * 10 + (x + 1); }
 
@@ -196,6 +203,19 @@ __device__ inline int face_dy(int f) { return f == FYM ? -1 : (f == FYP ? 1 : 0)
 __device__ inline int face_dz(int f) { return f == FZM ? -1 : (f == FZP ? 1 : 0); }
 __device__ inline int face_nb(const BlockPos& p, int f) { return p.nb(face_dx(f), face_dy(f), face_dz(f)); }
 
+// rd_step2f_kernel's parameters as plain arguments: the scalars that its first
+// loads depend on lie in front, where they are in registers when a wave starts
+// (build.py: kernarg preload), 0.4 us of a 6.1 us pair of steps at 128^3.
+template <typename Real>
+struct StepArgs {
+    Real rho;
+    double ih2, dt;
+    int bpd;
+    uint32_t magic;
+    const int32_t* slot_pos;  // packed solves: the solve of a slot and its SlotRange
+    const void* range;
+};
+
 // Step parameters of a slot: one solve (the same rho, 1/h^2, dt for every
 // slot) or many independent solves packed slot range after slot range.
 template <typename Real>
@@ -204,6 +224,12 @@ struct UniformStepParams {
     double ih2, dt;
     int bpd;
     uint32_t magic;  // bpd_magic(bpd)
+    static constexpr bool kPow2 = true;  // h = 2^-level / 8
+    __host__ __device__ static inline UniformStepParams make(Real r, double i, double d, int b, uint32_t m,
+                                                             const int32_t*, const void*) {
+        return {r, i, d, b, m};
+    }
+    StepArgs<Real> args() const { return {rho, ih2, dt, bpd, magic, nullptr, nullptr}; }
     __device__ inline void get(int, Real& r, double& i, double& d) const {
         r = rho;
         i = ih2;
@@ -431,8 +457,8 @@ __global__ __launch_bounds__(512) void rd_step2_kernel(int nslots, int per_xcd,
 //   * a neighbour's outside flag travels in the sign bit of its value in LDS
 //     (-phi when phi < tau), so a stencil reads six values instead of six
 //     values and six thresholds, and the flag doubles a face by ldexp.
-// The arithmetic after the no-flux doubling is rd_rhs_core, and doubling is
-// exact, so the results are those of rd_step2_kernel bit for bit.
+// The arithmetic after the no-flux doubling has rd_rhs_core's results, and
+// doubling is exact, so the results are those of rd_step2_kernel bit for bit.
 //
 // LDS: s_uu holds the encoded step-0 state on [-2,10)^3 and, in the second
 // half of each 24-value row, the encoded step-1 state on [-1,9)^3; rows of 24
@@ -453,19 +479,46 @@ __device__ inline double twice_if(double d, uint32_t o) { return __builtin_amdgc
 template <typename Real>
 __device__ inline Real flag_in_sign(Real u, Real tau) { return u < tau ? -u : u; }
 
-// dphidt from encoded neighbours e0..e5 (-x,+x,-y,+y,-z,+z) and the face
-// coefficients d0..d5 before the no-flux rule
-template <typename Real>
-__device__ inline Real rd_rhs_enc(Real d0, Real d1, Real d2, Real d3, Real d4, Real d5, Real e0, Real e1, Real e2,
-                                  Real e3, Real e4, Real e5, Real pc, bool inside, Real rho, double ih2) {
+// The state after one step from encoded neighbours e0..e5 (-x,+x,-y,+y,-z,+z)
+// and the face coefficients d0..d5 before the no-flux rule: rd_rhs_core and
+// rd_update with fewer operations and the same bits.
+//   DOM = false (every cell has p_w + p_g != 0 or p_w = p_g = 0): a cell out of
+//     the domain has six zero face coefficients and the state 0, so its dphidt
+//     comes out +0 without the test.
+//   POW2 (1/h^2 a power of two): the scalings of both fluxes are exact, so
+//     ih2*in - ih2*out = ih2*(in - out), and the sum with the reaction is one
+//     fused multiply-add of an exact product.
+template <bool DOM, bool POW2, typename Real>
+__device__ inline Real rd_step_enc(Real d0, Real d1, Real d2, Real d3, Real d4, Real d5, Real e0, Real e1, Real e2,
+                                   Real e3, Real e4, Real e5, Real pc, bool inside, Real rho, double ih2, double dt) {
     d1 = twice_if(d1, sign_of(e0));
     d0 = twice_if(d0, sign_of(e1));
     d3 = twice_if(d3, sign_of(e2));
     d2 = twice_if(d2, sign_of(e3));
     d5 = twice_if(d5, sign_of(e4));
     d4 = twice_if(d4, sign_of(e5));
-    return rd_rhs_core<Real>(d0, d1, d2, d3, d4, d5, std::fabs(e0), std::fabs(e1), std::fabs(e2), std::fabs(e3),
-                             std::fabs(e4), std::fabs(e5), pc, inside || pc > (Real)0., rho, ih2);
+    if constexpr (!POW2)
+        return rd_update(pc,
+                         rd_rhs_core<Real>(d0, d1, d2, d3, d4, d5, std::fabs(e0), std::fabs(e1), std::fabs(e2),
+                                           std::fabs(e3), std::fabs(e4), std::fabs(e5), pc,
+                                           !DOM || inside || pc > (Real)0., rho, ih2),
+                         dt);
+    Real sin_ = d0 * std::fabs(e0);
+    sin_ = sin_ + d1 * std::fabs(e1);
+    sin_ = sin_ + d2 * std::fabs(e2);
+    sin_ = sin_ + d3 * std::fabs(e3);
+    sin_ = sin_ + d4 * std::fabs(e4);
+    sin_ = sin_ + d5 * std::fabs(e5);
+    Real sdf = d0 + d1;
+    sdf = sdf + d2;
+    sdf = sdf + d3;
+    sdf = sdf + d4;
+    sdf = sdf + d5;
+    const Real sdp = sdf * pc;
+    const Real rp = rho * pc;
+    const double react = (double)rp * (1. - (double)pc);
+    const Real dphidt = (Real)__builtin_fma((double)sin_ - (double)sdp, ih2, react);
+    return rd_update(pc, !DOM || inside || pc > (Real)0. ? dphidt : (Real)0., dt);
 }
 
 // {dx, dy, dz, tau} + sigma -> the record of rd_step2f_kernel; counts the
@@ -533,49 +586,36 @@ __device__ inline Real rd_rhs_reaction_only(Real pc, bool dom, Real rho) {
 // diffusion are one item each (full: their slots, ascending; null: item i is
 // slot i), runs of up to ZF_GROUP consecutive blocks without diffusion one item
 // of grp {slot, blocks}.  Workgroup w runs on XCD w % 8 and takes item w / 8 of
-// that XCD's contiguous share of full -- neighbours' halos stay in one L2 --
-// and after these its share of grp, which fill the tail.
+// that XCD's contiguous share of full (fper items) -- neighbours' halos stay in
+// one L2 -- and after these its share of grp (gper), which fill the tail.
 // still (may be null) marks the grp items that need nothing (still_kernel).
-struct XcdSplit {
-    int start[9];
-};
-inline XcdSplit even_split(int n) {
-    XcdSplit x{};
-    for (int i = 0; i <= 8; ++i) x.start[i] = (int)((int64_t)n * i / 8);
-    return x;
-}
 struct StepWork {
-    XcdSplit fs, gs;
+    int nfull, fper, ngrp, gper;
     const int32_t* __restrict__ full;
     const int2* __restrict__ grp;
     const unsigned char* __restrict__ still;
     // this workgroup's item: its first slot, *nzf = 0 for a block with
     // diffusion, else the blocks without diffusion; -1: nothing to do
     __device__ inline int item(int* nzf) const {
-        const int x = (int)(blockIdx.x % 8), nf = fs.start[x + 1] - fs.start[x];
-        int i = (int)(blockIdx.x / 8);
+        const int x = (int)(blockIdx.x % 8), j = (int)(blockIdx.x / 8);
         *nzf = 0;
-        if (i < nf) {
-            i += fs.start[x];
+        if (j < fper) {
+            const int i = x * fper + j;
+            if (i >= nfull) return -1;
             return full ? full[i] : i;
         }
-        i += gs.start[x] - nf;
-        if (i >= gs.start[x + 1] || (still && still[i])) return -1;
+        const int i = x * gper + j - fper;
+        if (i >= ngrp || (still && still[i])) return -1;
         const int2 v = grp[i];
         *nzf = v.y;
         return v.x;
     }
-    unsigned grid() const {
-        int w = 0;
-        for (int x = 0; x < 8; ++x)
-            w = std::max(w, fs.start[x + 1] - fs.start[x] + gs.start[x + 1] - gs.start[x]);
-        return 8u * (unsigned)w;
-    }
+    unsigned grid() const { return 8u * (unsigned)(fper + gper); }
 };
 constexpr int ZF_GROUP = 8;  // blocks without diffusion per workgroup
 // the first nfull blocks and ngrp groups of a list
 inline StepWork step_work(int nfull, const int32_t* full, int ngrp, const int2* grp, const unsigned char* still) {
-    return StepWork{even_split(nfull), even_split(ngrp), full, grp, still};
+    return StepWork{nfull, (nfull + 7) / 8, ngrp, (ngrp + 7) / 8, full, grp, still};
 }
 
 // Zero is a fixed point of a block without diffusion: the reaction of 0 is 0.
@@ -652,23 +692,30 @@ struct FaceMap {
     int dm, dma, dmb;
     int lo, loa, lob;
 };
-__device__ inline FaceMap face_map(int f, int d) {
-    const int u0 = UU(0, 0, 0), m0 = DMI(0, 0, 0);
-    switch (f) {
-        case FXM: return {u0 - d, 24, 293, m0 - d, 10, 100, 8 - d, 8, 64};
-        case FXP: return {u0 + 7 + d, 24, 293, m0 + 7 + d, 10, 100, d - 1, 8, 64};
-        case FYM: return {u0 - 24 * d, 1, 293, m0 - 10 * d, 1, 100, 8 * (8 - d), 1, 64};
-        case FYP: return {u0 + 24 * (7 + d), 1, 293, m0 + 10 * (7 + d), 1, 100, 8 * (d - 1), 1, 64};
-        case FZM: return {u0 - 293 * d, 1, 24, m0 - 100 * d, 1, 10, 64 * (8 - d), 1, 8};
-        default:  return {u0 + 293 * (7 + d), 1, 24, m0 + 100 * (7 + d), 1, 10, 64 * (d - 1), 1, 8};
-    }
+__device__ inline FaceMap face_map(int f, int d) {  // f = 2 axis + (plus side), by selects: no branch for a uniform f
+    const bool ax = f < 2, az = f >= 4;
+    const int su = ax ? 1 : (az ? 293 : 24), sm = ax ? 1 : (az ? 100 : 10), sl = ax ? 1 : (az ? 64 : 8);
+    const int out = f & 1 ? 7 + d : -d, in = f & 1 ? d - 1 : 8 - d;
+    return {UU(0, 0, 0) + su * out, ax ? 24 : 1, az ? 24 : 293, DMI(0, 0, 0) + sm * out, ax ? 10 : 1, az ? 10 : 100,
+            sl * in, ax ? 8 : 1, az ? 8 : 64};
 }
 __device__ inline int mad24(int a, int b, int c) { return (int)__umul24((unsigned)a, (unsigned)b) + c; }
 
-template <typename Real, typename Params>
-__global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real* __restrict__ phi,
-                                                        Real* __restrict__ out, Real* __restrict__ mid,
-                                                        const Stat4<Real>* __restrict__ stf, Params prm) {
+// 512 lanes: wave w has the interior plane z = w and one of eight halo roles
+// (faces 0-5, then the two halves of the edge cells).  With 256 lanes of two
+// planes and two roles each, 14 % fewer vector instructions per block, a pair of
+// steps takes as long at 256^3 (27.5 us) and longer at 128^3 (6.6 -> 7.3 us):
+// the loads and barriers of a block bound it.  TWO = false: one step only (no
+// edges, no depth-2 halo), 18 instead of 73 us for 41,000 slots.
+template <typename Real, typename Params, bool DOM, bool TWO>
+__global__ __launch_bounds__(512) void rd_step2f_kernel(
+    int nfull, int fper, const int32_t* __restrict__ full, const Real* __restrict__ phi,
+    const Stat4<Real>* __restrict__ stf, int bpd, uint32_t magic, const int32_t* __restrict__ slot_pos,
+    const void* __restrict__ range, Real* __restrict__ out, Real* __restrict__ mid, Real rho_, double ih2_, double dt_,
+    int ngrp, int gper, const int2* __restrict__ grp, const unsigned char* __restrict__ still) {
+    const StepWork wk{nfull, fper, ngrp, gper, full, grp, still};
+    const Params prm = Params::make(rho_, ih2_, dt_, bpd, magic, slot_pos, range);
+    constexpr bool POW2 = Params::kPow2;
     int nzf;
     const int s = wk.item(&nzf);
     if (s < 0) return;
@@ -676,40 +723,31 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real*
     __shared__ Real s_dmx[1000], s_dmy[1000], s_dmz[1000];
 
     const int t = threadIdx.x;
-    if (nzf > 0) {  // uniform per workgroup: nzf blocks, all loads issued before the updates
-        Real u0[ZF_GROUP];
-        bool in0[ZF_GROUP];
-#pragma unroll
-        for (int k = 0; k < ZF_GROUP; ++k)
-            if (k < nzf) {
-                const size_t bc = (size_t)(s + k) * BCELLS + (unsigned)t;
-                u0[k] = phi[bc];
-                in0[k] = sign_of(stf[bc].tau) != 0;
-            }
-#pragma unroll
-        for (int k = 0; k < ZF_GROUP; ++k)
-            if (k < nzf) {
-                const size_t bc = (size_t)(s + k) * BCELLS + (unsigned)t;
-                Real rho0;
-                double ih20, dt0;
-                prm.get(s + k, rho0, ih20, dt0);
-                const Real u1 = rd_update(u0[k], rd_rhs_reaction_only(u0[k], in0[k] || u0[k] > (Real)0., rho0), dt0);
-                if (mid) mid[bc] = u1;
-                out[bc] = rd_update(u1, rd_rhs_reaction_only(u1, in0[k] || u1 > (Real)0., rho0), dt0);
-            }
+    const size_t base = (size_t)s * BCELLS;
+    Real rho;
+    double ih2, dt;
+    prm.get(s, rho, ih2, dt);  // a group's blocks belong to one solve
+    if (nzf > 0) {             // uniform per workgroup
+        for (int i = t; i < nzf * BCELLS; i += 512) {
+            const size_t bc = base + (unsigned)i;
+            const Real u0 = phi[bc];
+            const bool in0 = sign_of(stf[bc].tau) != 0;
+            const Real u1 = rd_update(u0, rd_rhs_reaction_only(u0, in0 || u0 > (Real)0., rho), dt);
+            if (TWO && mid) mid[bc] = u1;
+            out[bc] = TWO ? rd_update(u1, rd_rhs_reaction_only(u1, in0 || u1 > (Real)0., rho), dt) : u1;
+        }
         return;
     }
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // wave = interior plane z; halo role
     const int a = t & 7, b = (t >> 3) & 7;
     const BlockPos bp = prm.pos(s);
-    const size_t base = (size_t)s * BCELLS;
     const unsigned ut = (unsigned)t;
 
     // ---- loads: (waves 0-5) the depth-1 and depth-2 cells of face w, (waves
     // 6-7) the 96 edge cells next to the depth-1 faces, then the own cell; all
     // offsets are computed first so the loads issue back to back; block base
     // pointers are wave-uniform, lane offsets 32-bit
-    Real u_1 = 0, u_2 = 0, u_e = 0;  // depth-1, depth-2 and edge cell
+    Real u_1 = 0, u_2 = 0, u_e = 0;  // depth-1, depth-2 and edge cell: of their own, so that no load waits for another
     Stat4<Real> st_1, st_2, st_e;
     int uu1 = 0, dm1 = 0, uu2 = 0, dm2 = 0;
     int ex = 0, ey = 0, ez = 0;  // edge cell: tile coordinates
@@ -718,18 +756,18 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real*
         const FaceMap m1 = face_map(w, 1), m2 = face_map(w, 2);
         const size_t nb = (size_t)face_nb(bp, w) * BCELLS;
         const unsigned l1 = (unsigned)mad24(b, m1.lob, mad24(a, m1.loa, m1.lo)) & (BCELLS - 1);
-        const unsigned l2 = (l1 + (unsigned)(m2.lo - m1.lo)) & (BCELLS - 1);
         uu1 = mad24(b, m1.uub, mad24(a, m1.uua, m1.uu));
         dm1 = mad24(b, m1.dmb, mad24(a, m1.dma, m1.dm));
-        uu2 = uu1 + (m2.uu - m1.uu);
-        dm2 = dm1 + (m2.dm - m1.dm);
-        const Real* pn = phi + nb;
-        const Stat4<Real>* sn = stf + nb;
-        u_1 = pn[l1];
-        st_1 = sn[l1];
-        u_2 = pn[l2];
-        st_2 = sn[l2];
-    } else {
+        u_1 = (phi + nb)[l1];
+        st_1 = (stf + nb)[l1];
+        if (TWO) {
+            const unsigned l2 = (l1 + (unsigned)(m2.lo - m1.lo)) & (BCELLS - 1);
+            uu2 = uu1 + (m2.uu - m1.uu);
+            dm2 = dm1 + (m2.dm - m1.dm);
+            u_2 = (phi + nb)[l2];
+            st_2 = (stf + nb)[l2];
+        }
+    } else if (TWO) {
         const int e = (w - 6) * 64 + (t & 63);
         edge = e < 96;
         if (edge) {
@@ -753,32 +791,32 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real*
     }
     const Real u_c = (phi + base)[ut];
     const Stat4<Real> st_c = (stf + base)[ut];
-    Real rho;
-    double ih2, dt;
-    prm.get(s, rho, ih2, dt);
 
     // ---- LDS: encoded step-0 state, minus-face coefficients of the step-1 cells
     const int uuc = mad24(w, 293, mad24(b, 24, a + UU(0, 0, 0)));
     const int dmc = mad24(w, 100, mad24(b, 10, a + DMI(0, 0, 0)));
     const Real tau_c = std::fabs(st_c.tau);
+    Real tau_1 = 0;
     s_uu[uuc] = flag_in_sign(u_c, tau_c);
     s_dmx[dmc + 1] = st_c.dx;
     s_dmy[dmc + 10] = st_c.dy;
     s_dmz[dmc + 100] = st_c.dz;
-    Real tau_1 = 0;
     if (w < 6) {
         tau_1 = std::fabs(st_1.tau);
         s_uu[uu1] = flag_in_sign(u_1, tau_1);
-        s_uu[uu2] = flag_in_sign(u_2, std::fabs(st_2.tau));
-        // depth-1 cell: every component whose target stays in [-1,9)^3;
-        // depth-2 cell: only the normal component of a minus face
-        if (w != FXP) s_dmx[dm1 + 1] = st_1.dx;
-        if (w != FYP) s_dmy[dm1 + 10] = st_1.dy;
-        if (w != FZP) s_dmz[dm1 + 100] = st_1.dz;
-        if (w == FXM) s_dmx[dm2 + 1] = st_2.dx;
-        if (w == FYM) s_dmy[dm2 + 10] = st_2.dy;
-        if (w == FZM) s_dmz[dm2 + 100] = st_2.dz;
-    } else if (edge) {
+        // depth-1 cell: every component whose target stays in [-1,9)^3 (one
+        // step: the minus faces of interior cells); depth-2 cell: only the
+        // normal component of a minus face
+        if (TWO ? w != FXP : w == FXM) s_dmx[dm1 + 1] = st_1.dx;
+        if (TWO ? w != FYP : w == FYM) s_dmy[dm1 + 10] = st_1.dy;
+        if (TWO ? w != FZP : w == FZM) s_dmz[dm1 + 100] = st_1.dz;
+        if (TWO) {
+            s_uu[uu2] = flag_in_sign(u_2, std::fabs(st_2.tau));
+            if (w == FXM) s_dmx[dm2 + 1] = st_2.dx;
+            if (w == FYM) s_dmy[dm2 + 10] = st_2.dy;
+            if (w == FZM) s_dmz[dm2 + 100] = st_2.dz;
+        }
+    } else if (TWO && edge) {
         s_uu[UU(ex, ey, ez)] = flag_in_sign(u_e, std::fabs(st_e.tau));
         // an edge cell feeds the minus face of a depth-1 cell across each of
         // its crossed axes at -1
@@ -791,32 +829,42 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(StepWork wk, const Real*
     // ---- step 1 on the interior cell and (waves 0-5) the depth-1 face cell;
     // the step-1 half of a row (offsets 13..22) is disjoint from the step-0
     // half (offsets 0..11), so the writes race with no read
-    const bool in_c = sign_of(st_c.tau) != 0;
+    auto step = [&](Real dmx, Real dmy, Real dmz, const Stat4<Real>& st, int q, Real u) {
+        return rd_step_enc<DOM, POW2>(dmx, st.dx, dmy, st.dy, dmz, st.dz, s_uu[q - 1], s_uu[q + 1], s_uu[q - 24],
+                                      s_uu[q + 24], s_uu[q - 293], s_uu[q + 293], u, sign_of(st.tau) != 0, rho, ih2,
+                                      dt);
+    };
     const Real dmx_c = s_dmx[dmc], dmy_c = s_dmy[dmc], dmz_c = s_dmz[dmc];
-    Real u1c;
-    {
-        const int q = uuc;
-        const Real d = rd_rhs_enc<Real>(dmx_c, st_c.dx, dmy_c, st_c.dy, dmz_c, st_c.dz, s_uu[q - 1], s_uu[q + 1],
-                                        s_uu[q - 24], s_uu[q + 24], s_uu[q - 293], s_uu[q + 293], u_c, in_c, rho, ih2);
-        u1c = rd_update(u_c, d, dt);
-        s_uu[q + UU1] = flag_in_sign(u1c, tau_c);
+    const Real u1c = step(dmx_c, dmy_c, dmz_c, st_c, uuc, u_c);
+    if constexpr (!TWO) {
+        (out + base)[ut] = u1c;
+    } else {
+        s_uu[uuc + UU1] = flag_in_sign(u1c, tau_c);
         if (mid) (mid + base)[ut] = u1c;  // the state after the first step, when asked for
+        if (w < 6)
+            s_uu[uu1 + UU1] = flag_in_sign(step(s_dmx[dm1], s_dmy[dm1], s_dmz[dm1], st_1, uu1, u_1), tau_1);
+        __syncthreads();
+        // ---- step 2 on the interior cell
+        (out + base)[ut] = step(dmx_c, dmy_c, dmz_c, st_c, uuc + UU1, u1c);
     }
-    if (w < 6) {
-        const int q = uu1;
-        const Real d = rd_rhs_enc<Real>(s_dmx[dm1], st_1.dx, s_dmy[dm1], st_1.dy, s_dmz[dm1], st_1.dz, s_uu[q - 1], s_uu[q + 1],
-                                        s_uu[q - 24], s_uu[q + 24], s_uu[q - 293], s_uu[q + 293], u_1,
-                                        sign_of(st_1.tau) != 0, rho, ih2);
-        s_uu[q + UU1] = flag_in_sign(rd_update(u_1, d, dt), tau_1);
-    }
-    __syncthreads();
+}
 
-    // ---- step 2 on the interior cell
-    {
-        const int q = uuc + UU1;
-        const Real d = rd_rhs_enc<Real>(dmx_c, st_c.dx, dmy_c, st_c.dy, dmz_c, st_c.dz, s_uu[q - 1], s_uu[q + 1],
-                                        s_uu[q - 24], s_uu[q + 24], s_uu[q - 293], s_uu[q + 293], u1c, in_c, rho, ih2);
-        (out + base)[ut] = rd_update(u1c, d, dt);
+// rd_step2f_kernel by the anatomy (plain: DOM = false) and the number of steps
+template <typename Real, typename Params>
+inline void launch_step2f_kernel(hipStream_t stream, const StepWork& wk, bool plain, bool two, const Real* in,
+                                 Real* out, Real* mid, const Stat4<Real>* stf, const Params& prm) {
+    const auto q = prm.args();
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(wk.grid()), dim3(512), 0, stream, wk.nfull, wk.fper, wk.full, in, stf, q.bpd,
+                           q.magic, q.slot_pos, q.range, out, mid, q.rho, q.ih2, q.dt, wk.ngrp, wk.gper, wk.grp,
+                           wk.still);
+    };
+    if (two) {
+        if (plain) go(rd_step2f_kernel<Real, Params, false, true>);
+        else go(rd_step2f_kernel<Real, Params, true, true>);
+    } else {
+        if (plain) go(rd_step2f_kernel<Real, Params, false, false>);
+        else go(rd_step2f_kernel<Real, Params, true, false>);
     }
 }
 

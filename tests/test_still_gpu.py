@@ -94,3 +94,52 @@ def test_gpu_still_groups_in_a_batch_match_single_solves():
         l1, g1, _ = b.adjoint(gh.Context.LIK_DEFAULT, ckpt_every=64)
         assert np.array_equal(l1[0], loss[i]) and np.array_equal(g1[0], grad[i]) and np.array_equal(b.get_phi(0), phi[i])
     b.close()
+
+
+@pytest.mark.parametrize("real", ["f32", "f64"])
+@pytest.mark.parametrize("cancel", [False, True])
+@pytest.mark.parametrize("n", [8, 24, 32])
+def test_gpu_clamped_steps_match_oracle_with_cancelling_cells(oracle, real, cancel, n):
+    """Pairs and the single odd step on clamped states against the oracle, with
+    and without cells of p_w = -p_g != 0 -- out of the domain, but with nonzero
+    face coefficients -- and, as a batch sample, on a grid of 3 blocks per side
+    (1 / h^2 is no power of two)."""
+    t = np.float32 if real == "f32" else np.float64
+    rng = np.random.default_rng(n)
+    wm = rng.uniform(0.1, 0.9, (n, n, n))
+    gm = rng.uniform(0, 1, (n, n, n)) * (1 - wm)
+    hole = rng.uniform(size=wm.shape) < 0.3
+    wm[hole] = 0
+    gm[hole] = 0
+    Dw, rho = 0.0021, 0.31
+    dt = 0.9 / (6 * n * n * Dw)
+    if n == 24:  # through the batch: its anatomies have no negative fractions
+        b = gh.Batch(0, real)
+        a = b.add_anatomy(3, gm, wm, 0 * wm)
+        pw, pg = b.get_anatomy(a)
+        for steps in (2, 3, 4, 9):
+            b.set_adjoint_samples([a], [(Dw, rho, steps * dt, 11.0, 12.0, 13.0)], [steps], 2.0, 0.7)
+            u0 = b.get_phi(0)
+            b.run()
+            ref = oracle.rd_steps(u0, pw, pg, t(Dw), t(Dw / 10), t(rho), t(1.0 / n), steps * dt / steps, steps)
+            assert np.array_equal(b.get_phi(0).view(np.uint8), ref.view(np.uint8)), steps
+        b.close()
+        return
+    pw, pg = wm.astype(t), gm.astype(t)
+    if cancel:
+        c = rng.uniform(size=pw.shape) < 0.1
+        pg[c] = -pw[c]
+    phi = rng.uniform(0, 0.4, pw.shape).astype(t)
+    phi[rng.uniform(size=pw.shape) < 0.4] = 0
+    ctx = gh.Context(0, real)
+    ctx.grid_init_uniform(n // 8)
+    for f, v in ((FIELD_PW, pw), (FIELD_PG, pg)):
+        ctx.set_field(f, v)
+    ctx.rd_prepare(Dw, Dw / 10, rho)
+    assert ctx.rd_schedule_info() == (0, True)
+    for steps in (3, 4, 10):
+        ctx.set_field(FIELD_PHI, phi)
+        ctx.rd_steps(steps, dt)
+        ref = oracle.rd_steps(phi, pw, pg, t(Dw), t(Dw / 10), t(rho), t(1.0 / n), dt, steps)
+        assert np.array_equal(ctx.get_field(FIELD_PHI).view(np.uint8), ref.view(np.uint8)), steps
+    ctx.close()
