@@ -117,14 +117,13 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
             const int mask_out = k >= 1;
             const StepWork& wk = k >= 1 ? moving : all;
             if (c.fast_ok && k >= 1)  // u_k is a clamped state: the clamped-state records
-                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams, true>), dim3(wk.grid()), dim3(512), 0,
-                                   c.stream, wk, uk, mask_out, c.adjLam[lc].as<double>(),
-                                   c.adjLam[1 - lc].as<double>(), c.statF.as<Stat4<Real>>(), (const Real*)nullptr,
-                                   prm, c.adjPart.as<double>());
+                launch_adj_step<true, Real>(c.stream, wk, uk, mask_out, c.adjLam[lc].as<double>(),
+                                            c.adjLam[1 - lc].as<double>(), c.statF.as<Stat4<Real>>(),
+                                            (const Real*)nullptr, prm, c.adjPart.as<double>());
             else
-                hipLaunchKernelGGL((adj_step_kernel<Real, UniformAdjParams>), dim3(wk.grid()), dim3(512), 0, c.stream,
-                                   wk, uk, mask_out, c.adjLam[lc].as<double>(), c.adjLam[1 - lc].as<double>(),
-                                   c.statD.as<Stat4<Real>>(), c.statSig.as<Real>(), prm, c.adjPart.as<double>());
+                launch_adj_step<false, Real>(c.stream, wk, uk, mask_out, c.adjLam[lc].as<double>(),
+                                             c.adjLam[1 - lc].as<double>(), c.statD.as<Stat4<Real>>(),
+                                             c.statSig.as<Real>(), prm, c.adjPart.as<double>());
             GH_HIP_CHECK(hipGetLastError());
             lc = 1 - lc;
         }

@@ -9,7 +9,17 @@
 
 namespace gh {
 
-__device__ inline int Q(int x, int y, int z) { return (z + 2) * 144 + (y + 2) * 12 + (x + 2); }  // [-2,10)^3
+// LDS tiles of the reverse step: states and flags Q on [-2,10)^3, weights W on
+// [-1,9)^3, with rows padded so that the 8 x 8 lanes of a wave meet few bank
+// conflicts; 40.2 KB in FP32, four workgroups a CU, and shorter rows in FP64.
+template <typename Real>
+struct AdjTile {
+    static constexpr int RQ = sizeof(Real) == 4 ? 24 : 12, PQ = sizeof(Real) == 4 ? 293 : 148;
+    static constexpr int RW = sizeof(Real) == 4 ? 24 : 12, PW = 10 * RW;
+    static constexpr int NQ = 12 * PQ, NW = 10 * PW;
+    __device__ static inline int Q(int x, int y, int z) { return (z + 2) * PQ + (y + 2) * RQ + (x + 2); }
+    __device__ static inline int W(int x, int y, int z) { return (z + 1) * PW + (y + 1) * RW + (x + 1); }
+};
 
 // Doubles of parameter-gradient partials per slot: per wave of the 512-lane
 // workgroup the two sums A = sum w_c Rdiff_c and B = sum w_c u_c (1 - u_c)
@@ -32,23 +42,30 @@ __device__ inline double dpp_move(double v) {
     const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
-__device__ inline double read_lane(double v, int lane) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+__device__ inline double double_of(unsigned lo, unsigned hi) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
-// Sum over the 64 lanes of a wave (all lanes active), valid in lanes 0-15.
-// Each 16-lane row is reduced by butterflies (lane pairs, quad halves, row
-// half mirror, row mirror) that leave the same row sum in every lane of the
-// row (floating-point addition commutes); the rows are then added in order
-// 0, 1, 2, 3.  Fixed order, no LDS, no barrier.
-__device__ inline double wave_sum_dpp(double v) {
+__device__ inline unsigned lo_of(double v) { return (unsigned)(unsigned long long)__double_as_longlong(v); }
+__device__ inline unsigned hi_of(double v) { return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32); }
+// Sums of a and of b over the 64 lanes of a wave (all lanes active): a's in
+// lanes 0-31, b's in lanes 32-63.  The halves of the wave are exchanged so that
+// one addition leaves a's 32 partial sums in the lower and b's in the upper
+// half, then the rows of 16 lanes, then butterflies within a row (lane pairs,
+// quad halves, row half mirror, row mirror: floating-point addition commutes,
+// so every lane of a row ends with the same sum).  Fixed order, no LDS, no
+// barrier; 21 operations for both sums (42 with one reduction each).
+__device__ inline double wave_sum2(double a, double b) {
+    auto lo = __builtin_amdgcn_permlane32_swap(lo_of(a), lo_of(b), false, false);
+    auto hi = __builtin_amdgcn_permlane32_swap(hi_of(a), hi_of(b), false, false);
+    double v = double_of(lo[0], hi[0]) + double_of(lo[1], hi[1]);
+    lo = __builtin_amdgcn_permlane16_swap(lo_of(v), lo_of(v), false, false);
+    hi = __builtin_amdgcn_permlane16_swap(hi_of(v), hi_of(v), false, false);
+    v = double_of(lo[0], hi[0]) + double_of(lo[1], hi[1]);
     v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
     v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
     v += dpp_move<0x141>(v);  // row_half_mirror
     v += dpp_move<0x140>(v);  // row_mirror
-    return ((v + read_lane(v, 16)) + read_lane(v, 32)) + read_lane(v, 48);
+    return v;
 }
 
 __device__ inline double block_sum(double v, double* red) {
@@ -63,11 +80,25 @@ __device__ inline double block_sum(double v, double* red) {
     return s;  // valid in thread 0
 }
 
+// adj_step_kernel's parameters as plain arguments (StepArgs)
+struct AdjArgs {
+    double rho, ih2, dt, invN, invDw;
+    int bpd;
+    uint32_t magic;
+    const int32_t* slot_pos;
+    const void* range;
+};
+
 // Per-slot parameters of the reverse step: one solve, or packed solves.
 struct UniformAdjParams {
     double rho, ih2, dt, invN, invDw;
     int bpd;
     uint32_t magic;  // bpd_magic(bpd)
+    __host__ __device__ static inline UniformAdjParams make(double r, double i, double d, double n, double w, int b,
+                                                            uint32_t m, const int32_t*, const void*) {
+        return {r, i, d, n, w, b, m};
+    }
+    AdjArgs args() const { return {rho, ih2, dt, invN, invDw, bpd, magic, nullptr, nullptr}; }
     __device__ inline void get(int, double& r, double& i, double& d, double& n, double& w) const {
         r = rho;
         i = ih2;
@@ -96,49 +127,65 @@ __device__ inline bool adj_outside(Real u, const Stat4<Real>& r) {
 }
 
 // Face halo cell (a, b) of face f at depth d (1 or 2): the cell index in the
-// neighbour block across the face and the tile indices Q (state, flags) and,
-// at depth 1, P (w), each base + a * step_a + b * step_b with wave-uniform
-// bases and steps.
+// neighbour block across the face and the tile indices q (state, flags) and,
+// at depth 1, p (w), each base + a * step_a + b * step_b with wave-uniform
+// bases and steps (selects: no branch for a uniform f).
 struct AdjHalo {
     int src, sa, sb, q, qa, qb, p, pa, pb;
 };
+template <typename Real>
 __device__ inline AdjHalo adj_halo(int f, int d) {
-    const int q0 = Q(0, 0, 0), p0 = P(0, 0, 0);
-    switch (f) {
-        case FXM: return {8 - d, 8, 64, q0 - d, 12, 144, p0 - d, 10, 100};
-        case FXP: return {d - 1, 8, 64, q0 + 7 + d, 12, 144, p0 + 7 + d, 10, 100};
-        case FYM: return {8 * (8 - d), 1, 64, q0 - 12 * d, 1, 144, p0 - 10 * d, 1, 100};
-        case FYP: return {8 * (d - 1), 1, 64, q0 + 12 * (7 + d), 1, 144, p0 + 10 * (7 + d), 1, 100};
-        case FZM: return {64 * (8 - d), 1, 8, q0 - 144 * d, 1, 12, p0 - 100 * d, 1, 10};
-        default:  return {64 * (d - 1), 1, 8, q0 + 144 * (7 + d), 1, 12, p0 + 100 * (7 + d), 1, 10};
-    }
+    using T = AdjTile<Real>;
+    const bool ax = f < 2, az = f >= 4;
+    const int out = f & 1 ? 7 + d : -d, in = f & 1 ? d - 1 : 8 - d;
+    return {(ax ? 1 : (az ? 64 : 8)) * in, ax ? 8 : 1, az ? 8 : 64,
+            T::Q(0, 0, 0) + (ax ? 1 : (az ? T::PQ : T::RQ)) * out, ax ? T::RQ : 1, az ? T::RQ : T::PQ,
+            T::W(0, 0, 0) + (ax ? 1 : (az ? T::PW : T::RW)) * out, ax ? T::RW : 1, az ? T::RW : T::PW};
 }
 
 // One cell of one reverse step: lambda_k (lk) and ih2 sum_i d'_i (u_i - u_c)
-// (rdiff) from the face coefficients D (-x, +x, -y, +y, -z, +z), per face i
-// the outside flags of the opposite neighbour (oo: face i ^ 1's neighbour) and
-// of the cell two steps out (of), the neighbour state un and weight wn, and
-// the cell's state u0, masked adjoint l1 and domain test.
-// nb(i, oo, of, un, wn) reads face i's neighbour data where it is used.
-template <typename Nb>
-__device__ inline void adj_cell(const double D[6], Nb nb, double u0, double l1, bool dom, double rho, double ih2,
-                                double dt, double& lk, double& rdiff) {
+// (rdiff) from the face coefficients (-x, +x, -y, +y, -z, +z), per face i the
+// outside flags of the opposite neighbour (that of face i ^ 1) and of the cell
+// two steps out, the neighbour state and weight, and the cell's state u0,
+// masked adjoint l1 and domain test.  axis(a) gives both faces of axis a; its
+// data are read axis by axis (64 registers: eight waves a SIMD).
+template <typename Real>
+struct AdjAxis {
+    Real dm, dp;      // face coefficients towards - and +
+    Real um, up;      // neighbour states
+    int om, op;       // their outside flags
+    int om2, op2;     // the flags of the cells two steps out
+    double wm, wp;    // neighbour weights
+};
+template <typename Axis>
+__device__ inline void adj_cell(Axis axis, double u0, double l1, bool dom, double rho, double ih2, double dt,
+                                double& lk, double& rdiff) {
     double sdu = 0, sumd = 0, acc = 0;
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        int oo, of;
-        double un, wn;
-        nb(i, oo, of, un, wn);
+    for (int a = 0; a < 3; ++a) {
+        const auto f = axis(a);
         // face coefficients doubled (exactly: ldexp by the 0/1 flag) where the
         // opposite neighbour of c, or of the neighbour, is outside
-        const double dp = ldexp(D[i], oo);
-        sdu = fma(dp, un, sdu);
-        sumd += dp;
-        acc = fma(wn, ldexp(D[i], of), acc);
+        auto face = [&](double d, int oo, int of, double un, double wn) {
+            const double dd = ldexp(d, oo);
+            sdu = fma(dd, un, sdu);
+            sumd += dd;
+            acc = fma(wn, ldexp(d, of), acc);
+        };
+        face((double)f.dm, f.op, f.om2, (double)f.um, f.wm);
+        face((double)f.dp, f.om, f.op2, (double)f.up, f.wp);
+        asm volatile("" : "+v"(sdu), "+v"(sumd), "+v"(acc));  // (the sums are formed here, not after the last axis)
     }
     rdiff = fma(-sumd, u0, sdu) * ih2;  // ih2 sum_i d'_i (u_i - u_c)
     const double self = dom ? l1 * (1. + dt * (-ih2 * sumd + rho * (1. - 2. * u0))) : l1;
     lk = self + dt * ih2 * acc;
+}
+
+// adds the wave's sums of a and b to its two words of block s
+__device__ inline void adj_accumulate(double* __restrict__ partial, int s, double a, double b) {
+    const double v = wave_sum2(a, b);
+    const int t = threadIdx.x;
+    if ((t & 31) == 0) partial[ADJ_PART * (size_t)s + 2 * (t >> 6) + ((t >> 5) & 1)] += v;
 }
 
 // lambda[c] = 0 where u[c] >= 1 (the upper clamp of the step that produced u
@@ -169,136 +216,159 @@ __global__ __launch_bounds__(256) void adj_mask_kernel(size_t n, double* __restr
 // data -- the same bits with no halo and no LDS.  A still group (still_kernel)
 // needs nothing at all for k >= 1: its adjoint stays what the seed put into
 // both buffers, and its sums are zeros.
+// Every load of a wave -- its cells' and its halo roles' -- is issued before the
+// first wait, the sums of the previous steps with them, and halo and interior
+// results keep registers of their own; with the interior stored to LDS before
+// the halos were loaded the kernel waited for memory three times (128^3 FP32
+// 7.6 -> 7.0 us with the tissue blocks only, 64^3 FP64 5.1 -> 4.4 us, a mixed
+// population 24.3 -> 21.7 us).  On clamped states a neighbour's outside flag travels in
+// the sign bit of its LDS copy (rd_step2f_kernel).
 template <typename Real, typename Params, bool CLAMPED = false>
-__global__ __launch_bounds__(512) void adj_step_kernel(StepWork wk, const Real* __restrict__ uk, int mask_out,
-                                                       const double* __restrict__ lam1, double* __restrict__ lam0,
-                                                       const Stat4<Real>* __restrict__ st,
-                                                       const Real* __restrict__ sig, Params prm,
-                                                       double* __restrict__ partial) {
+__global__ __launch_bounds__(512) void adj_step_kernel(
+    int nfull, int fper, const int32_t* __restrict__ full, const Real* __restrict__ uk,
+    const Stat4<Real>* __restrict__ st, int bpd, uint32_t magic, const int32_t* __restrict__ slot_pos,
+    const void* __restrict__ range, const double* __restrict__ lam1, double* __restrict__ lam0,
+    const Real* __restrict__ sig, double* __restrict__ partial, int mask_out, double rho_, double ih2_, double dt_,
+    double invN_, double invDw_, int ngrp, int gper, const int2* __restrict__ grp,
+    const unsigned char* __restrict__ still) {
+    const StepWork wk{nfull, fper, ngrp, gper, full, grp, still};
+    const Params prm = Params::make(rho_, ih2_, dt_, invN_, invDw_, bpd, magic, slot_pos, range);
     int nzf;
     const int s = wk.item(&nzf);
     if (s < 0) return;
     double rho, ih2, dt, invN, invDw;
     prm.get(s, rho, ih2, dt, invN, invDw);  // a group's blocks belong to one solve
+    const int t = threadIdx.x;
     for (int b = 0; b < nzf; ++b) {  // uniform per workgroup
-        const int t = threadIdx.x;
         const size_t g = (size_t)(s + b) * BCELLS + t;
         const Real uc = uk[g];
         const Stat4<Real> sv = st[g];
         const bool domc = adj_in_domain<CLAMPED>(uc, sv, sig, g);
         const double l1c = lam1[g];
         const double u0 = (double)uc;
-        const double D[6] = {0., 0., 0., 0., 0., 0.};
         double lk, rdiff;
-        adj_cell(
-            D,
-            [&](int, int& oo, int& of, double& un, double& wn) {
-                oo = 0;
-                of = 0;
-                un = 0.;
-                wn = 0.;
-            },
-            u0, l1c, domc, rho, ih2, dt, lk, rdiff);
+        adj_cell([](int) { return AdjAxis<Real>{0, 0, 0, 0, 0, 0, 0, 0, 0., 0.}; }, u0, l1c, domc, rho, ih2, dt, lk,
+                 rdiff);
         lam0[g] = (mask_out && !(uc < (Real)1)) ? 0.0 : lk;
         const double wc = domc ? l1c : 0.0;
-        const double A = wave_sum_dpp(wc * rdiff), B = wave_sum_dpp(wc * (u0 * (1. - u0)));
-        if ((t & 63) == 0) {
-            double* pw = partial + ADJ_PART * (size_t)(s + b) + 2 * (t >> 6);
-            pw[0] += A;
-            pw[1] += B;
-        }
+        adj_accumulate(partial, s + b, wc * rdiff, wc * (u0 * (1. - u0)));
     }
     if (nzf > 0) return;
-    __shared__ Real s_u[1728];
-    __shared__ unsigned char s_o[1728];
-    __shared__ double s_w[1000];
+    using T = AdjTile<Real>;
+    __shared__ Real s_u[T::NQ];
+    __shared__ unsigned char s_o[CLAMPED ? 1 : T::NQ];
+    __shared__ double s_w[T::NW];
     __shared__ Real s_Dx[576], s_Dy[576], s_Dz[576];
 
-    const int t = threadIdx.x;
     const int x = t & 7, y = (t >> 3) & 7, z = t >> 6;
-    const size_t g = (size_t)s * BCELLS + t;
-    const Real uc = uk[g];
-    const Stat4<Real> sv = st[g];
-    const bool domc = adj_in_domain<CLAMPED>(uc, sv, sig, g);
-    const double l1c = lam1[g];
-    s_u[Q(x, y, z)] = uc;
-    s_o[Q(x, y, z)] = adj_outside<CLAMPED>(uc, sv);
-    s_w[P(x, y, z)] = domc ? l1c : 0.0;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const size_t base = (size_t)s * BCELLS;
+    const unsigned ut = (unsigned)t;
+    const BlockPos bp = prm.pos(s);
+    // halo roles: waves 0-5 the depth-1 cells of face wv (state, flags, w,
+    // minus-face D), waves 6, 7 and 0-3 the depth-2 cells of faces 0-5 (state,
+    // flags)
+    const int f2 = wv >= 6 ? wv - 6 : wv + 2;
+    const bool deep = wv >= 6 || wv < 4;
+    Real u_1, u_2, tau_2;  // no defaults: merging them with loaded values would wait for the loads
+    Stat4<Real> st_1;
+    double l_1;
+    int q1 = 0, p1 = 0, q2 = 0;
+    bool dom_1 = false;
+    size_t g1 = 0;
+    if (wv < 6) {
+        const AdjHalo m = adj_halo<Real>(wv, 1);
+        const size_t nb = (size_t)face_nb(bp, wv) * BCELLS;
+        const unsigned l = (unsigned)mad24(y, m.sb, mad24(x, m.sa, m.src)) & (BCELLS - 1);
+        u_1 = (uk + nb)[l];
+        st_1 = (st + nb)[l];
+        l_1 = (lam1 + nb)[l];
+        g1 = nb + l;
+        q1 = mad24(y, m.qb, mad24(x, m.qa, m.q));
+        p1 = mad24(y, m.pb, mad24(x, m.pa, m.p));
+    }
+    if (deep) {
+        const AdjHalo m = adj_halo<Real>(f2, 2);
+        const size_t nb = (size_t)face_nb(bp, f2) * BCELLS;
+        const unsigned l = (unsigned)mad24(y, m.sb, mad24(x, m.sa, m.src)) & (BCELLS - 1);
+        u_2 = (uk + nb)[l];
+        tau_2 = (st + nb)[l].tau;
+        q2 = mad24(y, m.qb, mad24(x, m.qa, m.q));
+    }
+    const Real uc = (uk + base)[ut];
+    const Stat4<Real> sv = (st + base)[ut];
+    const double l1c = (lam1 + base)[ut];
+    double* pw = partial + ADJ_PART * (size_t)s + 2 * wv + ((t >> 5) & 1);
+    const double sum0 = *pw;  // the sums of the steps before
+    const bool domc = adj_in_domain<CLAMPED>(uc, sv, sig, base + ut);
+    if (wv < 6) dom_1 = adj_in_domain<CLAMPED>(u_1, st_1, sig, g1);
+
+    auto put = [&](int q, Real u, Real tau) {  // a state and its outside flag
+        if constexpr (CLAMPED) {
+            s_u[q] = flag_in_sign(u, std::fabs(tau));
+        } else {
+            s_u[q] = u;
+            s_o[q] = u < tau;
+        }
+    };
+    put(T::Q(x, y, z), uc, sv.tau);
+    s_w[T::W(x, y, z)] = domc ? l1c : 0.0;
     s_Dx[z * 72 + y * 9 + x + 1] = sv.dx;
     s_Dy[z * 72 + (y + 1) * 8 + x] = sv.dy;
     s_Dz[(z + 1) * 64 + y * 8 + x] = sv.dz;
-    // face halos: depth 1 (state, flags, w, minus-face D) and depth 2 (state,
-    // flags).  Halo wave hw = wave (first pass) or wave + 8 (second pass,
-    // waves 0-3) covers depth hw / 6, face hw % 6: wave-uniform (scalar) face
-    // logic, and every load of both passes is issued before the first store.
-    struct HaloCell {
-        size_t src;  // global cell
-        int q, p;    // tile indices (state/flags, w)
-    };
-    auto halo_cell = [&](int hw) {
-        const int f = hw % 6, d = hw / 6 + 1, a = t & 7, b = (t >> 3) & 7;
-        const AdjHalo m = adj_halo(f, d);
-        return HaloCell{(size_t)face_nb(prm.pos(s), f) * BCELLS + (size_t)mad24(b, m.sb, mad24(a, m.sa, m.src)),
-                        mad24(b, m.qb, mad24(a, m.qa, m.q)), mad24(b, m.pb, mad24(a, m.pa, m.p))};
-    };
-    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const HaloCell h0 = halo_cell(wv);
-    const Real u_h0 = uk[h0.src];
-    const Stat4<Real> s_h0 = st[h0.src];
-    double l_h0 = 0;
-    bool dom_h0 = false;
-    if (wv < 6) {  // depth 1
-        dom_h0 = adj_in_domain<CLAMPED>(u_h0, s_h0, sig, h0.src);
-        l_h0 = lam1[h0.src];
-    }
-    HaloCell h1{0, 0, 0};
-    Real u_h1 = 0;
-    Stat4<Real> s_h1{};
-    if (wv < 4) {  // second pass: depth 2, faces 2-5
-        h1 = halo_cell(wv + 8);
-        u_h1 = uk[h1.src];
-        s_h1 = st[h1.src];
-    }
-    s_u[h0.q] = u_h0;
-    s_o[h0.q] = adj_outside<CLAMPED>(u_h0, s_h0);
     if (wv < 6) {
-        const int a = t & 7, b = (t >> 3) & 7;
-        s_w[h0.p] = dom_h0 ? l_h0 : 0.0;
-        if (wv == FXM) s_Dx[b * 72 + a * 9] = s_h0.dx;
-        else if (wv == FYM) s_Dy[b * 72 + a] = s_h0.dy;
-        else if (wv == FZM) s_Dz[b * 8 + a] = s_h0.dz;
+        put(q1, u_1, st_1.tau);
+        s_w[p1] = dom_1 ? l_1 : 0.0;
+        if (wv == FXM) s_Dx[y * 72 + x * 9] = st_1.dx;
+        else if (wv == FYM) s_Dy[y * 72 + x] = st_1.dy;
+        else if (wv == FZM) s_Dz[y * 8 + x] = st_1.dz;
     }
-    if (wv < 4) {
-        s_u[h1.q] = u_h1;
-        s_o[h1.q] = adj_outside<CLAMPED>(u_h1, s_h1);
-    }
+    if (deep) put(q2, u_2, tau_2);
     __syncthreads();
 
     const double u0 = (double)uc;
-    const double D[6] = {(double)s_Dx[z * 72 + y * 9 + x], (double)sv.dx, (double)s_Dy[z * 72 + y * 8 + x],
-                         (double)sv.dy, (double)s_Dz[z * 64 + y * 8 + x], (double)sv.dz};
-    const int nq[6] = {Q(x - 1, y, z), Q(x + 1, y, z), Q(x, y - 1, z), Q(x, y + 1, z), Q(x, y, z - 1), Q(x, y, z + 1)};
-    const int np[6] = {P(x - 1, y, z), P(x + 1, y, z), P(x, y - 1, z), P(x, y + 1, z), P(x, y, z - 1), P(x, y, z + 1)};
-    const int n2[6] = {Q(x - 2, y, z), Q(x + 2, y, z), Q(x, y - 2, z), Q(x, y + 2, z), Q(x, y, z - 2), Q(x, y, z + 2)};
+    const int q0 = T::Q(x, y, z), w0 = T::W(x, y, z);
     double lk, rdiff;
     adj_cell(
-        D,
-        [&](int i, int& oo, int& of, double& un, double& wn) {
-            oo = s_o[nq[i ^ 1]];
-            of = s_o[n2[i]];
-            un = (double)s_u[nq[i]];
-            wn = s_w[np[i]];
+        [&](int a) {
+            const int dq = a == 0 ? 1 : (a == 1 ? T::RQ : T::PQ), dw = a == 0 ? 1 : (a == 1 ? T::RW : T::PW);
+            AdjAxis<Real> f;
+            f.dm = a == 0 ? s_Dx[z * 72 + y * 9 + x] : (a == 1 ? s_Dy[z * 72 + y * 8 + x] : s_Dz[z * 64 + y * 8 + x]);
+            f.dp = a == 0 ? sv.dx : (a == 1 ? sv.dy : sv.dz);
+            const Real em = s_u[q0 - dq], ep = s_u[q0 + dq];
+            if constexpr (CLAMPED) {
+                f.um = std::fabs(em);
+                f.up = std::fabs(ep);
+                f.om = (int)sign_of(em);
+                f.op = (int)sign_of(ep);
+                f.om2 = (int)sign_of(s_u[q0 - 2 * dq]);
+                f.op2 = (int)sign_of(s_u[q0 + 2 * dq]);
+            } else {
+                f.um = em;
+                f.up = ep;
+                f.om = s_o[q0 - dq];
+                f.op = s_o[q0 + dq];
+                f.om2 = s_o[q0 - 2 * dq];
+                f.op2 = s_o[q0 + 2 * dq];
+            }
+            f.wm = s_w[w0 - dw];
+            f.wp = s_w[w0 + dw];
+            return f;
         },
         u0, l1c, domc, rho, ih2, dt, lk, rdiff);
-    lam0[g] = (mask_out && !(uc < (Real)1)) ? 0.0 : lk;
+    (lam0 + base)[ut] = (mask_out && !(uc < (Real)1)) ? 0.0 : lk;
+    const double wc = domc ? l1c : 0.0;
+    const double v = sum0 + wave_sum2(wc * rdiff, wc * (u0 * (1. - u0)));
+    if ((t & 31) == 0) *pw = v;
+}
 
-    const double wc = s_w[P(x, y, z)];
-    const double A = wave_sum_dpp(wc * rdiff), B = wave_sum_dpp(wc * (u0 * (1. - u0)));
-    if ((t & 63) == 0) {
-        double* pw = partial + ADJ_PART * (size_t)s + 2 * (t >> 6);
-        pw[0] += A;
-        pw[1] += B;
-    }
+template <bool CLAMPED, typename Real, typename Params>
+inline void launch_adj_step(hipStream_t stream, const StepWork& wk, const Real* uk, int mask_out, const double* lam1,
+                            double* lam0, const Stat4<Real>* st, const Real* sig, const Params& prm, double* partial) {
+    const AdjArgs q = prm.args();
+    hipLaunchKernelGGL((adj_step_kernel<Real, Params, CLAMPED>), dim3(wk.grid()), dim3(512), 0, stream, wk.nfull,
+                       wk.fper, wk.full, uk, st, q.bpd, q.magic, q.slot_pos, q.range, lam1, lam0, sig, partial,
+                       mask_out, q.rho, q.ih2, q.dt, q.invN, q.invDw, wk.ngrp, wk.gper, wk.grp, wk.still);
 }
 
 // sum over cells of lam0 * u0 * (X - x0) / sigma^2 for X = ix, iy, iz, by

@@ -71,6 +71,11 @@ template <typename Real>
 struct BatchAdjParams {
     const int32_t* __restrict__ slot_pos;
     const SlotRange<Real>* __restrict__ range;
+    __host__ __device__ static inline BatchAdjParams make(double, double, double, double, double, int, uint32_t,
+                                                          const int32_t* sp, const void* r) {
+        return {sp, (const SlotRange<Real>*)r};
+    }
+    AdjArgs args() const { return {0., 0., 0., 0., 0., 0, 0u, slot_pos, range}; }
     __device__ inline void get(int s, double& r, double& i, double& d, double& n, double& w) const {
         const SlotRange<Real>& q = range[slot_pos[s]];
         r = q.rho_d;
@@ -774,17 +779,13 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
             const Real* uk = (const Real*)(tape + (size_t)(k - k0) * nsl * slot_bytes);
             const int mask_out = k >= 1;
             if (b.fast_ok && k >= 1)  // clamped states: the clamped-state records
-                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>, true>), dim3(wk.grid()), dim3(512),
-                                   0, b.stream, wk, uk, mask_out,
-                                   b.lam[(k + 1) & 1].as<double>(),
-                                   b.lam[k & 1].as<double>(), b.statF.as<Stat4<Real>>(), (const Real*)nullptr, aprm,
-                                   b.apart.as<double>());
+                launch_adj_step<true, Real>(b.stream, wk, uk, mask_out, b.lam[(k + 1) & 1].as<double>(),
+                                            b.lam[k & 1].as<double>(), b.statF.as<Stat4<Real>>(),
+                                            (const Real*)nullptr, aprm, b.apart.as<double>());
             else
-                hipLaunchKernelGGL((adj_step_kernel<Real, BatchAdjParams<Real>>), dim3(wk.grid()), dim3(512), 0,
-                                   b.stream, wk, uk, mask_out,
-                                   b.lam[(k + 1) & 1].as<double>(),
-                                   b.lam[k & 1].as<double>(), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(), aprm,
-                                   b.apart.as<double>());
+                launch_adj_step<false, Real>(b.stream, wk, uk, mask_out, b.lam[(k + 1) & 1].as<double>(),
+                                             b.lam[k & 1].as<double>(), b.statD.as<Stat4<Real>>(),
+                                             b.statSig.as<Real>(), aprm, b.apart.as<double>());
         }
         GH_HIP_CHECK(hipGetLastError());
     }
