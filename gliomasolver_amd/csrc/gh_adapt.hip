@@ -296,10 +296,12 @@ __global__ __launch_bounds__(256) void face_flag_kernel(int n, const int32_t* __
 }
 
 // the jump faces in slot-face order: faces[pos[i]] = i and pk_of[i] = pos[i]
-// for a jump face i = 6 * slot + f, pk_of[i] = -1 for the others
+// for a jump face i = 6 * slot + f, pk_of[i] = -1 for the others; code[i] =
+// the neighbour of the others
 __global__ __launch_bounds__(256) void face_list_kernel(int n, const int32_t* __restrict__ nbr6,
                                                         const int32_t* __restrict__ pos,
-                                                        int32_t* __restrict__ faces, int32_t* __restrict__ pk_of) {
+                                                        int32_t* __restrict__ faces, int32_t* __restrict__ pk_of,
+                                                        int32_t* __restrict__ code) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     if (nbr6[i] < 0) {
@@ -307,6 +309,7 @@ __global__ __launch_bounds__(256) void face_list_kernel(int n, const int32_t* __
         pk_of[i] = pos[i];
     } else {
         pk_of[i] = -1;
+        code[i] = nbr6[i];
     }
 }
 
@@ -381,6 +384,170 @@ __global__ __launch_bounds__(256) void face_packet_kernel(int n, const int32_t* 
         acc = acc + prod;
     }
     out[(size_t)faces[k] * 64 + p] = acc;
+}
+
+// Face-ghost patches.  Every ghost of a jump face is one cell (a finer
+// neighbour: the coincident vertex) or the Hs synthesis of level-(L-1) points,
+// all of which lie in one patch of the face: NT normal taps (one for a plus
+// face, whose ghosts have an even normal coordinate) by PT x PT tangential
+// points.  On a 2:1 grid each of these points is a single cell, so a face needs
+// its patch's cells once -- 196 at order 4, 49 for a plus face -- instead of a
+// source and a weight for each of its 64 ghosts' up to 64 terms; the ghosts are
+// summed from the patch in LDS with the same products in the same order.
+// A face with a point that needs a further synthesis sets bad, and the grid
+// takes the packets below.
+template <int ORDER>
+struct PatchGeom {
+    static constexpr int NT = ORDER == 4 ? 4 : 2, PT = ORDER == 4 ? 7 : 5;
+    static constexpr int T0 = ORDER == 4 ? -1 : 0;  // first tangential point, from 4 * index
+    static constexpr int N0 = ORDER == 4 ? -2 : -1; // first normal point of a minus face
+    static constexpr int MAX = NT * PT * PT;
+};
+constexpr int PATCH_STRIDE = 256;  // table entries per face
+constexpr int PATCH_FINER = 64;    // entries of a face towards a finer region
+
+// What a slot's face is, as the patched step reads it: the same-level
+// neighbour's slot, or -2 - (2 * patch + finer).  A patch's table row holds its
+// n cells: entry e of a patch of up to 64 in word e, of a larger one in word
+// 4 * (e % 64) + e / 64 -- one load of four words a lane either way.
+__device__ inline int patch_word(int n, int e) { return n > 64 ? 4 * (e & 63) + (e >> 6) : e; }
+template <int ORDER>
+__device__ inline int patch_cells(int f, bool finer) {
+    using G = PatchGeom<ORDER>;
+    return finer ? PATCH_FINER : (f & 1 ? G::PT * G::PT : G::MAX);
+}
+
+// one workgroup per jump face: the patch's cells (slot * 512 + cell) and the
+// face's code; *nf faces, the table holds at least gridDim.x of them
+template <int ORDER>
+__global__ __launch_bounds__(256) void face_patch_table_kernel(const int32_t* __restrict__ nf, const int32_t* __restrict__ faces,
+                                                               const int4* __restrict__ blk, LevelMaps m,
+                                                               int32_t* __restrict__ code, int32_t* __restrict__ tab,
+                                                               int* __restrict__ bad) {
+    using G = PatchGeom<ORDER>;
+    const int k = blockIdx.x, e = threadIdx.x;
+    if (k >= *nf) return;
+    const int sf = faces[k], s = sf / 6, f = sf % 6, a = f >> 1;
+    const int4 b = blk[s];
+    const int idx[3] = {b.y, b.z, b.w};
+    int L = b.x;
+    auto value = [&](int l, int x, int y, int z) {
+        return l < m.nlev ? m.map[dense_level_offset(l) + x + (y << l) + (z << (2 * l))] : hashed_node(m, l, x, y, z);
+    };
+    int nb[3] = {idx[0], idx[1], idx[2]};
+    nb[a] = (idx[a] + (f & 1 ? 1 : -1)) & ((1 << L) - 1);
+    const bool finer = L <= m.top && value(L, nb[0], nb[1], nb[2]) == -2;
+    const int n = patch_cells<ORDER>(f, finer);
+    if (e == 0) code[sf] = -2 - (2 * k + (finer ? 1 : 0));
+    if (n > 64 && e >= n) tab[(size_t)k * PATCH_STRIDE + patch_word(n, e)] = 0;  // read, not used
+    if (e >= n) return;
+    int q[3];
+    const int ta = a == 0 ? 1 : 0, tb = a == 2 ? 1 : 2;  // tangential axes
+    if (finer) {
+        q[a] = 8 * idx[a] + (f & 1 ? 8 : -1);
+        q[ta] = 8 * idx[ta] + (e & 7);
+        q[tb] = 8 * idx[tb] + (e >> 3);
+    } else {
+        --L;
+        const int tu = e % G::PT, tv = (e / G::PT) % G::PT, kn = e / (G::PT * G::PT);
+        q[a] = 4 * idx[a] + (f & 1 ? 4 : G::N0 + kn);
+        q[ta] = 4 * idx[ta] + G::T0 + tu;
+        q[tb] = 4 * idx[tb] + G::T0 + tv;
+    }
+    int32_t src = -1;
+    while (L >= 0 && L <= m.top) {  // ghost_visit's walk without synthesis
+        const int mask = (BS << L) - 1;
+        for (int c = 0; c < 3; ++c) q[c] &= mask;
+        const int32_t v = value(L, q[0] >> 3, q[1] >> 3, q[2] >> 3);
+        if (v >= 0) src = v * BCELLS + (q[0] & 7) + 8 * (q[1] & 7) + 64 * (q[2] & 7);
+        if (v != -2) break;
+        ++L;
+        for (int c = 0; c < 3; ++c) q[c] *= 2;
+    }
+    if (src < 0) {
+        atomicOr(bad, 1);
+        src = 0;
+    }
+    tab[(size_t)k * PATCH_STRIDE + patch_word(n, e)] = src;
+}
+
+// the ghost (u, v) = (lane & 7, lane >> 3) of face f from its patch p of n
+// values: the taps z-major, then y, then x (ghost_visit's order); wave-uniform
+// f; a coarser neighbour's face
+template <typename Real, int ORDER>
+__device__ inline Real patch_ghost(const Real* p, int f, int lane) {
+    using G = PatchGeom<ORDER>;
+    const int u = lane & 7, v = lane >> 3, a = f >> 1;
+    const int nn = f & 1 ? 1 : G::NT;
+    const int nu = u & 1 ? G::NT : 1, nv = v & 1 ? G::NT : 1;
+    // first tap of an odd coordinate c: (c - 3) / 2 (order 4) or (c - 1) / 2, from T0 on
+    const int iu = (u & 1 ? (ORDER == 4 ? (u - 3) / 2 : (u - 1) / 2) : u / 2) - G::T0;
+    const int iv = (v & 1 ? (ORDER == 4 ? (v - 3) / 2 : (v - 1) / 2) : v / 2) - G::T0;
+    auto w = [](int taps, int k) {
+        return taps == 1 ? (Real)1 : ORDER == 2 ? (Real)0.5 : (k == 0 || k == 3) ? (Real)(-1.0 / 16) : (Real)(9.0 / 16);
+    };
+    const Real* q = p + iu + G::PT * iv;
+    Real acc = (Real)0;
+    auto term = [&](int kn, int kv, int ku) {
+        // (the weights are dyadic: their product is exact in any order)
+        const Real prod = q[ku + G::PT * kv + G::PT * G::PT * kn] * (w(nv, kv) * w(nn, kn) * w(nu, ku));
+        acc = acc + prod;
+    };
+    if (a == 0) {  // x normal: v = z, u = y
+        for (int kv = 0; kv < nv; ++kv)
+            for (int ku = 0; ku < nu; ++ku)
+                for (int kn = 0; kn < nn; ++kn) term(kn, kv, ku);
+    } else if (a == 1) {  // y normal: v = z, u = x
+        for (int kv = 0; kv < nv; ++kv)
+            for (int kn = 0; kn < nn; ++kn)
+                for (int ku = 0; ku < nu; ++ku) term(kn, kv, ku);
+    } else {  // z normal: v = y, u = x
+        for (int kn = 0; kn < nn; ++kn)
+            for (int kv = 0; kv < nv; ++kv)
+                for (int ku = 0; ku < nu; ++ku) term(kn, kv, ku);
+    }
+    return acc;
+}
+
+// the ghosts of two fields from the patches, one wave per jump face (p_w and
+// p_g for the constants)
+template <typename Real, int ORDER>
+__global__ __launch_bounds__(256) void face_patch_kernel(int nf, const int32_t* __restrict__ faces,
+                                                         const int32_t* __restrict__ code,
+                                                         const int32_t* __restrict__ tab, const Real* __restrict__ f0,
+                                                         const Real* __restrict__ f1, Real* __restrict__ out0,
+                                                         Real* __restrict__ out1) {
+    using G = PatchGeom<ORDER>;
+    __shared__ Real s_p[4][2][256];
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int k = 4 * (int)blockIdx.x + w;
+    if (k >= nf) return;
+    const int sf = faces[k], f = sf % 6;
+    const bool finer = (-2 - code[sf]) & 1;
+    const int n = patch_cells<ORDER>(f, finer);
+    const int32_t* row = tab + (size_t)k * PATCH_STRIDE;
+    if (finer) {
+        const int32_t src = row[lane];
+        out0[(size_t)sf * 64 + lane] = (Real)0 + f0[src];  // the one term of weight 1
+        out1[(size_t)sf * 64 + lane] = (Real)0 + f1[src];
+        return;
+    }
+    if (n > 64) {
+        const int4 q = reinterpret_cast<const int4*>(row)[lane];
+        const int32_t src[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s_p[w][0][lane + 64 * j] = f0[src[j]];
+            s_p[w][1][lane + 64 * j] = f1[src[j]];
+        }
+    } else if (lane < n) {
+        const int32_t src = row[lane];
+        s_p[w][0][lane] = f0[src];
+        s_p[w][1][lane] = f1[src];
+    }
+    __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations are in order
+    out0[(size_t)sf * 64 + lane] = patch_ghost<Real, ORDER>(s_p[w][0], f, lane);
+    out1[(size_t)sf * 64 + lane] = patch_ghost<Real, ORDER>(s_p[w][1], f, lane);
 }
 
 // BlockFWT::_fwt / _filter (MRAGBlockFWT.h:219-298): 64 coarse points x 8
@@ -985,6 +1152,130 @@ __global__ __launch_bounds__(NT) void rd_step_ghosted_kernel(int nslots, int per
     }
 }
 
+// RD step on a multi-level grid with patches: the wave that owns a jump face
+// gathers the face's patch (its indices known since the grid changed) into LDS
+// and sums its 64 ghosts there, while the block's own loads are in flight; one
+// launch per step.  NT lanes, 512 / NT cells each; wave w has the planes and
+// the faces w, w + NT / 64, ...  1,900 / 3,816 blocks, FP32: 11.1 / 14.2 us a
+// step instead of 12.5 (packets summed in the step) / 28.2 us (packet kernel and
+// step); the constants' face tables 12 instead of 150 us.
+template <typename Real, bool FUSED, int ORDER, int NT>
+__global__ __launch_bounds__(NT) void rd_step_patched_kernel(
+    int nslots, int per_xcd, const int32_t* __restrict__ code, const Real* __restrict__ phi,
+    const Stat4<Real>* __restrict__ st, const int32_t* __restrict__ tab, const int32_t* __restrict__ level,
+    const Real* __restrict__ sig, Real* __restrict__ out, const Real* __restrict__ fgTau,
+    const Real* __restrict__ fgDm, Real rho, double dt) {
+    constexpr int NW = NT / 64, C = 8 / NW;
+    const int s = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    if (s >= nslots) return;
+    __shared__ Real s_phi[1000];
+    __shared__ unsigned char s_out[1000];
+    __shared__ Real s_Dx[576], s_Dy[576], s_Dz[576];
+    __shared__ Real s_patch[NW < 6 ? NW : 6][256];
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int u = t & 7, v = (t >> 3) & 7;
+    const size_t base = (size_t)s * BCELLS;
+    int cd[C], lev = level[s];
+#pragma unroll
+    for (int c = 0; c < C; ++c) cd[c] = code[6 * s + (w + c * NW < 6 ? w + c * NW : 0)];
+    // all loads before the first wait; the same-level halo and the patch keep
+    // registers of their own
+    Real pc[C], sc[C], hp[C], gt[C], gd[C], pv[C][4];
+    Stat4<Real> sv[C], hs[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const unsigned i = (unsigned)(t + c * NT);
+        pc[c] = (phi + base)[i];
+        sv[c] = (st + base)[i];
+        sc[c] = (sig + base)[i];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int f = w + c * NW;
+        if (f >= 6) continue;
+        if (cd[c] >= 0) {
+            const int l0 = f & 1 ? 0 : 7;  // the neighbour's layer at the face
+            const unsigned l = (unsigned)(f < 2 ? l0 + 8 * u + 64 * v : (f < 4 ? u + 8 * l0 + 64 * v : u + 8 * v + 64 * l0));
+            const size_t nb = (size_t)cd[c] * BCELLS;
+            hs[c] = (st + nb)[l];
+            hp[c] = (phi + nb)[l];
+        } else {
+            const int k = (-2 - cd[c]) >> 1;
+            const int32_t* row = tab + (size_t)k * PATCH_STRIDE;
+            if (patch_cells<ORDER>(f, (-2 - cd[c]) & 1) > 64) {
+                const int4 q = reinterpret_cast<const int4*>(row)[lane];
+                pv[c][0] = phi[q.x];
+                pv[c][1] = phi[q.y];
+                pv[c][2] = phi[q.z];
+                pv[c][3] = phi[q.w];
+            } else if (lane < patch_cells<ORDER>(f, (-2 - cd[c]) & 1)) {
+                pv[c][0] = phi[row[lane]];
+            }
+            gt[c] = (fgTau + (size_t)s * 384)[64 * f + lane];
+            gd[c] = (fgDm + (size_t)s * 192)[32 * (f & 6) + lane];
+        }
+    }
+    const double ih2 = ldexp(64.0, 2 * lev);  // 1 / h^2, h = 2^-level / 8 (MRAGrid.inl:200-206)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int z = w + c * NW;
+        s_phi[P(u, v, z)] = pc[c];
+        s_out[P(u, v, z)] = pc[c] < sv[c].tau;
+        s_Dx[z * 72 + v * 9 + u + 1] = sv[c].dx;
+        s_Dy[z * 72 + (v + 1) * 8 + u] = sv[c].dy;
+        s_Dz[(z + 1) * 64 + v * 8 + u] = sv[c].dz;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int f = w + c * NW;
+        if (f >= 6) continue;
+        const int o = f & 1 ? 8 : -1;
+        const int dst = f < 2 ? P(o, u, v) : (f < 4 ? P(u, o, v) : P(u, v, o));
+        auto put = [&](Real ph, Real tau, Real dx, Real dy, Real dz) {
+            s_phi[dst] = ph;
+            s_out[dst] = ph < tau;
+            if (f == FXM) s_Dx[v * 72 + u * 9] = dx;
+            else if (f == FYM) s_Dy[v * 72 + u] = dy;
+            else if (f == FZM) s_Dz[v * 8 + u] = dz;
+        };
+        if (cd[c] >= 0) {
+            put(hp[c], hs[c].tau, hs[c].dx, hs[c].dy, hs[c].dz);
+        } else if ((-2 - cd[c]) & 1) {  // a finer neighbour: the coincident vertex, one term of weight 1
+            put((Real)0 + pv[c][0], gt[c], gd[c], gd[c], gd[c]);
+        } else {
+            Real* p = s_patch[w];
+            if (patch_cells<ORDER>(f, false) > 64) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) p[lane + 64 * j] = pv[c][j];
+            } else {
+                p[lane] = pv[c][0];  // (lanes past the patch: not used)
+            }
+            __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations are in order
+            const Real g = patch_ghost<Real, ORDER>(p, f, lane);
+            __builtin_amdgcn_wave_barrier();
+            put(g, gt[c], gd[c], gd[c], gd[c]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int x = u, y = v, z = w + c * NW;
+        Real d0 = s_Dx[z * 72 + y * 9 + x], d1 = sv[c].dx, d2 = s_Dy[z * 72 + y * 8 + x], d3 = sv[c].dy;
+        Real d4 = s_Dz[z * 64 + y * 8 + x], d5 = sv[c].dz;
+        d1 = twice_if(d1, s_out[P(x - 1, y, z)]);  // _applyNoFluxBC: an outside neighbour doubles the opposite face
+        d0 = twice_if(d0, s_out[P(x + 1, y, z)]);
+        d3 = twice_if(d3, s_out[P(x, y - 1, z)]);
+        d2 = twice_if(d2, s_out[P(x, y + 1, z)]);
+        d5 = twice_if(d5, s_out[P(x, y, z - 1)]);
+        d4 = twice_if(d4, s_out[P(x, y, z + 1)]);
+        const Real r = rd_rhs_pow2<Real>(d0, d1, d2, d3, d4, d5, s_phi[P(x - 1, y, z)], s_phi[P(x + 1, y, z)],
+                                         s_phi[P(x, y - 1, z)], s_phi[P(x, y + 1, z)], s_phi[P(x, y, z - 1)],
+                                         s_phi[P(x, y, z + 1)], pc[c], pc[c] > sc[c], rho, ih2);
+        (out + base)[(unsigned)(t + c * NT)] = FUSED ? rd_update(pc[c], r, dt) : r;
+    }
+}
+
 // _dumpUQoutput (Glioma_ReactionDiffusion.cpp:208-267): leaf cells onto the
 // finest uniform gpd^3 lattice; h = hf writes 1, 2hf writes 2^3, 3hf writes
 // 3^3 and anything coarser writes 4^3 cells (the reference's quirk is kept)
@@ -1163,6 +1454,7 @@ HostTable build_lab_table(const Octree& t, const std::vector<int>& slots, const 
 // the device recursion (the caller then builds it on the host).
 int device_face_table(Ctx& c, bool& done) {
     done = false;
+    c.nFacePatch = 0;
     c.nFacePk = 0;
     c.nFaceEnt = 0;
     const int nb = c.topo.nblocks();
@@ -1170,7 +1462,7 @@ int device_face_table(Ctx& c, bool& done) {
     int rc;
     DevBuf& dfaces = c.faceList;  // kept across calls: no allocation per adaptation
     if ((rc = c.faceScan.ensure_grow(((size_t)n6 + 1) * 4)) || (rc = dfaces.ensure_grow(std::max(1, n6) * 4)) ||
-        (rc = c.facePkOf.ensure_grow(std::max(1, n6) * 4)))
+        (rc = c.facePkOf.ensure_grow(std::max(1, n6) * 4)) || (rc = c.faceCode.ensure_grow(std::max(1, n6) * 4)))
         return rc;
     // the jump faces in slot-face order, listed on the device from the
     // neighbour table: flags, their exclusive prefix sum, the list
@@ -1188,20 +1480,41 @@ int device_face_table(Ctx& c, bool& done) {
         hipLaunchKernelGGL(scan_chunk_apply, dim3(nch), dim3(1024), 0, c.stream, np6, pos, sums + nch);
         if (n6 > 0)
             hipLaunchKernelGGL(face_list_kernel, dim3((unsigned)((n6 + 255) / 256)), dim3(256), 0, c.stream, n6,
-                               c.nbr.as<int32_t>(), pos, dfaces.as<int32_t>(), c.facePkOf.as<int32_t>());
+                               c.nbr.as<int32_t>(), pos, dfaces.as<int32_t>(), c.facePkOf.as<int32_t>(),
+                               c.faceCode.as<int32_t>());
         GH_HIP_CHECK(hipGetLastError());
     }
-    int nf = 0;
-    GH_HIP_CHECK(hipMemcpyAsync(&nf, pos + n6, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    const int n = nf * 64;
-    if (n == 0) {
-        done = true;
-        return GH_OK;
-    }
+    // the patches, for as many faces as the table of the grid before has room,
+    // before the number of faces is known: one synchronization for both
     const LevelMaps m = level_maps(c);
     const int order = c.tree.order;
     DevBuf& dcount = c.faceCount;
+    int nf = 0, bad = 1;
+    for (int cap = std::min<int64_t>(n6, (int64_t)(c.faceSrc.bytes / (PATCH_STRIDE * 4)));;) {
+        GH_HIP_CHECK(hipMemsetAsync(c.dBad.p, 0, sizeof(int), c.stream));
+        if (cap > 0) {
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(cap), dim3(256), 0, c.stream, pos + n6, dfaces.as<int32_t>(),
+                                   c.dBlk.as<int4>(), m, c.faceCode.as<int32_t>(), c.faceSrc.as<int32_t>(),
+                                   c.dBad.as<int>());
+            };
+            if (order == 4) go(face_patch_table_kernel<4>);
+            else go(face_patch_table_kernel<2>);
+            GH_HIP_CHECK(hipGetLastError());
+        }
+        GH_HIP_CHECK(hipMemcpyAsync(&nf, pos + n6, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
+        GH_HIP_CHECK(hipMemcpyAsync(&bad, c.dBad.p, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+        GH_HIP_CHECK(hipStreamSynchronize(c.stream));
+        if (nf <= cap) break;
+        if ((rc = c.faceSrc.ensure_grow((size_t)nf * PATCH_STRIDE * 4))) return rc;
+        cap = nf;
+    }
+    if (!bad) {
+        c.nFacePatch = nf;
+        done = true;
+        return GH_OK;
+    }
+    const int n = nf * 64;
     if ((rc = dcount.ensure_grow((size_t)n * 4)) || (rc = c.facePkBase.ensure_grow(((size_t)nf + 1) * 4))) return rc;
     GH_HIP_CHECK(hipMemsetAsync(c.dBad.p, 0, sizeof(int), c.stream));
     GH_HIP_CHECK(hipMemsetAsync(c.facePkBase.as<int32_t>() + nf, 0, sizeof(int32_t), c.stream));
@@ -1222,7 +1535,6 @@ int device_face_table(Ctx& c, bool& done) {
                        sums + 2 * nchunk);
     hipLaunchKernelGGL(scan_chunk_apply, dim3(nchunk), dim3(1024), 0, c.stream, np, pk, sums + nchunk);
     GH_HIP_CHECK(hipGetLastError());
-    int bad = 1;
     long long total = 0;
     GH_HIP_CHECK(hipMemcpyAsync(&total, sums + 2 * nchunk, sizeof(long long), hipMemcpyDeviceToHost, c.stream));
     GH_HIP_CHECK(hipMemcpyAsync(&bad, c.dBad.p, sizeof(int), hipMemcpyDeviceToHost, c.stream));
@@ -1318,6 +1630,7 @@ int apply_topology(Ctx& c) {
         GH_HIP_CHECK(hipGetLastError());
     }
     c.faces_stale = true;  // built by ensure_faces when an RD step or the constants need them
+    c.nFacePatch = 0;
     c.nFacePk = 0;
     c.nFaceEnt = 0;
     const size_t rs = c.real_size;
@@ -1392,9 +1705,20 @@ int face_ghosts(Ctx& c, const Real* field, Real* out) {
 template <typename Real>
 int prepare_ghosted_t(Ctx& c, double Dw, double Dg) {
     int rc;
-    if ((rc = ensure_faces(c)) || (rc = face_ghosts<Real>(c, c.pw.as<Real>(), c.fgPw.as<Real>())) ||
-        (rc = face_ghosts<Real>(c, c.pg.as<Real>(), c.fgPg.as<Real>())))
+    if ((rc = ensure_faces(c))) return rc;
+    if (c.nFacePatch > 0) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((c.nFacePatch + 3) / 4), dim3(256), 0, c.stream, c.nFacePatch,
+                               c.faceList.as<int32_t>(), c.faceCode.as<int32_t>(), c.faceSrc.as<int32_t>(),
+                               c.pw.as<Real>(), c.pg.as<Real>(), c.fgPw.as<Real>(), c.fgPg.as<Real>());
+        };
+        if (c.tree.order == 4) go(face_patch_kernel<Real, 4>);
+        else go(face_patch_kernel<Real, 2>);
+        GH_HIP_CHECK(hipGetLastError());
+    } else if ((rc = face_ghosts<Real>(c, c.pw.as<Real>(), c.fgPw.as<Real>())) ||
+               (rc = face_ghosts<Real>(c, c.pg.as<Real>(), c.fgPg.as<Real>()))) {
         return rc;
+    }
     const int ns = c.topo.nblocks();
     const size_t nc = c.ncells();
     hipLaunchKernelGGL(statics_ghosted_kernel<Real>, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, c.stream, ns,
@@ -1405,6 +1729,11 @@ int prepare_ghosted_t(Ctx& c, double Dw, double Dg) {
     return GH_OK;
 }
 
+// Largest FP32 grid whose patched step has 512 lanes a block; above it 256 lanes
+// of two cells (more blocks in flight a CU): 500 / 3,816 / 9,500 blocks 5.4 /
+// 14.8 / 32.1 us with 512, 6.2 / 14.2 / 28.6 us with 256.  In FP64 512 is the
+// faster at every size measured (3,816 blocks: 21.2 and 22.9 us).
+constexpr int kPatchedFewBlocks = 2500;
 constexpr int kFusedGhostMaxBlocks = 1450;  // largest grid whose step kernel gathers its own ghosts
 
 // The step kernel with 512 lanes per block when it gathers the face ghosts
@@ -1433,6 +1762,25 @@ int step_ghosted_t(Ctx& c, const Real* in, Real* out, double dt) {
     if (rc0) return rc0;
     const int ns = c.topo.nblocks();
     const int per_xcd = (ns + 7) / 8;
+    if (c.nFacePatch > 0) {
+        auto go = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(8 * per_xcd), dim3(lanes), 0, c.stream, ns, per_xcd, c.faceCode.as<int32_t>(), in,
+                               c.statD.as<Stat4<Real>>(), c.faceSrc.as<int32_t>(), c.dLevel.as<int32_t>(),
+                               c.statSig.as<Real>(), out, c.fgTau.as<Real>(), c.fgDm.as<Real>(), (Real)c.rho, dt);
+        };
+        constexpr int MANY = sizeof(Real) == 4 ? 256 : 512;
+        const bool few = ns <= kPatchedFewBlocks;
+        if (c.tree.order == 4) {
+            if (few) go(rd_step_patched_kernel<Real, FUSED, 4, 512>, 512);
+            else go(rd_step_patched_kernel<Real, FUSED, 4, MANY>, MANY);
+        } else {
+            if (few) go(rd_step_patched_kernel<Real, FUSED, 2, 512>, 512);
+            else go(rd_step_patched_kernel<Real, FUSED, 2, MANY>, MANY);
+        }
+        GH_HIP_CHECK(hipGetLastError());
+        return GH_OK;
+    }
+    // Packets (a face with a ghost of two synthesis levels).
     // Small grids: ghosts summed inside the step kernel (one launch per step).
     // Larger grids: a packet kernel first, whose one-thread-per-ghost gather
     // hides the scattered reads better than the step kernel's ghost threads,

@@ -92,8 +92,13 @@ struct Ctx {
     // lists interleaved (term k of ghost p at facePkBase[face] + 64 k + p for
     // k below its own term count in faceCount), so a wave's loads are contiguous
     DevBuf facePkBase;               // int32 per face + 1: packet starts (exclusive scan)
+    DevBuf faceCode;                 // int32 per slot face: neighbour slot or patch (patched step)
     DevBuf facePkOf;                 // int32 per slot face: its packet (index in the face list), -1 if none
     int nFacePk = 0;                 // faces in packets (0: the GhostEntry table is used)
+    // device-built face table in patches (every ghost of the grid from single
+    // cells of its face's patch): cells in faceSrc, a face's neighbour
+    // or patch in faceCode; 0: packets or the GhostEntry table
+    int nFacePatch = 0;
     DevBuf fgPhi, fgTau, fgDm;       // per slot: 6*64 ghost phi, 6*64 ghost tau, 3*64 minus-face D
     DevBuf fgPw, fgPg;               // per slot: 6*64 ghost p_w, p_g (statics)
     // FWT / split labs (compact, one per listed slot)

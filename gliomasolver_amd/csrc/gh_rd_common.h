@@ -479,36 +479,18 @@ __device__ inline double twice_if(double d, uint32_t o) { return __builtin_amdgc
 template <typename Real>
 __device__ inline Real flag_in_sign(Real u, Real tau) { return u < tau ? -u : u; }
 
-// The state after one step from encoded neighbours e0..e5 (-x,+x,-y,+y,-z,+z)
-// and the face coefficients d0..d5 before the no-flux rule: rd_rhs_core and
-// rd_update with fewer operations and the same bits.
-//   DOM = false (every cell has p_w + p_g != 0 or p_w = p_g = 0): a cell out of
-//     the domain has six zero face coefficients and the state 0, so its dphidt
-//     comes out +0 without the test.
-//   POW2 (1/h^2 a power of two): the scalings of both fluxes are exact, so
-//     ih2*in - ih2*out = ih2*(in - out), and the sum with the reaction is one
-//     fused multiply-add of an exact product.
-template <bool DOM, bool POW2, typename Real>
-__device__ inline Real rd_step_enc(Real d0, Real d1, Real d2, Real d3, Real d4, Real d5, Real e0, Real e1, Real e2,
-                                   Real e3, Real e4, Real e5, Real pc, bool inside, Real rho, double ih2, double dt) {
-    d1 = twice_if(d1, sign_of(e0));
-    d0 = twice_if(d0, sign_of(e1));
-    d3 = twice_if(d3, sign_of(e2));
-    d2 = twice_if(d2, sign_of(e3));
-    d5 = twice_if(d5, sign_of(e4));
-    d4 = twice_if(d4, sign_of(e5));
-    if constexpr (!POW2)
-        return rd_update(pc,
-                         rd_rhs_core<Real>(d0, d1, d2, d3, d4, d5, std::fabs(e0), std::fabs(e1), std::fabs(e2),
-                                           std::fabs(e3), std::fabs(e4), std::fabs(e5), pc,
-                                           !DOM || inside || pc > (Real)0., rho, ih2),
-                         dt);
-    Real sin_ = d0 * std::fabs(e0);
-    sin_ = sin_ + d1 * std::fabs(e1);
-    sin_ = sin_ + d2 * std::fabs(e2);
-    sin_ = sin_ + d3 * std::fabs(e3);
-    sin_ = sin_ + d4 * std::fabs(e4);
-    sin_ = sin_ + d5 * std::fabs(e5);
+// rd_rhs_core where 1/h^2 is a power of two: the scalings of both fluxes are
+// exact, so ih2*in - ih2*out = ih2*(in - out), and the sum with the reaction is
+// one fused multiply-add of an exact product.  The same bits.
+template <typename Real>
+__device__ inline Real rd_rhs_pow2(Real d0, Real d1, Real d2, Real d3, Real d4, Real d5, Real p0, Real p1, Real p2,
+                                   Real p3, Real p4, Real p5, Real pc, bool dom, Real rho, double ih2) {
+    Real sin_ = d0 * p0;
+    sin_ = sin_ + d1 * p1;
+    sin_ = sin_ + d2 * p2;
+    sin_ = sin_ + d3 * p3;
+    sin_ = sin_ + d4 * p4;
+    sin_ = sin_ + d5 * p5;
     Real sdf = d0 + d1;
     sdf = sdf + d2;
     sdf = sdf + d3;
@@ -518,7 +500,30 @@ __device__ inline Real rd_step_enc(Real d0, Real d1, Real d2, Real d3, Real d4, 
     const Real rp = rho * pc;
     const double react = (double)rp * (1. - (double)pc);
     const Real dphidt = (Real)__builtin_fma((double)sin_ - (double)sdp, ih2, react);
-    return rd_update(pc, !DOM || inside || pc > (Real)0. ? dphidt : (Real)0., dt);
+    return dom ? dphidt : (Real)0.;
+}
+
+// The state after one step from encoded neighbours e0..e5 (-x,+x,-y,+y,-z,+z)
+// and the face coefficients d0..d5 before the no-flux rule.  DOM = false (every
+// cell has p_w + p_g != 0 or p_w = p_g = 0): a cell out of the domain has six
+// zero face coefficients and the state 0, so its dphidt comes out +0 without the
+// test.  POW2: rd_rhs_pow2.
+template <bool DOM, bool POW2, typename Real>
+__device__ inline Real rd_step_enc(Real d0, Real d1, Real d2, Real d3, Real d4, Real d5, Real e0, Real e1, Real e2,
+                                   Real e3, Real e4, Real e5, Real pc, bool inside, Real rho, double ih2, double dt) {
+    d1 = twice_if(d1, sign_of(e0));
+    d0 = twice_if(d0, sign_of(e1));
+    d3 = twice_if(d3, sign_of(e2));
+    d2 = twice_if(d2, sign_of(e3));
+    d5 = twice_if(d5, sign_of(e4));
+    d4 = twice_if(d4, sign_of(e5));
+    const bool dom = !DOM || inside || pc > (Real)0.;
+    const Real p0 = std::fabs(e0), p1 = std::fabs(e1), p2 = std::fabs(e2), p3 = std::fabs(e3), p4 = std::fabs(e4),
+               p5 = std::fabs(e5);
+    return rd_update(pc,
+                     POW2 ? rd_rhs_pow2<Real>(d0, d1, d2, d3, d4, d5, p0, p1, p2, p3, p4, p5, pc, dom, rho, ih2)
+                          : rd_rhs_core<Real>(d0, d1, d2, d3, d4, d5, p0, p1, p2, p3, p4, p5, pc, dom, rho, ih2),
+                     dt);
 }
 
 // {dx, dy, dz, tau} + sigma -> the record of rd_step2f_kernel; counts the
