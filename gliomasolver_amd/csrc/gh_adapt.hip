@@ -614,8 +614,12 @@ __device__ __forceinline__ Real fwt_code(const Real* __restrict__ p) {
 // Lanes per lab: 512 while the labs are fewer than the CUs can hold several
 // of, 256 beyond that (more labs in flight per CU hide the dependent map and
 // field loads better; at least 256: the FWT epilogue takes four waves).
-// Details of 1,114 / 7,225 / 13,455 blocks: 0.12 / 0.41 / 0.54 ms with 512,
-// 0.15 / 0.38 / 0.47 ms with 256 lanes.
+// Details of 7,225 / 13,455 blocks when the line was drawn: 0.41 / 0.54 ms with
+// 512, 0.38 / 0.47 ms with 256 lanes.  With the plain tap sums of all_single
+// (three operations a term instead of about ten) and the regions looked up once
+// instead of per point the labs of a 1,900-block grid's details take 25 us
+// instead of 62, of its 5,000 blocks after a refinement 66 instead of 168, the
+// four-field labs of a refinement 26 instead of 46.
 constexpr int kLabThreadsFewMax = 2048;  // largest list built with 512 lanes per lab
 // up to four fields whose labs are built together: the ghost recursion (map
 // lookups, terms, weights) runs once and each field accumulates its own sum
@@ -631,7 +635,6 @@ struct LabFields {
 // the lab out.
 template <typename Real, int NF, int ORDER, bool FWT, int LAB_THREADS>
 __global__ __launch_bounds__(LAB_THREADS) void lab_kernel(int nlist, const int32_t* __restrict__ slots,
-                                                  const int32_t* __restrict__ nbr27,
                                                   const int4* __restrict__ blk, LevelMaps m,
                                                   const int16_t* __restrict__ perm, LabFields<Real> lf,
                                                   double* __restrict__ detail, int* __restrict__ bad) {
@@ -645,76 +648,126 @@ __global__ __launch_bounds__(LAB_THREADS) void lab_kernel(int nlist, const int32
     const int4 b = blk[s];
     constexpr int lab3 = LAB * LAB * LAB;
     int my_bad = 0;
+    const int L = b.x;
+    auto node = [&](int l, int x, int y, int z) {  // what block position (l, x, y, z) is (LevelMaps)
+        if (l > m.top) return -1;
+        return l < m.nlev ? m.map[dense_level_offset(l) + x + (y << l) + (z << (2 * l))] : hashed_node(m, l, x, y, z);
+    };
+    // the leaf that holds the coincident vertex of point (x, y, z) of a
+    // subdivided node of level l; the point in the leaf's level
+    auto descend = [&](int l, int& x, int& y, int& z) {
+        int v;
+        do {
+            ++l;
+            x *= 2;
+            y *= 2;
+            z *= 2;
+            const int mk = (1 << l) - 1;
+            v = node(l, (x >> 3) & mk, (y >> 3) & mk, (z >> 3) & mk);
+        } while (v == -2);
+        return v;
+    };
+    // The 27 level-L regions around the block, looked up once: a leaf (its
+    // slot), subdivided (-2) or inside a coarser leaf (-1); and the 2^3
+    // level-(L-1) blocks that the coarse points below lie in.
+    constexpr int PC = ORDER == 4 ? 9 : 6, PL = ORDER == 4 ? 2 : 1;
+    __shared__ int32_t s_reg[27], s_creg[8];
+    // first coarse block per axis: that of point 4 * index - PL
+    const int c0[3] = {(4 * b.y - PL) >> 3, (4 * b.z - PL) >> 3, (4 * b.w - PL) >> 3};
+    bool lead = false;
+    if (threadIdx.x < 27) {
+        const int k = threadIdx.x, msk = (1 << L) - 1;
+        const int32_t v = node(L, (b.y + k % 3 - 1) & msk, (b.z + (k / 3) % 3 - 1) & msk, (b.w + k / 9 - 1) & msk);
+        s_reg[k] = v;
+        lead = v < 0;
+    } else if (threadIdx.x >= 32 && threadIdx.x < 40 && L >= 1) {
+        const int k = threadIdx.x - 32, msk = (1 << (L - 1)) - 1;
+        s_creg[k] = node(L - 1, (c0[0] + (k & 1)) & msk, (c0[1] + ((k >> 1) & 1)) & msk, (c0[2] + (k >> 2)) & msk);
+    }
+    const bool jump = __syncthreads_or(lead);
     // Coarse-point cache.  A lab ghost inside a coarser leaf is the Hs
     // synthesis of level-(L-1) points; all of them lie in the PC^3 patch of
     // coarse points from 4*idx - PL on (PC = 9, PL = 2 for order 4; 6 and 1 for
-    // order 2).  Most such points are a single leaf cell (or the coincident
-    // vertex of a finer region); their values are resolved once per lab into
-    // LDS, and a ghost's term then reads them there: the same cells, weights
-    // and order of accumulation as the recursion, which the points that need
-    // a further synthesis (flag 0) still take.
-    const int L = b.x;
-    constexpr int PC = ORDER == 4 ? 9 : 6, PL = ORDER == 4 ? 2 : 1;
-    __shared__ Real s_cv[NF][729];
-    __shared__ unsigned char s_cf[729];
-    bool jump = false;
-    for (int k = 0; k < 27; ++k) jump |= (k != 13 && nbr27[27 * s + k] < 0);
+    // order 2).  Their values are resolved once per lab into LDS: a cell of a
+    // level-(L-1) leaf, or the coincident vertex of a finer region.  On a 2:1
+    // grid every one is such a single cell (all_single), and a ghost is then the
+    // plain sum of its taps from LDS -- the recursion's cells, weights and order
+    // of accumulation; otherwise each term tests its point's flag, and points
+    // that need a further synthesis take the recursion.
+    __shared__ Real s_cv[NF][PC * PC * PC];
+    __shared__ unsigned char s_cf[PC * PC * PC];
     const bool use_cache = jump && L >= 1;  // uniform per workgroup
-    // what each of the 27 level-L regions around the block is: a leaf (its
-    // slot), subdivided (-2) or inside a coarser leaf (-1) -- looked up once
-    // here instead of for every ghost point
-    __shared__ int32_t s_reg[27];
-    if (jump && threadIdx.x < 27) {
-        const int k = threadIdx.x, msk = (1 << L) - 1;
-        const int bx = (b.y + k % 3 - 1) & msk, by = (b.z + (k / 3) % 3 - 1) & msk, bz = (b.w + k / 9 - 1) & msk;
-        const int32_t v = L < m.nlev ? m.map[dense_level_offset(L) + bx + (by << L) + (bz << (2 * L))]
-                                     : hashed_node(m, L, bx, by, bz);
-        s_reg[k] = v >= 0 ? v : (v == -2 ? -2 : -1);
-    }
-    if (jump && !use_cache) __syncthreads();
+    bool all_single = false;
     if (use_cache) {
-        const int ox = 4 * b.y - PL, oy = 4 * b.z - PL, oz = 4 * b.w - PL;
+        bool multi = false;
         for (int q = threadIdx.x; q < PC * PC * PC; q += LAB_THREADS) {
-            int Lc = L - 1, qx = ox + q % PC, qy = oy + (q / PC) % PC, qz = oz + q / (PC * PC);
-            int32_t src = -1;
-            for (;;) {  // ghost_visit's walk without synthesis
-                const int mask = (BS << Lc) - 1;
-                qx &= mask;
-                qy &= mask;
-                qz &= mask;
-                if (Lc > m.top) break;
-                const int bx = qx >> 3, by = qy >> 3, bz = qz >> 3;
-                const int32_t v = Lc < m.nlev ? m.map[dense_level_offset(Lc) + bx + (by << Lc) + (bz << (2 * Lc))]
-                                              : hashed_node(m, Lc, bx, by, bz);
-                if (v >= 0) {
-                    src = v * BCELLS + (qx & 7) + 8 * (qy & 7) + 64 * (qz & 7);
-                    break;
-                }
-                if (v != -2) break;
-                ++Lc;
-                qx *= 2;
-                qy *= 2;
-                qz *= 2;
+            const int gx = 4 * b.y - PL + q % PC, gy = 4 * b.z - PL + (q / PC) % PC, gz = 4 * b.w - PL + q / (PC * PC);
+            int32_t v = s_creg[((gx >> 3) - c0[0]) + 2 * ((gy >> 3) - c0[1]) + 4 * ((gz >> 3) - c0[2])];
+            int x = gx, y = gy, z = gz;
+            if (v == -2) {  // the coincident vertex at level L, in one of the 27 regions
+                x *= 2;
+                y *= 2;
+                z *= 2;
+                v = s_reg[((x >> 3) - b.y + 1) + 3 * ((y >> 3) - b.z + 1) + 9 * ((z >> 3) - b.w + 1)];
+                if (v == -2) v = descend(L, x, y, z);
             }
-            s_cf[q] = src >= 0 ? 1 : 0;
+            const int32_t src = v * BCELLS + (x & 7) + 8 * (y & 7) + 64 * (z & 7);
+            s_cf[q] = v >= 0 ? 1 : 0;
+            multi |= v < 0;
 #pragma unroll
-            for (int k = 0; k < NF; ++k) s_cv[k][q] = src >= 0 ? lf.f[k][src] : (Real)0;
+            for (int k = 0; k < NF; ++k) s_cv[k][q] = v >= 0 ? lf.f[k][src] : (Real)0;
         }
-        __syncthreads();
+        all_single = !__syncthreads_or(multi);
     }
     for (int i = threadIdx.x; i < lab3; i += LAB_THREADS) {
         // a lab without level jumps is copies only: cells in storage order
         // (coalesced); else in lab_order(), so that waves see uniform work
         const int p = jump ? perm[i] : i;
         const int ix = p % LAB + LS, iy = (p / LAB) % LAB + LS, iz = p / (LAB * LAB) + LS;
-        const int code = dir_code(ix, iy, iz);
-        const int src = code == 13 ? s : nbr27[27 * s + code];
+        const int32_t reg = s_reg[dir_code(ix, iy, iz)];
         Real v[NF];
-        if (src >= 0) {
+        if (reg >= 0) {
             const int cx = (ix + 8) & 7, cy = (iy + 8) & 7, cz = (iz + 8) & 7;
-            const size_t c = (size_t)src * BCELLS + cx + 8 * cy + 64 * cz;
+            const size_t c = (size_t)reg * BCELLS + cx + 8 * cy + 64 * cz;
 #pragma unroll
             for (int k = 0; k < NF; ++k) v[k] = lf.f[k][c];
+        } else if (reg == -2) {  // subdivided: the coincident fine vertex, one term of weight 1
+            int x = 8 * b.y + ix, y = 8 * b.z + iy, z = 8 * b.w + iz;
+            const int32_t d = descend(L, x, y, z);
+            if (d < 0) my_bad = 1;  // (no such node in a tree)
+            const int32_t src = d < 0 ? 0 : d * BCELLS + (x & 7) + 8 * (y & 7) + 64 * (z & 7);
+#pragma unroll
+            for (int k = 0; k < NF; ++k) v[k] = (Real)0 + lf.f[k][src];
+        } else if (all_single) {
+            constexpr int NT = ORDER == 4 ? 4 : 2;  // taps of an odd coordinate
+            // first tap: (i - 3) / 2 (order 4) or (i - 1) / 2 of an odd coordinate, i / 2 of an even one
+            const int ox = (ix & 1) ? 1 : 0, oy = (iy & 1) ? 1 : 0, oz = (iz & 1) ? 1 : 0;
+            constexpr int back = ORDER == 4 ? 3 : 1;
+            const int tx = (ix - back * ox) / 2 + PL, ty = (iy - back * oy) / 2 + PL, tz = (iz - back * oz) / 2 + PL;
+            const int nx = ox ? NT : 1, ny = oy ? NT : 1, nz = oz ? NT : 1;
+            auto w1 = [](int n, int k) {  // Hs weights: dyadic, and so are their products
+                return n == 1 ? (Real)1 : ORDER == 2 ? (Real)0.5
+                                        : (k == 0 || k == 3) ? (Real)(-1.0 / 16) : (Real)(9.0 / 16);
+            };
+#pragma unroll
+            for (int k = 0; k < NF; ++k) v[k] = (Real)0;
+            for (int kz = 0; kz < nz; ++kz) {
+                const Real wz = w1(nz, kz);
+                for (int ky = 0; ky < ny; ++ky) {
+                    const Real wzy = wz * w1(ny, ky);
+                    const int row = tx + PC * (ty + ky + PC * (tz + kz));
+#pragma unroll
+                    for (int kx = 0; kx < NT; ++kx) {
+                        if (kx >= nx) break;
+                        const Real w = wzy * w1(nx, kx);
+#pragma unroll
+                        for (int k = 0; k < NF; ++k) {
+                            const Real prod = s_cv[k][row + kx] * w;
+                            v[k] = v[k] + prod;
+                        }
+                    }
+                }
+            }
         } else {
 #pragma unroll
             for (int k = 0; k < NF; ++k) v[k] = (Real)0;
@@ -726,27 +779,13 @@ __global__ __launch_bounds__(LAB_THREADS) void lab_kernel(int nlist, const int32
                     v[k] = v[k] + prod;
                 }
             };
-            // the level-L region of this point: inside a coarser leaf?
             const int mask = (BS << L) - 1;
             const int qx = (8 * b.y + ix) & mask, qy = (8 * b.z + iy) & mask, qz = (8 * b.w + iz) & mask;
-            const int32_t reg = s_reg[code];  // src < 0: the block has a level jump
-            if (reg == -2) {  // subdivided: ghost_visit<2>'s first step, the coincident fine vertex
-                ghost_visit<2>(m, order, L + 1, 2 * qx, 2 * qy, 2 * qz, 1.0, visit, my_bad);
-            } else if (!(use_cache && reg == -1)) {
+            if (!use_cache) {
                 ghost_visit<2>(m, order, L, qx, qy, qz, 1.0, visit, my_bad);
             } else {  // ghost_visit<2>'s synthesis step, coarse points from the cache
                 const int nc = BS << (L - 1);  // coarse lattice size (a power of two: & wraps)
-                constexpr int NT = ORDER == 4 ? 4 : 2;  // taps of an odd coordinate
                 const int nz = synth_n(order, qz), ny = synth_n(order, qy), nx = synth_n(order, qx);
-                // the x taps once per ghost (entries k >= nx unused)
-                int sxk[NT], pxk[NT];
-                double wxk[NT];
-#pragma unroll
-                for (int k = 0; k < NT; ++k) {
-                    sxk[k] = synth_src(order, qx, k);
-                    pxk[k] = (sxk[k] - (4 * b.y - PL)) & (nc - 1);
-                    wxk[k] = synth_w(order, qx, k);
-                }
 #pragma unroll 1
                 for (int kz = 0; kz < nz; ++kz) {
                     const int sz = synth_src(order, qz, kz);
@@ -757,14 +796,13 @@ __global__ __launch_bounds__(LAB_THREADS) void lab_kernel(int nlist, const int32
                         const int sy = synth_src(order, qy, ky);
                         const int py = (sy - (4 * b.z - PL)) & (nc - 1);
                         const double wzy = wz * synth_w(order, qy, ky);
-                        const bool row_in = py < PC && pz < PC;
-                        const int row = PC * (py + PC * pz);
-#pragma unroll
-                        for (int kx = 0; kx < NT; ++kx) {
-                            if (kx >= nx) break;
-                            const double w = 1.0 * (wzy * wxk[kx]);
-                            const int pq = pxk[kx] + row;
-                            if (row_in && pxk[kx] < PC && s_cf[pq]) {
+#pragma unroll 1
+                        for (int kx = 0; kx < nx; ++kx) {
+                            const int sx = synth_src(order, qx, kx);
+                            const int px = (sx - (4 * b.y - PL)) & (nc - 1);
+                            const double w = 1.0 * (wzy * synth_w(order, qx, kx));
+                            const int pq = px + PC * (py + PC * pz);
+                            if (px < PC && py < PC && pz < PC && s_cf[pq]) {
                                 const Real wr = (Real)w;
 #pragma unroll
                                 for (int k = 0; k < NF; ++k) {
@@ -772,7 +810,7 @@ __global__ __launch_bounds__(LAB_THREADS) void lab_kernel(int nlist, const int32
                                     v[k] = v[k] + prod;
                                 }
                             } else {
-                                ghost_visit<1>(m, order, L - 1, sxk[kx], sy, sz, w, visit, my_bad);
+                                ghost_visit<1>(m, order, L - 1, sx, sy, sz, w, visit, my_bad);
                             }
                         }
                     }
@@ -1869,7 +1907,7 @@ void launch_labs(Ctx& c, int order, int nlist, const int32_t* dslots, const Leve
     const bool few = nlist <= kLabThreadsFewMax;
     auto go = [&](auto kern, int threads) {
         hipLaunchKernelGGL(kern, dim3((unsigned)nlist), dim3(threads), 0, c.stream, nlist, dslots,
-                           c.dNbr27.as<int32_t>(), c.dBlk.as<int4>(), m, c.labPerm.as<int16_t>(), lf, detail,
+                           c.dBlk.as<int4>(), m, c.labPerm.as<int16_t>(), lf, detail,
                            c.dBad.as<int>());
     };
     if (order == 4) {

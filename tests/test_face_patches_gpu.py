@@ -50,3 +50,20 @@ def test_gpu_face_ghosts_match_oracle(oracle, real, order, grid):
                               t(rho), dt, k)
     assert bits_equal(out, ref), "max |diff| %g" % np.abs(out.astype(float) - ref).max()
     assert counts["faces_device"] >= 1 and counts["faces_host"] == 0, counts
+
+
+@pytest.mark.parametrize("real", ["f32", "f64"])
+@pytest.mark.parametrize("order", [4, 2])
+@pytest.mark.parametrize("grid", ["jump-526", "balanced-small"])
+def test_gpu_lab_details_match_oracle(oracle, real, order, grid):
+    """Details whose labs hold coarse points that need a further synthesis
+    (two-level jump) and labs of single cells only: equal to the oracle's."""
+    rows = GRIDS[grid]()
+    fields = random_fields(rows, np.float32 if real == "f32" else np.float64, 13)
+    ctx = make_ctx(real, rows, order, fields, max_level=6)
+    det = ctx.fwt_details()
+    counts = ctx.adapt_counters()
+    ctx.close()
+    ref = oracle.amr_details(rows, order, fields[FIELD_PHI], list(range(len(rows))))
+    assert np.array_equal(det, ref), "max |diff| %g" % np.abs(det - ref).max()
+    assert counts["labs_device"] >= 1 and counts["labs_host"] == 0, counts
