@@ -989,7 +989,7 @@ __global__ __launch_bounds__(512) void remap_kernel(int nnew, const Remap* __res
     for (int f = 0; f < 4; ++f) rf.out[f][(size_t)ns * BCELLS + cell] = v[f];
 }
 
-// per-cell constants on a multi-level grid: as rd_statics_kernel, with the
+// per-cell constants on a multi-level grid: as constants_kernel, with the
 // face towards an interpolated ghost taken from the ghost's p_w, p_g; also the
 // ghosts' tau and the harmonic diffusivity of the minus faces towards ghosts
 template <typename Real>

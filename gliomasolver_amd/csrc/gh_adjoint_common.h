@@ -111,7 +111,7 @@ struct UniformAdjParams {
 
 // Domain test and outside flag of a cell with state u and record r.  Generic
 // records (CLAMPED false) carry tau, with the domain threshold in sig.  Clamped
-// records (stat_fast_kernel: every threshold <= 0, state u >= +0, i.e. any step
+// records (constants_kernel: every threshold <= 0, state u >= +0, i.e. any step
 // k >= 1) carry +-max(tau, 0) with the sign set where the threshold is < 0:
 // then u > sig holds there, and elsewhere it is u > 0; u < tau is
 // u < max(tau, 0).
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void adj_mask_kernel(size_t n, double* __restr
 // partial[ADJ_PART s + 2 w + q] accumulates wave w's sums A (q = 0) and B
 // (q = 1) of block s, step after step.  CLAMPED: st holds the clamped-state records and
 // sig is not read (steps k >= 1 when every threshold is <= 0).
-// Blocks without diffusion (zero_flux_kernel; wk's groups): every face
+// Blocks without diffusion (constants_kernel; wk's groups): every face
 // coefficient their cells use is +0, so each of adj_cell's face terms is a
 // signed zero whatever the neighbour's state, flag or weight (finite values),
 // the sums come out +0, and the cell's update is adj_cell with zero neighbour

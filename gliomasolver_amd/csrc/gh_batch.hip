@@ -154,41 +154,25 @@ struct BatchStepParams {
     }
 };
 
-// Statics of every slot (rd_statics_kernel per sample): anatomy cell =
-// (slot - slot0) * 512 + lane, Dw, Dg of the sample.
+// constants_kernel's source: the anatomy, Dw and Dg of the slot's sample
 template <typename Real>
-__global__ __launch_bounds__(256) void batch_statics_kernel(size_t nslots, const int32_t* __restrict__ nbr,
-                                                            const int32_t* __restrict__ slot_pos,
-                                                            const SlotRange<Real>* __restrict__ range,
-                                                            const Real* const* __restrict__ apw,
-                                                            const Real* const* __restrict__ apg,
-                                                            Stat4<Real>* __restrict__ st, Real* __restrict__ sig,
-                                                            unsigned int* __restrict__ flags) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= nslots * BCELLS) return;
-    const size_t s = gid / BCELLS;
-    const int l = (int)(gid % BCELLS);
-    const int x = l & 7, y = (l >> 3) & 7, z = l >> 6;
-    const int pos = slot_pos[s];
-    const SlotRange<Real>& q = range[pos];
-    const Real* pw = apw[pos];
-    const Real* pg = apg[pos];
-    const size_t base = q.slot0 * BCELLS;
-    const size_t a = gid - base;
-    const Real pwc = pw[a], pgc = pg[a];
-    const Real dc = diffusivity(pwc, pgc, q.Dw, q.Dg);
-    const size_t nx = (x < 7) ? a + 1 : (size_t)nbr[6 * s + FXP] * BCELLS + (l - 7) - base;
-    const size_t ny = (y < 7) ? a + 8 : (size_t)nbr[6 * s + FYP] * BCELLS + (l - 56) - base;
-    const size_t nz = (z < 7) ? a + 64 : (size_t)nbr[6 * s + FZP] * BCELLS + (l - 448) - base;
-    Stat4<Real> r;
-    r.dx = harmonic(diffusivity(pw[nx], pg[nx], q.Dw, q.Dg), dc);
-    r.dy = harmonic(diffusivity(pw[ny], pg[ny], q.Dw, q.Dg), dc);
-    r.dz = harmonic(diffusivity(pw[nz], pg[nz], q.Dw, q.Dg), dc);
-    r.tau = chf_threshold(pwc, pgc);
-    st[gid] = r;
-    sig[gid] = domain_threshold(pwc, pgc);
-    if (cancels(pwc, pgc)) atomicOr(flags + 1, 1u);
-}
+struct BatchAnatomySrc {
+    const int32_t* __restrict__ slot_pos;
+    const SlotRange<Real>* __restrict__ range;
+    const Real* const* __restrict__ apw;
+    const Real* const* __restrict__ apg;
+    __device__ inline void anatomy(int s, const Real*& w, const Real*& g, Real& dw, Real& dg) const {
+        const int p = slot_pos[s];
+        w = apw[p];
+        g = apg[p];
+        dw = range[p].Dw;
+        dg = range[p].Dg;
+    }
+    __device__ inline BlockPos pos(int s) const {
+        const SlotRange<Real>& q = range[slot_pos[s]];
+        return block_pos(s, (int)q.slot0, q.bpd, q.magic);
+    }
+};
 
 template <typename Real>
 __global__ __launch_bounds__(256) void scatter_kernel(size_t n, const uint64_t* __restrict__ idx,
@@ -225,27 +209,6 @@ __global__ __launch_bounds__(256) void batch_lik_final_kernel(const double* __re
     lik_final_body(LIK_GRID, partials + (size_t)blockIdx.x * 4 * LIK_GRID, out + 4 * (size_t)blockIdx.x);
 }
 
-// uniform periodic neighbours of block (bx,by,bz) of a bpd^3 grid, slot order
-// bx + bpd*(by + bpd*bz), faces -x,+x,-y,+y,-z,+z
-void periodic_neighbours(int bpd, size_t slot0, std::vector<int32_t>& nbr) {
-    for (int bz = 0; bz < bpd; ++bz)
-        for (int by = 0; by < bpd; ++by)
-            for (int bx = 0; bx < bpd; ++bx) {
-                auto id = [&](int x, int y, int z) {
-                    x = (x + bpd) % bpd;
-                    y = (y + bpd) % bpd;
-                    z = (z + bpd) % bpd;
-                    return (int32_t)(slot0 + (size_t)x + (size_t)bpd * ((size_t)y + (size_t)bpd * z));
-                };
-                nbr.push_back(id(bx - 1, by, bz));
-                nbr.push_back(id(bx + 1, by, bz));
-                nbr.push_back(id(bx, by - 1, bz));
-                nbr.push_back(id(bx, by + 1, bz));
-                nbr.push_back(id(bx, by, bz - 1));
-                nbr.push_back(id(bx, by, bz + 1));
-            }
-}
-
 // dense (x fastest, n = 8*bpd) -> block-major index of a uniform grid
 inline size_t block_index(int bpd, size_t c) {
     const size_t n = (size_t)BS * bpd;
@@ -266,10 +229,10 @@ struct Batch {
     std::vector<int> order;         // position -> sample index
     std::vector<int> pos_of;        // sample index -> position
     std::vector<size_t> slot0;      // per position, plus the total
-    DevBuf phi[2], statD, statSig, nbr, slotPos, range, apw, apg, likPart, likOut, likJobs;
+    DevBuf phi[2], statD, statSig, slotPos, range, apw, apg, likPart, likOut, likJobs;
     DevBuf statF, flag;  // rd_step2f_kernel records (valid iff fast_ok), count scratch
     bool fast_ok = false, plain_dom = false;
-    DevBuf zeroFlux;                 // per slot: != 0 a block without diffusion (zero_flux_kernel)
+    DevBuf zeroFlux;                 // per slot: != 0 a block without diffusion (constants_kernel)
     // StepWork lists of all slots and their lengths per count of positions (index p: positions 0..p)
     DevBuf fullList, grpList, stillGrp;
     std::vector<int> nFull, nGrp;
@@ -338,18 +301,17 @@ int build_layout_t(Batch& b) {
     int rc;
     if ((rc = b.phi[0].ensure(nc * sizeof(Real))) || (rc = b.phi[1].ensure(nc * sizeof(Real))) ||
         (rc = b.statD.ensure(nc * sizeof(Stat4<Real>))) || (rc = b.statSig.ensure(nc * sizeof(Real))) ||
-        (rc = b.nbr.ensure(6 * nsl * sizeof(int32_t))) || (rc = b.slotPos.ensure(nsl * sizeof(int32_t))) ||
+        (rc = b.statF.ensure_grow(std::max<size_t>(1, nc) * sizeof(Stat4<Real>))) ||
+        (rc = b.zeroFlux.ensure_grow(std::max<size_t>(1, nsl))) || (rc = b.slotPos.ensure(nsl * sizeof(int32_t))) ||
         (rc = b.range.ensure(ns * sizeof(SlotRange<Real>))) || (rc = b.apw.ensure(ns * sizeof(void*))) ||
         (rc = b.apg.ensure(ns * sizeof(void*))))
         return rc;
-    std::vector<int32_t> nbr, spos(nsl);
-    nbr.reserve(6 * nsl);
+    std::vector<int32_t> spos(nsl);
     std::vector<SlotRange<Real>> rng(ns);
     std::vector<const void*> apw(ns), apg(ns);
     for (int p = 0; p < ns; ++p) {
         const BatchSample& q = b.smp[b.order[p]];
         const BatchAnatomy& a = *b.anat[q.anat];
-        periodic_neighbours(a.bpd, b.slot0[p], nbr);
         for (size_t s = b.slot0[p]; s < b.slot0[p + 1]; ++s) spos[s] = p;
         const Real hr = (Real)(1.0 / (double)(BS * a.bpd));  // info.h[0] of a uniform grid
         rng[p].slot0 = b.slot0[p];
@@ -367,35 +329,33 @@ int build_layout_t(Batch& b) {
         apw[p] = a.pw.p;
         apg[p] = a.pg.p;
     }
-    GH_HIP_CHECK(hipMemcpyAsync(b.nbr.p, nbr.data(), nbr.size() * sizeof(int32_t), hipMemcpyHostToDevice, b.stream));
     GH_HIP_CHECK(hipMemcpyAsync(b.slotPos.p, spos.data(), spos.size() * sizeof(int32_t), hipMemcpyHostToDevice,
                                 b.stream));
     GH_HIP_CHECK(hipMemcpyAsync(b.range.p, rng.data(), rng.size() * sizeof(SlotRange<Real>), hipMemcpyHostToDevice,
                                 b.stream));
     GH_HIP_CHECK(hipMemcpyAsync(b.apw.p, apw.data(), ns * sizeof(void*), hipMemcpyHostToDevice, b.stream));
     GH_HIP_CHECK(hipMemcpyAsync(b.apg.p, apg.data(), ns * sizeof(void*), hipMemcpyHostToDevice, b.stream));
-    const unsigned g = (unsigned)((nc + 255) / 256);
     if ((rc = clear_stat_flags(b.stream, b.flag))) return rc;
-    hipLaunchKernelGGL(batch_statics_kernel<Real>, dim3(g), dim3(256), 0, b.stream, nsl, b.nbr.as<int32_t>(),
-                       b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>(), b.apw.as<const Real* const>(),
-                       b.apg.as<const Real* const>(), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
-                       b.flag.as<unsigned int>());
-    GH_HIP_CHECK(hipGetLastError());
-    if ((rc = build_stat_fast(b.stream, sizeof(Real) == 4 ? GH_REAL_F32 : GH_REAL_F64, nc, b.statD.p, b.statSig.p,
-                              b.statF, b.flag, &b.fast_ok, &b.plain_dom)))
-        return rc;
     b.nFull.clear();
     b.nGrp.clear();
     b.skip_still = false;
-    if (b.fast_ok && nsl > 0) {  // blocks without diffusion
-        if ((rc = b.zeroFlux.ensure_grow(nsl))) return rc;
-        const BatchStepParams<Real> prm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
-        hipLaunchKernelGGL((zero_flux_kernel<Real, BatchStepParams<Real>>), dim3((unsigned)nsl), dim3(256), 0,
-                           b.stream, (int)nsl, b.statF.as<Stat4<Real>>(), prm, b.zeroFlux.as<unsigned char>());
+    std::vector<unsigned char> z(nsl);
+    if (nsl > 0) {
+        const BatchAnatomySrc<Real> src{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>(),
+                                        b.apw.as<const Real* const>(), b.apg.as<const Real* const>()};
+        hipLaunchKernelGGL((constants_kernel<Real, BatchAnatomySrc<Real>>), dim3((unsigned)nsl), dim3(512), 0,
+                           b.stream, src, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(), b.statF.as<Stat4<Real>>(),
+                           b.zeroFlux.as<unsigned char>(), b.flag.as<unsigned int>());
         GH_HIP_CHECK(hipGetLastError());
-        std::vector<unsigned char> z(nsl);
         GH_HIP_CHECK(hipMemcpyAsync(z.data(), b.zeroFlux.p, nsl, hipMemcpyDeviceToHost, b.stream));
-        GH_HIP_CHECK(hipStreamSynchronize(b.stream));
+    }
+    unsigned int flags[2] = {1, 1};
+    GH_HIP_CHECK(hipMemcpyAsync(flags, b.flag.p, sizeof(flags), hipMemcpyDeviceToHost, b.stream));
+    GH_HIP_CHECK(hipMemsetAsync(b.phi[0].p, 0, nc * sizeof(Real), b.stream));
+    GH_HIP_CHECK(hipStreamSynchronize(b.stream));  // (also: the host tables above are read by their copies)
+    b.fast_ok = flags[0] == 0;
+    b.plain_dom = flags[1] == 0;
+    if (b.fast_ok && nsl > 0) {  // the work list
         std::vector<int32_t> full;
         std::vector<int2> grp;
         const std::vector<size_t> cut(b.slot0.begin() + 1, b.slot0.end());
@@ -412,8 +372,6 @@ int build_layout_t(Batch& b) {
             GH_HIP_CHECK(hipStreamSynchronize(b.stream));  // the lists are read by the copies
         }
     }
-    GH_HIP_CHECK(hipMemsetAsync(b.phi[0].p, 0, nc * sizeof(Real), b.stream));
-    GH_HIP_CHECK(hipStreamSynchronize(b.stream));
     return GH_OK;
 }
 
@@ -866,7 +824,7 @@ int gh_batch_destroy(gh_batch* bh) {
         a->pet.release();
         a->roi.release();
     }
-    DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->nbr,    &b->slotPos, &b->range,
+    DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->slotPos, &b->range,
                       &b->apw,    &b->apg,    &b->likPart, &b->likOut, &b->likJobs, &b->ck,     &b->tape,
                       &b->lam[0], &b->lam[1], &b->apart,   &b->icpart, &b->adjJobs, &b->statF,  &b->flag,
                       &b->zeroFlux, &b->fullList, &b->grpList, &b->stillGrp};

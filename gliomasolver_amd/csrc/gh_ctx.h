@@ -146,7 +146,7 @@ struct Ctx {
     DevBuf flag;        // small scratch word for device-side counts
     bool fast_ok = false;  // every cell has p_w + p_g >= 0: clamped states may take rd_step2f_kernel
     bool plain_dom = false;  // no cell has p_w = -p_g != 0: rd_step2f_kernel needs no domain test
-    DevBuf zeroFlux;       // per slot: != 0 a block without diffusion (zero_flux_kernel), uniform grids
+    DevBuf zeroFlux;       // per slot: != 0 a block without diffusion (constants_kernel), uniform grids
     int nZeroFlux = 0;     // blocks without diffusion
     // work list of the two-step and reverse-step kernels (StepWork, plan_step2f):
     // slots of the blocks with diffusion, groups of blocks without (nGrp = 0:
@@ -211,12 +211,7 @@ int rd_zero_still(Ctx& c, void* states, int n);
 struct StepWork;
 StepWork rd_step_work(const Ctx& c, bool skip_still);
 double block_h_of(const Ctx& c);
-// the rd_step2f_kernel records of n cells from {D+, tau} and sigma into out;
-// *ok = every cell has sigma <= 0 (p_w + p_g >= 0); *plain = flag's second word
-// is 0 (no cell cancels).  Synchronizes the stream.
-int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st, const void* sig, DevBuf& out,
-                    DevBuf& flag, bool* ok, bool* plain);
-// zeroes flag's two words, before the kernel that fills st and sig
+// zeroes the two words of constants_kernel's flags
 int clear_stat_flags(hipStream_t stream, DevBuf& flag);
 int rd_autotune(Ctx& c, double dt, int trial_steps, int* best);
 

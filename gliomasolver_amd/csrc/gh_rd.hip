@@ -10,7 +10,7 @@
 // for the harmonic mean.
 //
 // Split of the work:
-//   rd_statics_kernel  once per solve (Dw, Dg, anatomy fixed): the harmonic
+//   constants_kernel   once per solve (Dw, Dg, anatomy fixed): the harmonic
 //                      face diffusivity of each cell's +x,+y,+z face (the
 //                      harmonic mean is symmetric, so each face is computed
 //                      once), the threshold tau with "chf = phi+p_w+p_g < 0.1
@@ -35,33 +35,6 @@ namespace gh {
 namespace {
 
 template <typename Real>
-__global__ __launch_bounds__(256) void rd_statics_kernel(int nslots, const int32_t* __restrict__ nbr,
-                                                         const Real* __restrict__ pw, const Real* __restrict__ pg,
-                                                         Real Dw, Real Dg, Stat4<Real>* __restrict__ st,
-                                                         Real* __restrict__ sig, unsigned int* __restrict__ flags) {
-    const size_t nc = (size_t)nslots * BCELLS;
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= nc) return;
-    const int s = (int)(gid / BCELLS);
-    const int l = (int)(gid % BCELLS);
-    const int x = l & 7, y = (l >> 3) & 7, z = l >> 6;
-    const Real pwc = pw[gid], pgc = pg[gid];
-    const Real dc = diffusivity(pwc, pgc, Dw, Dg);
-    // +x, +y, +z neighbour cells (same slot or the same-level neighbour slot)
-    const size_t nx = (x < 7) ? gid + 1 : (size_t)nbr[6 * s + FXP] * BCELLS + (l - 7);
-    const size_t ny = (y < 7) ? gid + 8 : (size_t)nbr[6 * s + FYP] * BCELLS + (l - 56);
-    const size_t nz = (z < 7) ? gid + 64 : (size_t)nbr[6 * s + FZP] * BCELLS + (l - 448);
-    Stat4<Real> r;
-    r.dx = harmonic(diffusivity(pw[nx], pg[nx], Dw, Dg), dc);
-    r.dy = harmonic(diffusivity(pw[ny], pg[ny], Dw, Dg), dc);
-    r.dz = harmonic(diffusivity(pw[nz], pg[nz], Dw, Dg), dc);
-    r.tau = chf_threshold(pwc, pgc);
-    st[gid] = r;
-    sig[gid] = domain_threshold(pwc, pgc);
-    if (cancels(pwc, pgc)) atomicOr(flags + 1, 1u);
-}
-
-template <typename Real>
 __global__ __launch_bounds__(256) void rd_update_kernel(size_t nc, Real* __restrict__ phi,
                                                         const Real* __restrict__ dphidt, double dt) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -76,39 +49,54 @@ inline double block_h(const Ctx& c) {
     return std::ldexp(1.0, -c.topo.blocks[0].level) / BS;
 }
 
-// The work list of the two-step and reverse-step kernels on a uniform grid
-// (StepWork): zero_flux_kernel's flags decide.
+// The per-solve constants (constants_kernel) and, from its flags, the work list
+// of the two-step and reverse-step kernels (StepWork).
 template <typename Real>
-int plan_step2f(Ctx& c) {
+int prepare_t(Ctx& c, double Dw, double Dg, double rho) {
     const int ns = c.topo.nblocks();
+    const size_t nc = c.ncells();
+    int rc;
+    if ((rc = c.statF.ensure_grow(std::max<size_t>(1, nc) * sizeof(Stat4<Real>))) ||
+        (rc = c.zeroFlux.ensure_grow(std::max(1, ns))) || (rc = clear_stat_flags(c.stream, c.flag)))
+        return rc;
+    const int bpd = c.topo.uniform_bpd;
+    const UniformAnatomy<Real> src{c.pw.as<Real>(), c.pg.as<Real>(), (Real)Dw, (Real)Dg, bpd, bpd_magic(bpd)};
+    hipLaunchKernelGGL((constants_kernel<Real, UniformAnatomy<Real>>), dim3(ns), dim3(512), 0, c.stream, src,
+                       c.statD.as<Stat4<Real>>(), c.statSig.as<Real>(), c.statF.as<Stat4<Real>>(),
+                       c.zeroFlux.as<unsigned char>(), c.flag.as<unsigned int>());
+    GH_HIP_CHECK(hipGetLastError());
+    std::vector<unsigned char> z(ns);
+    unsigned int flags[2] = {1, 1};
+    GH_HIP_CHECK(hipMemcpyAsync(flags, c.flag.p, sizeof(flags), hipMemcpyDeviceToHost, c.stream));
+    GH_HIP_CHECK(hipMemcpyAsync(z.data(), c.zeroFlux.p, ns, hipMemcpyDeviceToHost, c.stream));
+    GH_HIP_CHECK(hipStreamSynchronize(c.stream));
+    c.fast_ok = flags[0] == 0;
+    c.plain_dom = flags[1] == 0;
     c.nZeroFlux = 0;
     c.nFull = ns;
     c.nGrp = 0;
-    if (!c.fast_ok || c.topo.uniform_bpd <= 0 || ns == 0) return GH_OK;
-    int rc;
-    if ((rc = c.zeroFlux.ensure_grow(ns))) return rc;
-    const UniformStepParams<Real> prm{(Real)c.rho, 0., 0., c.topo.uniform_bpd, bpd_magic(c.topo.uniform_bpd)};
-    hipLaunchKernelGGL((zero_flux_kernel<Real, UniformStepParams<Real>>), dim3(ns), dim3(256), 0, c.stream, ns,
-                       c.statF.as<Stat4<Real>>(), prm, c.zeroFlux.as<unsigned char>());
-    GH_HIP_CHECK(hipGetLastError());
-    std::vector<unsigned char> z(ns);
-    GH_HIP_CHECK(hipMemcpyAsync(z.data(), c.zeroFlux.p, ns, hipMemcpyDeviceToHost, c.stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c.stream));
     std::vector<int32_t> full;
     std::vector<int2> grp;
-    build_step_work(z.data(), {(size_t)ns}, full, grp, nullptr, nullptr);
+    if (c.fast_ok) build_step_work(z.data(), {(size_t)ns}, full, grp, nullptr, nullptr);
     for (const int2& g : grp) c.nZeroFlux += g.y;
-    if (grp.empty()) return GH_OK;  // item i is slot i
-    if ((rc = c.fullList.ensure_grow(std::max<size_t>(1, full.size()) * sizeof(int32_t))) ||
-        (rc = c.grpList.ensure_grow(grp.size() * sizeof(int2))) || (rc = c.stillGrp.ensure_grow(grp.size())))
-        return rc;
-    if (!full.empty())
-        GH_HIP_CHECK(hipMemcpyAsync(c.fullList.p, full.data(), full.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+    if (!grp.empty()) {  // (without: item i is slot i)
+        if ((rc = c.fullList.ensure_grow(std::max<size_t>(1, full.size()) * sizeof(int32_t))) ||
+            (rc = c.grpList.ensure_grow(grp.size() * sizeof(int2))) || (rc = c.stillGrp.ensure_grow(grp.size())))
+            return rc;
+        if (!full.empty())
+            GH_HIP_CHECK(hipMemcpyAsync(c.fullList.p, full.data(), full.size() * sizeof(int32_t),
+                                        hipMemcpyHostToDevice, c.stream));
+        GH_HIP_CHECK(hipMemcpyAsync(c.grpList.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice,
                                     c.stream));
-    GH_HIP_CHECK(hipMemcpyAsync(c.grpList.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice, c.stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    c.nFull = (int)full.size();
-    c.nGrp = (int)grp.size();
+        GH_HIP_CHECK(hipStreamSynchronize(c.stream));
+        c.nFull = (int)full.size();
+        c.nGrp = (int)grp.size();
+    }
+    c.Dw = Dw;
+    c.Dg = Dg;
+    c.rho = rho;
+    c.prepared = true;
+    c.constants_stale = false;
     return GH_OK;
 }
 
@@ -120,29 +108,6 @@ int mark_still(Ctx& c, const Real* in, Real* out) {
     hipLaunchKernelGGL(still_kernel<Real>, dim3(c.nGrp), dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
                        c.zeroFlux.as<unsigned char>(), in, out, c.stillGrp.as<unsigned char>());
     GH_HIP_CHECK(hipGetLastError());
-    return GH_OK;
-}
-
-template <typename Real>
-int prepare_t(Ctx& c, double Dw, double Dg, double rho) {
-    const int ns = c.topo.nblocks();
-    const size_t nc = c.ncells();
-    const unsigned grid = (unsigned)((nc + 255) / 256);
-    int rc;
-    if ((rc = clear_stat_flags(c.stream, c.flag))) return rc;
-    hipLaunchKernelGGL(rd_statics_kernel<Real>, dim3(grid), dim3(256), 0, c.stream, ns, c.nbr.as<int32_t>(),
-                       c.pw.as<Real>(), c.pg.as<Real>(), (Real)Dw, (Real)Dg, c.statD.as<Stat4<Real>>(),
-                       c.statSig.as<Real>(), c.flag.as<unsigned int>());
-    GH_HIP_CHECK(hipGetLastError());
-    if ((rc = build_stat_fast(c.stream, c.real_kind, nc, c.statD.p, c.statSig.p, c.statF, c.flag, &c.fast_ok,
-                              &c.plain_dom)))
-        return rc;
-    if ((rc = plan_step2f<Real>(c))) return rc;
-    c.Dw = Dw;
-    c.Dg = Dg;
-    c.rho = rho;
-    c.prepared = true;
-    c.constants_stale = false;
     return GH_OK;
 }
 
@@ -287,29 +252,6 @@ StepWork rd_step_work(const Ctx& c, bool skip_still) {
 int clear_stat_flags(hipStream_t stream, DevBuf& flag) {
     if (int rc = flag.ensure(2 * sizeof(unsigned int))) return rc;
     GH_HIP_CHECK(hipMemsetAsync(flag.p, 0, 2 * sizeof(unsigned int), stream));
-    return GH_OK;
-}
-
-int build_stat_fast(hipStream_t stream, int real_kind, size_t n, const void* st, const void* sig, DevBuf& out,
-                    DevBuf& flag, bool* ok, bool* plain) {
-    const size_t rs = real_kind == GH_REAL_F32 ? 4 : 8;
-    int rc;
-    if ((rc = out.ensure_grow(std::max<size_t>(1, n) * 4 * rs))) return rc;
-    const unsigned grid = (unsigned)((n + 255) / 256);
-    if (n > 0) {
-        if (real_kind == GH_REAL_F32)
-            hipLaunchKernelGGL(stat_fast_kernel<float>, dim3(grid), dim3(256), 0, stream, n, (const Stat4<float>*)st,
-                               (const float*)sig, out.as<Stat4<float>>(), flag.as<unsigned int>());
-        else
-            hipLaunchKernelGGL(stat_fast_kernel<double>, dim3(grid), dim3(256), 0, stream, n, (const Stat4<double>*)st,
-                               (const double*)sig, out.as<Stat4<double>>(), flag.as<unsigned int>());
-        GH_HIP_CHECK(hipGetLastError());
-    }
-    unsigned int bad[2] = {1, 1};
-    GH_HIP_CHECK(hipMemcpyAsync(bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost, stream));
-    GH_HIP_CHECK(hipStreamSynchronize(stream));
-    *ok = bad[0] == 0;
-    *plain = bad[1] == 0;
     return GH_OK;
 }
 
