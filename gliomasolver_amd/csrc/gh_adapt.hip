@@ -2781,8 +2781,7 @@ int gh_set_field_blocks(gh_ctx* ctx, int field, const void* values) {
               : field == GH_FIELD_DPHIDT ? &c->dphidt : nullptr;
     if (!b) return set_error(GH_EINVAL, "gh_set_field_blocks: bad field");
     GH_HIP_CHECK(hipSetDevice(c->device));
-    GH_HIP_CHECK(hipMemcpyAsync(b->p, values, c->ncells() * c->real_size, hipMemcpyHostToDevice, c->stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (int rc = stage_send(c->device, c->stream, b->p, c->ncells(), 0, c->real_size, values)) return rc;
     if (field == GH_FIELD_PW || field == GH_FIELD_PG) c->prepared = false;
     return GH_OK;
 }
@@ -2797,9 +2796,7 @@ int gh_get_field_blocks(gh_ctx* ctx, int field, void* values) {
               : field == GH_FIELD_DPHIDT ? &c->dphidt : nullptr;
     if (!b) return set_error(GH_EINVAL, "gh_get_field_blocks: bad field");
     GH_HIP_CHECK(hipSetDevice(c->device));
-    GH_HIP_CHECK(hipMemcpyAsync(values, b->p, c->ncells() * c->real_size, hipMemcpyDeviceToHost, c->stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    return GH_OK;
+    return stage_fetch(c->device, c->stream, b->p, c->ncells(), 0, c->real_size, values);
 }
 
 int gh_uq_resample(gh_ctx* ctx, int gpd, double* out) {

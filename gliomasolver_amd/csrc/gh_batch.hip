@@ -807,6 +807,7 @@ int gh_batch_create(int device, int real_kind, gh_batch** out) {
     GH_HIP_CHECK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
     GH_HIP_CHECK(hipEventCreate(&b->ev0));
     GH_HIP_CHECK(hipEventCreate(&b->ev1));
+    stage_retain();
     *out = reinterpret_cast<gh_batch*>(b.release());
     return GH_OK;
 }
@@ -833,6 +834,7 @@ int gh_batch_destroy(gh_batch* bh) {
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
+    stage_release();
     return GH_OK;
 }
 
@@ -993,16 +995,9 @@ int gh_batch_get_phi(gh_batch* bh, int sample, void* dense) {
     GH_HIP_CHECK(hipSetDevice(b->device));
     const int p = b->pos_of[sample];
     const BatchAnatomy& a = *b->anat[b->smp[sample].anat];
-    const size_t nc = a.nslots * BCELLS;
     const int buf = b->ran ? b->final_buf[p] : 0;  // before the run: the initial state
     const unsigned char* src = (const unsigned char*)b->phi[buf].p + b->slot0[p] * BCELLS * b->real_size;
-    std::vector<unsigned char> bm(nc * b->real_size);
-    GH_HIP_CHECK(hipMemcpyAsync(bm.data(), src, bm.size(), hipMemcpyDeviceToHost, b->stream));
-    GH_HIP_CHECK(hipStreamSynchronize(b->stream));
-    for (size_t c = 0; c < nc; ++c)
-        std::memcpy((unsigned char*)dense + c * b->real_size, bm.data() + block_index(a.bpd, c) * b->real_size,
-                    b->real_size);
-    return GH_OK;
+    return stage_fetch(b->device, b->stream, src, a.nslots * BCELLS, a.bpd, b->real_size, dense);
 }
 
 int gh_batch_get_anatomy(gh_batch* bh, int anatomy_id, void* p_w, void* p_g) {
@@ -1011,18 +1006,11 @@ int gh_batch_get_anatomy(gh_batch* bh, int anatomy_id, void* p_w, void* p_g) {
         return set_error(GH_EINVAL, "gh_batch_get_anatomy: no such anatomy");
     GH_HIP_CHECK(hipSetDevice(b->device));
     const BatchAnatomy& a = *b->anat[anatomy_id];
-    const size_t nc = a.nslots * BCELLS;
-    std::vector<unsigned char> bm(nc * b->real_size);
     const DevBuf* src[2] = {&a.pw, &a.pg};
     void* dst[2] = {p_w, p_g};
-    for (int f = 0; f < 2; ++f) {
-        if (!dst[f]) continue;
-        GH_HIP_CHECK(hipMemcpyAsync(bm.data(), src[f]->p, bm.size(), hipMemcpyDeviceToHost, b->stream));
-        GH_HIP_CHECK(hipStreamSynchronize(b->stream));
-        for (size_t c = 0; c < nc; ++c)
-            std::memcpy((unsigned char*)dst[f] + c * b->real_size, bm.data() + block_index(a.bpd, c) * b->real_size,
-                        b->real_size);
-    }
+    for (int f = 0; f < 2; ++f)
+        if (dst[f])
+            if (int rc = stage_fetch(b->device, b->stream, src[f]->p, a.nslots * BCELLS, a.bpd, b->real_size, dst[f])) return rc;
     return GH_OK;
 }
 

@@ -235,6 +235,16 @@ int grid_compress(Ctx& c, const std::vector<char>& flagged, int* ncollapsed,
                   std::vector<uint64_t>* parents = nullptr, std::vector<int>* old_slot = nullptr,
                   const std::vector<Octree::CollapseCand>* cands = nullptr);
 
+// fields to and from the caller's memory (gh_stage.hip), in stream order; each
+// returns when the caller's memory has been read or written.  The caller's array
+// is block-major like the field for bpd 0, dense x-fastest otherwise (a uniform
+// grid of bpd blocks per dimension).
+int stage_fetch(int device, hipStream_t stream, const void* field, size_t cells, int bpd, size_t real_size, void* dst);
+int stage_send(int device, hipStream_t stream, void* field, size_t cells, int bpd, size_t real_size, const void* src);
+// a context (or batch) that may use them is created / destroyed
+void stage_retain();
+void stage_release();
+
 // likelihood helpers (gh_lik.hip): -logL of the current phi; dJ/du of a state buffer
 int lik_eval_current(Ctx& c, const double* params, int stepPET, int stepTi, int use_roi, double* out,
                      int64_t* npet);

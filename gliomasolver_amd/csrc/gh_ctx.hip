@@ -94,7 +94,7 @@ void Ctx::release_all() {
     labPermOrder = 0;
 }
 
-// dense x-fastest n^3 <-> block-major [slot][z][y][x] for a uniform grid in
+// dense x-fastest n^3 -> block-major [slot][z][y][x] for a uniform grid in
 // slot order bx + bpd*(by + bpd*bz)
 template <typename T>
 static void dense_to_blocks(int n, const T* dense, T* bm) {
@@ -110,20 +110,6 @@ static void dense_to_blocks(int n, const T* dense, T* bm) {
                                     BS * sizeof(T));
             }
 }
-template <typename T>
-static void blocks_to_dense(int n, const T* bm, T* dense) {
-    const int bpd = n / BS;
-    for (int bz = 0; bz < bpd; ++bz)
-        for (int by = 0; by < bpd; ++by)
-            for (int bx = 0; bx < bpd; ++bx) {
-                const T* src = bm + ((size_t)bx + (size_t)bpd * (by + (size_t)bpd * bz)) * BCELLS;
-                for (int z = 0; z < BS; ++z)
-                    for (int y = 0; y < BS; ++y)
-                        std::memcpy(dense + (size_t)BS * bx + (size_t)n * ((size_t)BS * by + y + (size_t)n * (BS * bz + z)),
-                                    src + BS * (y + BS * z), BS * sizeof(T));
-            }
-}
-
 static int check_dense(Ctx* c, int n) {
     if (!c) return set_error(GH_EINVAL, "null context");
     if (c->topo.uniform_bpd <= 0) return set_error(GH_ESTATE, "dense transfer needs a uniform grid");
@@ -279,6 +265,7 @@ int gh_ctx_create(int device, int real_kind, gh_ctx** out) {
     // device (once per device); a failure here leaves every other entry point
     // working and gh_likelihood_noalloc retries and reports it
     (void)lik_scratch_resolve(device);
+    stage_retain();
     *out = reinterpret_cast<gh_ctx*>(c);
     return GH_OK;
 }
@@ -294,6 +281,7 @@ int gh_ctx_destroy(gh_ctx* ctx) {
     if (c->evStage) (void)hipEventDestroy(c->evStage);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    stage_release();
     return GH_OK;
 }
 
@@ -360,14 +348,7 @@ int gh_set_field_dense(gh_ctx* ctx, int field, int n, const void* values) {
     DevBuf* b = field_buf(c, field);
     if (!b || !values) return set_error(GH_EINVAL, "gh_set_field_dense: bad field or null values");
     GH_HIP_CHECK(hipSetDevice(c->device));
-    const size_t nc = c->ncells();
-    std::vector<unsigned char> bm(nc * c->real_size);
-    if (c->real_kind == GH_REAL_F32)
-        dense_to_blocks<float>(n, (const float*)values, (float*)bm.data());
-    else
-        dense_to_blocks<double>(n, (const double*)values, (double*)bm.data());
-    GH_HIP_CHECK(hipMemcpyAsync(b->p, bm.data(), bm.size(), hipMemcpyHostToDevice, c->stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if ((rc = stage_send(c->device, c->stream, b->p, c->ncells(), c->topo.uniform_bpd, c->real_size, values))) return rc;
     if (field == GH_FIELD_PW || field == GH_FIELD_PG) c->prepared = false;
     return GH_OK;
 }
@@ -379,15 +360,7 @@ int gh_get_field_dense(gh_ctx* ctx, int field, int n, void* values) {
     DevBuf* b = field_buf(c, field);
     if (!b || !values) return set_error(GH_EINVAL, "gh_get_field_dense: bad field or null values");
     GH_HIP_CHECK(hipSetDevice(c->device));
-    const size_t nc = c->ncells();
-    std::vector<unsigned char> bm(nc * c->real_size);
-    GH_HIP_CHECK(hipMemcpyAsync(bm.data(), b->p, bm.size(), hipMemcpyDeviceToHost, c->stream));
-    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    if (c->real_kind == GH_REAL_F32)
-        blocks_to_dense<float>(n, (const float*)bm.data(), (float*)values);
-    else
-        blocks_to_dense<double>(n, (const double*)bm.data(), (double*)values);
-    return GH_OK;
+    return stage_fetch(c->device, c->stream, b->p, c->ncells(), c->topo.uniform_bpd, c->real_size, values);
 }
 
 int gh_schedule(int real_kind, double Dw_phys, double L, double tend, int gpd, double cfl, double* Dw, double* Dg,
