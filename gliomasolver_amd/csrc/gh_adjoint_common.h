@@ -34,40 +34,6 @@ inline void adj_param_grads(const double ab[2], double dt, double invDw, double 
     out[2] = (ab[0] + rho * ab[1]) * invN;
 }
 
-// v moved across lanes by the DPP pattern CTRL (both 32-bit halves)
-template <int CTRL>
-__device__ inline double dpp_move(double v) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-__device__ inline double double_of(unsigned lo, unsigned hi) {
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ inline unsigned lo_of(double v) { return (unsigned)(unsigned long long)__double_as_longlong(v); }
-__device__ inline unsigned hi_of(double v) { return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32); }
-// Sums of a and of b over the 64 lanes of a wave (all lanes active): a's in
-// lanes 0-31, b's in lanes 32-63.  The halves of the wave are exchanged so that
-// one addition leaves a's 32 partial sums in the lower and b's in the upper
-// half, then the rows of 16 lanes, then butterflies within a row (lane pairs,
-// quad halves, row half mirror, row mirror: floating-point addition commutes,
-// so every lane of a row ends with the same sum).  Fixed order, no LDS, no
-// barrier; 21 operations for both sums (42 with one reduction each).
-__device__ inline double wave_sum2(double a, double b) {
-    auto lo = __builtin_amdgcn_permlane32_swap(lo_of(a), lo_of(b), false, false);
-    auto hi = __builtin_amdgcn_permlane32_swap(hi_of(a), hi_of(b), false, false);
-    double v = double_of(lo[0], hi[0]) + double_of(lo[1], hi[1]);
-    lo = __builtin_amdgcn_permlane16_swap(lo_of(v), lo_of(v), false, false);
-    hi = __builtin_amdgcn_permlane16_swap(hi_of(v), hi_of(v), false, false);
-    v = double_of(lo[0], hi[0]) + double_of(lo[1], hi[1]);
-    v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp_move<0x141>(v);  // row_half_mirror
-    v += dpp_move<0x140>(v);  // row_mirror
-    return v;
-}
-
 __device__ inline double block_sum(double v, double* red) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void batch_seed_kernel(const AdjJob<Real>* __r
     const AdjJob<Real>& j = jobs[blockIdx.y];
     const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= j.ncells) return;
-    Layout lay{0, 0, 0, j.bpd};
+    const Layout lay{0, 0, 0, j.bpd, bpd_magic(j.bpd)};
     lik_seed_cell<Real>(c, lay, j.u, j.t1, j.fl, j.pet, j.p, full_bern, j.lam);
 }
 
@@ -199,14 +199,14 @@ template <typename T>
 __global__ __launch_bounds__(LIK_THREADS) void batch_lik_partials_kernel(const LikJob<T>* __restrict__ jobs,
                                                                          double* __restrict__ partials) {
     const LikJob<T>& j = jobs[blockIdx.y];
-    Layout lay{0, 0, 0, j.bpd};
-    lik_partials_body<T>((int)blockIdx.x, (int)gridDim.x, j.ncells, lay, j.u, j.t1, j.fl, j.pet, j.roi, j.nroi, j.p,
+    const Layout lay{0, 0, 0, j.bpd, bpd_magic(j.bpd)};
+    lik_partials_body<T>((int)blockIdx.x, j.ncells, lay, j.u, j.t1, j.fl, j.pet, j.roi, j.nroi, j.p,
                          partials + (size_t)blockIdx.y * 4 * LIK_GRID);
 }
 
 __global__ __launch_bounds__(256) void batch_lik_final_kernel(const double* __restrict__ partials,
                                                               double* __restrict__ out) {
-    lik_final_body(LIK_GRID, partials + (size_t)blockIdx.x * 4 * LIK_GRID, out + 4 * (size_t)blockIdx.x);
+    lik_final_body(partials + (size_t)blockIdx.x * 4 * LIK_GRID, out + 4 * (size_t)blockIdx.x);
 }
 
 // dense (x fastest, n = 8*bpd) -> block-major index of a uniform grid

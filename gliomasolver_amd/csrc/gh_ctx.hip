@@ -90,7 +90,7 @@ void Ctx::release_all() {
     faceScan.release();
     dHashKey.release();
     dHashVal.release();
-    for (PinnedBuf* b : {&pinRemap, &pinDense, &pinBlk, &pinSplit, &pinSlots, &pinDet}) b->release();
+    for (PinnedBuf* b : {&pinRemap, &pinDense, &pinBlk, &pinSplit, &pinSlots, &pinDet, &pinLik}) b->release();
     labPermOrder = 0;
 }
 

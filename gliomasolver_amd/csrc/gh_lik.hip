@@ -19,10 +19,10 @@
 namespace gh {
 
 // Partials of gh_likelihood_noalloc: 4 sums per workgroup of the fixed
-// LIK_GRID partition plus the 4 final sums (32.8 KB).  Each GPU holds its own
+// LIK_GRID partition (32.8 KB).  Each GPU holds its own
 // copy until the process ends; in host code the name is only a stand-in, the
 // device address comes from hipGetSymbolAddress (lik_scratch_resolve).
-constexpr int LIK_SCRATCH_DOUBLES = 4 * (LIK_GRID + 1);
+constexpr int LIK_SCRATCH_DOUBLES = 4 * LIK_GRID;
 static __device__ __align__(256) double scratch[LIK_SCRATCH_DOUBLES];
 
 namespace {
@@ -55,17 +55,19 @@ __global__ __launch_bounds__(LIK_THREADS) void lik_partials_kernel(size_t ncells
                                                                    const double* __restrict__ pet,
                                                                    const int4* __restrict__ roi, int nroi,
                                                                    LikParams p, double* __restrict__ partials) {
-    lik_partials_body<T>((int)blockIdx.x, (int)gridDim.x, ncells, lay, u, t1, fl, pet, roi, nroi, p, partials);
+    lik_partials_body<T>((int)blockIdx.x, ncells, lay, u, t1, fl, pet, roi, nroi, p, partials);
 }
 
 // stage 2: one workgroup sums the partials in a fixed order
-__global__ __launch_bounds__(256) void lik_final_kernel(int nparts, const double* __restrict__ partials,
+__global__ __launch_bounds__(256) void lik_final_kernel(const double* __restrict__ partials,
                                                         double* __restrict__ out) {
-    lik_final_body(nparts, partials, out);
+    lik_final_body(partials, out);
 }
 
-// parts: 4 * (LIK_GRID + 1) doubles of device scratch (null: the context's
-// own buffer, allocated on first use); every slot is written before it is read
+// parts: 4 * LIK_GRID doubles of device scratch (null: the context's own buffer,
+// allocated on first use); every slot is written before it is read.  The four
+// sums go straight into pinned memory: a copy of 32 bytes into pageable memory
+// took 12 us of a call's 53.
 template <typename T>
 int run_lik(Ctx& c, size_t ncells, Layout lay, const T* u, const unsigned char* t1, const unsigned char* fl,
             const double* pet, const int4* roi, int nroi, const LikParams& p, double out[4], int64_t* npet,
@@ -75,13 +77,12 @@ int run_lik(Ctx& c, size_t ncells, Layout lay, const T* u, const unsigned char* 
         if (rc) return rc;
         parts = c.likPart.as<double>();
     }
+    double* const sums = c.pinLik.as<double>();
     hipLaunchKernelGGL(lik_partials_kernel<T>, dim3(LIK_GRID), dim3(LIK_THREADS), 0, c.stream, ncells, lay, u, t1,
                        fl, pet, roi, nroi, p, parts);
     GH_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(lik_final_kernel, dim3(1), dim3(256), 0, c.stream, LIK_GRID, parts, parts + 4 * LIK_GRID);
+    hipLaunchKernelGGL(lik_final_kernel, dim3(1), dim3(256), 0, c.stream, parts, sums);
     GH_HIP_CHECK(hipGetLastError());
-    double sums[4];
-    GH_HIP_CHECK(hipMemcpyAsync(sums, parts + 4 * LIK_GRID, sizeof(sums), hipMemcpyDeviceToHost, c.stream));
     GH_HIP_CHECK(hipStreamSynchronize(c.stream));
     finish(sums, p, out, npet);
     return GH_OK;
@@ -110,7 +111,7 @@ int lik_eval_into(Ctx& c, const double* params, int stepPET, int stepTi, int use
     LikParams p;
     int rc = check_params(params, stepPET, stepTi, p);
     if (rc) return rc;
-    Layout lay{0, 0, 0, c.topo.uniform_bpd};
+    const Layout lay = block_layout(c.topo.uniform_bpd);
     const int4* roi = use_roi ? c.obsRoi.as<int4>() : nullptr;
     if (c.real_kind == GH_REAL_F32)
         return run_lik<float>(c, c.ncells(), lay, c.phi[c.cur].as<float>(), c.obsT1.as<unsigned char>(),
@@ -134,7 +135,7 @@ int lik_seed_gradient(Ctx& c, const void* u, double* g, const double* params, in
     int rc = check_params(params, stepPET, stepTi, p);
     if (rc) return rc;
     if (use_roi && c.nroi == 0) return set_error(GH_ESTATE, "likelihood: no ROI was given");
-    Layout lay{0, 0, 0, c.topo.uniform_bpd};
+    const Layout lay = block_layout(c.topo.uniform_bpd);
     const size_t nc = c.ncells();
     const unsigned grid = (unsigned)((nc + 255) / 256);
     if (c.real_kind == GH_REAL_F32)
@@ -187,7 +188,8 @@ int gh_lik_set_data(gh_ctx* ctx, int n, const double* t1c, const double* flair, 
     to_blocks(n, y2.data(), b2.data());
     to_blocks(n, pet, pb.data());
     int rc;
-    if ((rc = c->obsT1.ensure(nc)) || (rc = c->obsFl.ensure(nc)) || (rc = c->obsPet.ensure(nc * sizeof(double))))
+    if ((rc = c->obsT1.ensure(nc)) || (rc = c->obsFl.ensure(nc)) || (rc = c->obsPet.ensure(nc * sizeof(double))) ||
+        (rc = c->pinLik.ensure_grow(4 * sizeof(double))))
         return rc;
     GH_HIP_CHECK(hipMemcpyAsync(c->obsT1.p, b1.data(), nc, hipMemcpyHostToDevice, c->stream));
     GH_HIP_CHECK(hipMemcpyAsync(c->obsFl.p, b2.data(), nc, hipMemcpyHostToDevice, c->stream));
@@ -228,7 +230,7 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
     if (!c || !out) return set_error(GH_EINVAL, "null argument");
     // the partition is fixed at LIK_GRID workgroups whatever the grid size, so
     // the scratch bounds the partition, not the grid
-    static_assert(LIK_SCRATCH_DOUBLES == 4 * (LIK_GRID + 1), "scratch holds the LIK_GRID partials + 4 sums");
+    static_assert(LIK_SCRATCH_DOUBLES == 4 * LIK_GRID, "scratch holds the LIK_GRID partials");
     GH_HIP_CHECK(hipSetDevice(c->device));
     int rc = lik_scratch_resolve(c->device);  // a no-op once gh_ctx_create has resolved it
     if (rc) return rc;
@@ -262,7 +264,7 @@ int gh_likelihood_dense(gh_ctx* ctx, int nx, int ny, int nz, const double* model
     }
     DevBuf dm, dy1, dy2, dp, dr;
     if ((rc = dm.ensure(nc * 8)) || (rc = dy1.ensure(nc)) || (rc = dy2.ensure(nc)) || (rc = dp.ensure(nc * 8)) ||
-        (rc = dr.ensure((size_t)nroi * sizeof(int4)))) {
+        (rc = dr.ensure((size_t)nroi * sizeof(int4))) || (rc = c->pinLik.ensure_grow(4 * sizeof(double)))) {
         dm.release(); dy1.release(); dy2.release(); dp.release(); dr.release();
         return rc;
     }
@@ -272,7 +274,7 @@ int gh_likelihood_dense(gh_ctx* ctx, int nx, int ny, int nz, const double* model
     GH_HIP_CHECK(hipMemcpyAsync(dp.p, pet, nc * 8, hipMemcpyHostToDevice, c->stream));
     if (nroi > 0)
         GH_HIP_CHECK(hipMemcpyAsync(dr.p, q.data(), nroi * sizeof(int4), hipMemcpyHostToDevice, c->stream));
-    Layout lay{nx, ny, nz, 0};
+    const Layout lay{nx, ny, nz, 0, 0};
     rc = run_lik<double>(*c, nc, lay, dm.as<double>(), dy1.as<unsigned char>(), dy2.as<unsigned char>(),
                          dp.as<double>(), nroi > 0 ? dr.as<int4>() : nullptr, nroi, p, out, npet);
     (void)hipStreamSynchronize(c->stream);
