@@ -302,7 +302,7 @@ int build_layout_t(Batch& b) {
     if ((rc = b.phi[0].ensure(nc * sizeof(Real))) || (rc = b.phi[1].ensure(nc * sizeof(Real))) ||
         (rc = b.statD.ensure(nc * sizeof(Stat4<Real>))) || (rc = b.statSig.ensure(nc * sizeof(Real))) ||
         (rc = b.statF.ensure_grow(std::max<size_t>(1, nc) * sizeof(Stat4<Real>))) ||
-        (rc = b.zeroFlux.ensure_grow(std::max<size_t>(1, nsl))) || (rc = b.slotPos.ensure(nsl * sizeof(int32_t))) ||
+        (rc = b.zeroFlux.ensure_grow(nsl + 3)) || (rc = b.slotPos.ensure(nsl * sizeof(int32_t))) ||
         (rc = b.range.ensure(ns * sizeof(SlotRange<Real>))) || (rc = b.apw.ensure(ns * sizeof(void*))) ||
         (rc = b.apg.ensure(ns * sizeof(void*))))
         return rc;
@@ -534,10 +534,8 @@ struct ForwardSweep {
             hipLaunchKernelGGL((rd_step2_kernel<Real, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
                                b.stream, nsl, per_xcd, in, out, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(), prm);
         } else {
-            const int per_xcd = ((nsl + 1) / 2 + 7) / 8;  // two blocks per workgroup
-            hipLaunchKernelGGL((rd_step_kernel<Real, true, 2, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512),
-                               0, b.stream, nsl, per_xcd, in, out, b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
-                               prm);
+            launch_step_kernel<Real, true, 2>(b.stream, nsl, b.zeroFlux, in, out, b.statD.as<Stat4<Real>>(),
+                                              b.statSig.as<Real>(), prm);
         }
         cur = 1 - cur;
         return two ? 2 : 1;
@@ -642,10 +640,8 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     const BatchStepParams<Real> fprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
     auto step = [&](const void* in, void* out, int nslots) {  // one Euler step (tape recompute)
-        const int per_xcd = ((nslots + 1) / 2 + 7) / 8;
-        hipLaunchKernelGGL((rd_step_kernel<Real, true, 2, BatchStepParams<Real>>), dim3(8 * per_xcd), dim3(512), 0,
-                           b.stream, nslots, per_xcd, (const Real*)in, (Real*)out, b.statD.as<Stat4<Real>>(),
-                           b.statSig.as<Real>(), fprm);
+        launch_step_kernel<Real, true, 2>(b.stream, nslots, b.zeroFlux, (const Real*)in, (Real*)out, b.statD.as<Stat4<Real>>(),
+                                          b.statSig.as<Real>(), fprm);
     };
     char* ck = (char*)b.ck.p;
     char* tape = (char*)b.tape.p;
@@ -718,7 +714,6 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         // the two gets a second state past its end that no reverse step reads
         for (int64_t k = k0; k < k1;) {
             char* in = tape + (size_t)(k - k0) * nsl * slot_bytes;
-            const int nslots = (int)b.slot0[active(k)];
             if (b.fast_ok && k >= 1) {
                 const bool two = k + 2 <= k1;
                 Real* next = (Real*)(in + (size_t)nsl * slot_bytes);
@@ -727,7 +722,7 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
                                            two ? next : (Real*)nullptr, b.statF.as<Stat4<Real>>(), fprm);
                 k += two ? 2 : 1;
             } else {
-                step(in, in + (size_t)nsl * slot_bytes, nslots);
+                step(in, in + (size_t)nsl * slot_bytes, (int)b.slot0[active(k)]);
                 k += 1;
             }
         }

@@ -285,89 +285,6 @@ struct UniformStepParams {
     __device__ inline BlockPos pos(int s) const { return block_pos(s, 0, bpd, magic); }
 };
 
-// BPW blocks per workgroup of 512 lanes; lane = cell (x fastest) of each
-// block.  All loads of a lane (BPW cells, one vector load of constants each)
-// are issued before the first wait.  Group mapping is XCD-aware: consecutive
-// workgroups land on different XCDs, so workgroup w serves group
-// (w % 8) * per_xcd + w / 8 and each XCD sweeps a contiguous range of blocks
-// whose halos stay in its own L2.
-template <typename Real, bool FUSED, int BPW, typename Params>
-__global__ __launch_bounds__(512) void rd_step_kernel(int nslots, int per_xcd,
-                                                      const Real* __restrict__ phi, Real* __restrict__ out,
-                                                      const Stat4<Real>* __restrict__ st,
-                                                      const Real* __restrict__ sig, Params prm) {
-    const int grp = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-    if (grp * BPW >= nslots) return;
-    __shared__ Real s_phi[BPW][1000];
-    __shared__ unsigned char s_out[BPW][1000];
-    __shared__ Real s_Dx[BPW][576], s_Dy[BPW][576], s_Dz[BPW][576];
-
-    const int t = threadIdx.x;
-    const int x = t & 7, y = (t >> 3) & 7, z = t >> 6;
-    Real pc[BPW], sc[BPW];
-    Stat4<Real> sv[BPW];
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-        const int s = grp * BPW + j;
-        if (s >= nslots) break;
-        const size_t g = (size_t)s * BCELLS + t;
-        pc[j] = phi[g];
-        sv[j] = st[g];
-        sc[j] = sig[g];
-    }
-    if (t < 384) {  // six face halos of 64 cells, one lane each
-        const int f = t >> 6, u = t & 7, v = (t >> 3) & 7;
-        int src, dst;
-        switch (f) {
-            case FXM: src = 7 + 8 * u + 64 * v; dst = P(-1, u, v); break;
-            case FXP: src = 0 + 8 * u + 64 * v; dst = P(8, u, v); break;
-            case FYM: src = u + 8 * 7 + 64 * v; dst = P(u, -1, v); break;
-            case FYP: src = u + 8 * 0 + 64 * v; dst = P(u, 8, v); break;
-            case FZM: src = u + 8 * v + 64 * 7; dst = P(u, v, -1); break;
-            default:  src = u + 8 * v + 64 * 0; dst = P(u, v, 8); break;
-        }
-#pragma unroll
-        for (int j = 0; j < BPW; ++j) {
-            const int s = grp * BPW + j;
-            if (s >= nslots) break;
-            const size_t nb = (size_t)face_nb(prm.pos(s), f) * BCELLS + src;
-            const Real ph = phi[nb];
-            const Stat4<Real> hs = st[nb];
-            s_phi[j][dst] = ph;
-            s_out[j][dst] = ph < hs.tau;
-            if (f == FXM) s_Dx[j][v * 72 + u * 9] = hs.dx;
-            else if (f == FYM) s_Dy[j][v * 72 + u] = hs.dy;
-            else if (f == FZM) s_Dz[j][v * 8 + u] = hs.dz;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-        if (grp * BPW + j >= nslots) break;
-        s_phi[j][P(x, y, z)] = pc[j];
-        s_out[j][P(x, y, z)] = pc[j] < sv[j].tau;
-        s_Dx[j][z * 72 + y * 9 + x + 1] = sv[j].dx;
-        s_Dy[j][z * 72 + (y + 1) * 8 + x] = sv[j].dy;
-        s_Dz[j][(z + 1) * 64 + y * 8 + x] = sv[j].dz;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-        const int s = grp * BPW + j;
-        if (s >= nslots) break;
-        Real rho;
-        double ih2, dt;
-        prm.get(s, rho, ih2, dt);
-        const Real d = rd_cell_rhs<Real>(
-            s_Dx[j][z * 72 + y * 9 + x], sv[j].dx, s_Dy[j][z * 72 + y * 8 + x], sv[j].dy,
-            s_Dz[j][z * 64 + y * 8 + x], sv[j].dz, s_phi[j][P(x - 1, y, z)], s_phi[j][P(x + 1, y, z)],
-            s_phi[j][P(x, y - 1, z)], s_phi[j][P(x, y + 1, z)], s_phi[j][P(x, y, z - 1)], s_phi[j][P(x, y, z + 1)],
-            s_out[j][P(x - 1, y, z)], s_out[j][P(x + 1, y, z)], s_out[j][P(x, y - 1, z)],
-            s_out[j][P(x, y + 1, z)], s_out[j][P(x, y, z - 1)], s_out[j][P(x, y, z + 1)], pc[j], sc[j], rho, ih2);
-        out[(size_t)s * BCELLS + t] = FUSED ? rd_update(pc[j], d, dt) : d;
-    }
-}
-
-
 // Two fused Euler steps per launch (temporal blocking): one workgroup per 8^3
 // block.  Step 1 is evaluated on the block and its six depth-1 face halos
 // (the cells step 2 reads), from the state on the block, the depth-1 and
@@ -707,6 +624,98 @@ constexpr int ZF_GROUP = 8;  // blocks without diffusion per workgroup
 // the first nfull blocks and ngrp groups of a list
 inline StepWork step_work(int nfull, const int32_t* full, int ngrp, const int2* grp, const unsigned char* still) {
     return StepWork{nfull, (nfull + 7) / 8, ngrp, (ngrp + 7) / 8, full, grp, still};
+}
+
+// One step, or dphidt, of any state.  BPW blocks per workgroup of 512 lanes; lane =
+// cell (x fastest) of each block.  All loads of a lane -- wave w < 6 the halo of
+// face w, one vector load of constants per cell -- are issued before the first
+// wait.  A block without diffusion (zflux[s] != 0, constants_kernel) has +0 in
+// every face coefficient: its records are not read, 16 of 28 B a cell.  Group
+// mapping is XCD-aware: consecutive workgroups land on different XCDs, so
+// workgroup w serves group (w % 8) * per_xcd + w / 8 and each XCD sweeps a
+// contiguous range of blocks, whose halos -- and, from launch to launch, states --
+// stay in its own L2.  (The work list of the two-step kernel, which deals the two
+// kinds of blocks out evenly, gives an XCD other blocks' states than the kernels
+// around it do: dphidt 15.1 us, and rd_update 7.4 instead of 5.1.)  dphidt of
+// 128^3 FP32, 62 % of the blocks without diffusion: 13.7 -> 9.3 us; a step of 24
+// samples of 96^3 148 -> 105 us.
+template <typename Real, bool FUSED, int BPW, typename Params>
+__global__ __launch_bounds__(512) void rd_step_kernel(int nslots, int per_xcd, const uint32_t* __restrict__ zflux,
+                                                      const Real* __restrict__ phi, Real* __restrict__ out,
+                                                      const Stat4<Real>* __restrict__ st,
+                                                      const Real* __restrict__ sig, Params prm) {
+    const int s0 = ((int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8)) * BPW;
+    if (s0 >= nslots) return;
+    __shared__ Real s_phi[BPW][1000];
+    __shared__ unsigned char s_out[BPW][1000];
+    __shared__ Real s_Dx[BPW][576], s_Dy[BPW][576], s_Dz[BPW][576];
+
+    const int t = threadIdx.x;
+    const int x = t & 7, y = (t >> 3) & 7, z = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t zf = zflux[s0 >> 2] >> (8 * (s0 & 3));  // a byte per block; BPW divides 4
+    const int f = z;                                       // this wave's face
+    const bool fx = f < 2, fz = f >= 4, plus = f & 1;
+    const int lane = x + 8 * y;
+    // cell (x, y) of the face in the neighbour block and in the tile
+    const int src = fx ? (plus ? 0 : 7) + 8 * lane : (fz ? lane + (plus ? 0 : 448) : x + (plus ? 0 : 56) + 64 * y);
+    const int dst = fx ? P(plus ? 8 : -1, x, y) : (fz ? P(x, y, plus ? 8 : -1) : P(x, plus ? 8 : -1, y));
+    Real pc[BPW], sc[BPW], ph[BPW];
+    Stat4<Real> sv[BPW], hs[BPW];
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+        const int s = s0 + j;
+        if (s >= nslots) break;
+        const size_t nb = (size_t)(f < 6 ? face_nb(prm.pos(s), f) : s) * BCELLS, base = (size_t)s * BCELLS;
+        ph[j] = (phi + nb)[src];
+        pc[j] = (phi + base)[t];
+        sc[j] = (sig + base)[t];
+        hs[j] = sv[j] = Stat4<Real>{0, 0, 0, 0};
+        if (!((zf >> (8 * j)) & 0xffu)) {
+            hs[j] = (st + nb)[src];
+            sv[j] = (st + base)[t];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+        if (s0 + j >= nslots) break;
+        if (f < 6) {
+            s_phi[j][dst] = ph[j];
+            s_out[j][dst] = ph[j] < hs[j].tau;
+            if (f == FXM) s_Dx[j][y * 72 + x * 9] = hs[j].dx;
+            else if (f == FYM) s_Dy[j][y * 72 + x] = hs[j].dy;
+            else if (f == FZM) s_Dz[j][y * 8 + x] = hs[j].dz;
+        }
+        s_phi[j][P(x, y, z)] = pc[j];
+        s_out[j][P(x, y, z)] = pc[j] < sv[j].tau;
+        s_Dx[j][z * 72 + y * 9 + x + 1] = sv[j].dx;
+        s_Dy[j][z * 72 + (y + 1) * 8 + x] = sv[j].dy;
+        s_Dz[j][(z + 1) * 64 + y * 8 + x] = sv[j].dz;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+        const int s = s0 + j;
+        if (s >= nslots) break;
+        Real rho;
+        double ih2, dt;
+        prm.get(s, rho, ih2, dt);
+        const Real d = rd_cell_rhs<Real>(
+            s_Dx[j][z * 72 + y * 9 + x], sv[j].dx, s_Dy[j][z * 72 + y * 8 + x], sv[j].dy,
+            s_Dz[j][z * 64 + y * 8 + x], sv[j].dz, s_phi[j][P(x - 1, y, z)], s_phi[j][P(x + 1, y, z)],
+            s_phi[j][P(x, y - 1, z)], s_phi[j][P(x, y + 1, z)], s_phi[j][P(x, y, z - 1)], s_phi[j][P(x, y, z + 1)],
+            s_out[j][P(x - 1, y, z)], s_out[j][P(x + 1, y, z)], s_out[j][P(x, y - 1, z)],
+            s_out[j][P(x, y + 1, z)], s_out[j][P(x, y, z - 1)], s_out[j][P(x, y, z + 1)], pc[j], sc[j], rho, ih2);
+        out[(size_t)s * BCELLS + t] = FUSED ? rd_update(pc[j], d, dt) : d;
+    }
+}
+// rd_step_kernel over slots [0, nslots); zflux: a byte per slot, padded to four
+template <typename Real, bool FUSED, int BPW, typename Params>
+void launch_step_kernel(hipStream_t stream, int nslots, const DevBuf& zflux, const Real* in, Real* out,
+                        const Stat4<Real>* st, const Real* sig, const Params& prm) {
+    static_assert(BPW == 1 || BPW == 2 || BPW == 4, "a workgroup's flags lie in one word");
+    const int per_xcd = ((nslots + BPW - 1) / BPW + 7) / 8;
+    hipLaunchKernelGGL((rd_step_kernel<Real, FUSED, BPW, Params>), dim3(8 * per_xcd), dim3(512), 0, stream, nslots,
+                       per_xcd, zflux.as<uint32_t>(), in, out, st, sig, prm);
 }
 
 // Zero is a fixed point of a block without diffusion: the reaction of 0 is 0.
