@@ -22,8 +22,11 @@
 // A = sum w_c Rdiff_c and B = sum w_c u_c (1 - u_c), which are accumulated in
 // FP64 per wave (dt, rho, N and Dw are constant over the solve and applied
 // once at the end); every wave owns the same cells in every step, so the
-// accumulation order is fixed.  States u_k are recomputed per segment of K
-// steps from checkpoints taken in the forward sweep.
+// accumulation order is fixed.  The states that fit the tape
+// (tape_ensure) stay on it from the forward sweep, which writes them there; the
+// steps before them are cut into segments of the tape's length, recomputed from
+// checkpoints taken in the forward sweep.  With every segment recomputed, 343
+// steps of 64^3 FP64 took 3.3 ms (2.7 with none), 1,000 of 128^3 FP32 12.8 (11.0).
 #include <cmath>
 #include <vector>
 
@@ -38,36 +41,65 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
               const double* ic, double sigma, double* loss, double* grad) {
     const size_t nc = c.ncells();
     const size_t nb = nc * sizeof(Real);
-    const int64_t nck = (N + K - 1) / K;
     int rc;
-    if ((rc = c.adjCk.ensure((size_t)nck * nb)) || (rc = c.adjSeg.ensure((size_t)(K + 1) * nb)) ||
-        (rc = c.adjLam[0].ensure(nc * 8)) || (rc = c.adjLam[1].ensure(nc * 8)))
+    if ((rc = tape_ensure(c.adjSeg, ((size_t)std::min<int64_t>(K, N) + 1) * nb, ((size_t)N + 1) * nb))) return rc;
+    // segments of `len` steps, the first one shorter; the last stays on the tape
+    const int64_t len = std::min<int64_t>(N, (int64_t)(c.adjSeg.bytes / nb) - 1);
+    const int64_t nseg = (N + len - 1) / len;
+    auto start = [&](int64_t i) { return i == 0 ? (int64_t)0 : N - (nseg - i) * len; };
+    if ((rc = c.adjCk.ensure(std::max<size_t>(1, (size_t)(nseg - 1)) * nb)) || (rc = c.adjLam[0].ensure(nc * 8)) ||
+        (rc = c.adjLam[1].ensure(nc * 8)))
         return rc;
     const double dt = T / (double)N;
     char* ck = (char*)c.adjCk.p;
     char* seg = (char*)c.adjSeg.p;
-    // forward sweep with checkpoints every K steps; two steps per launch from
-    // a clamped state (k >= 1) when no checkpoint falls in between
+    // two steps per launch from a clamped state (k >= 1) within a segment
     const bool pairs = c.fast_ok && c.topo.uniform_bpd > 0;
     // the two-step schedule (tile 0) leaves out the groups of blocks without
     // diffusion that u_1 leaves at zero, in both directions
     const bool skip = pairs && c.rd_bpw == 0 && c.nGrp > 0;
-    for (int64_t k = 0; k < N;) {
-        if (k == 1 && skip && (rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p))) return rc;
-        if (k % K == 0)
-            GH_HIP_CHECK(hipMemcpyAsync(ck + (size_t)(k / K) * nb, c.phi[c.cur].p, nb, hipMemcpyDeviceToDevice,
-                                        c.stream));
-        if (pairs && k >= 1 && k + 2 <= N && (k + 1) % K != 0) {
-            if ((rc = rd_step2_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, nullptr, dt, skip))) return rc;
-            k += 2;
-        } else {
-            if ((rc = pairs && k >= 1 ? rd_step1_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt, skip)
-                                      : rd_step_buffers(c, c.phi[c.cur].p, c.phi[1 - c.cur].p, dt)))
-                return rc;
-            k += 1;
+    // u_{k+1} (and u_{k+2}: returns 2) from u_k in `in`
+    auto launch = [&](int64_t k, int64_t end, const void* in, void* one, void* mid, void* two, int* steps) -> int {
+        *steps = pairs && k >= 1 && k + 2 <= end ? 2 : 1;
+        if (*steps == 2) return rd_step2_buffers(c, in, two, mid, dt, skip);
+        return pairs && k >= 1 ? rd_step1_buffers(c, in, one, dt, skip) : rd_step_buffers(c, in, one, dt);
+    };
+    // u_{k0+1} .. u_end on the tape, u_k0 at its start; u_N goes to last (if not null)
+    auto run_on_tape = [&](int64_t k0, int64_t end, void* last) -> int {
+        for (int64_t k = k0; k < end;) {
+            char* in = seg + (size_t)(k - k0) * nb;
+            auto at = [&](int64_t s) { return s == N && last ? (char*)last : seg + (size_t)(s - k0) * nb; };
+            if (k == 1 && k0 == 0 && last && skip) {  // (the first sweep: the marks are not known yet)
+                if ((rc = rd_mark_still(c, in, last)) || (rc = rd_zero_still(c, seg + 2 * nb, len - 1))) return rc;
+            }
+            int steps;
+            if ((rc = launch(k, end, in, at(k + 1), at(k + 1), at(k + 2), &steps))) return rc;
+            k += steps;
         }
-        c.cur = 1 - c.cur;
+        return GH_OK;
+    };
+    // forward sweep
+    for (int64_t i = 0; i + 1 < nseg; ++i) {
+        const int64_t end = start(i + 1);
+        GH_HIP_CHECK(hipMemcpyAsync(ck + (size_t)i * nb, c.phi[c.cur].p, nb, hipMemcpyDeviceToDevice, c.stream));
+        for (int64_t k = start(i); k < end;) {
+            if (k == 1 && skip && ((rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p)) ||
+                                   (rc = rd_zero_still(c, seg, len + 1))))
+                return rc;
+            void* out = c.phi[1 - c.cur].p;
+            int steps;
+            if ((rc = launch(k, end, c.phi[c.cur].p, out, nullptr, out, &steps))) return rc;
+            k += steps;
+            c.cur = 1 - c.cur;
+        }
     }
+    const int64_t tape0 = start(nseg - 1);
+    if (tape0 == 1 && skip && ((rc = rd_mark_still(c, c.phi[c.cur].p, c.phi[1 - c.cur].p)) ||
+                               (rc = rd_zero_still(c, seg, len + 1))))
+        return rc;
+    GH_HIP_CHECK(hipMemcpyAsync(seg, c.phi[c.cur].p, nb, hipMemcpyDeviceToDevice, c.stream));
+    if ((rc = run_on_tape(tape0, N, c.phi[1 - c.cur].p))) return rc;
+    c.cur = 1 - c.cur;
     // loss at u_N and its gradient as the terminal adjoint
     int64_t npet = 0;
     if ((rc = lik_eval_current(c, lik, stepPET, stepTi, use_roi, loss, &npet))) return rc;
@@ -78,10 +110,8 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
                        c.adjLam[lc].as<double>(), (const Real*)c.phi[c.cur].p);
     GH_HIP_CHECK(hipGetLastError());
     const bool still = skip && N > 1;  // (marked before step 1)
-    if (still) {  // what the launches leave out: zero states, the seed in both adjoint buffers
-        if ((rc = rd_zero_still(c, seg, K + 1))) return rc;
+    if (still)  // the launches leave out the seed in the still groups: it stands in both adjoint buffers
         GH_HIP_CHECK(hipMemcpyAsync(c.adjLam[1 - lc].p, c.adjLam[lc].p, nc * 8, hipMemcpyDeviceToDevice, c.stream));
-    }
     // reverse sweep
     const int ns = c.topo.nblocks();
     if ((rc = c.adjPart.ensure(sizeof(double) * ADJ_PART * ns))) return rc;
@@ -95,22 +125,11 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     // nothing out
     const StepWork all = c.rd_bpw == 0 ? rd_step_work(c, false) : step_work(ns, nullptr, 0, nullptr, nullptr);
     const StepWork moving = still ? rd_step_work(c, true) : all;
-    for (int64_t sgi = nck - 1; sgi >= 0; --sgi) {
-        const int64_t k0 = sgi * K, k1 = std::min<int64_t>(N, k0 + K);
-        GH_HIP_CHECK(hipMemcpyAsync(seg, ck + (size_t)sgi * nb, nb, hipMemcpyDeviceToDevice, c.stream));
-        for (int64_t j = 0; j < k1 - k0;) {  // the segment's states, pairs from clamped states
-            if (pairs && k0 + j >= 1 && j + 2 <= k1 - k0) {
-                if ((rc = rd_step2_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 2) * nb,
-                                           seg + (size_t)(j + 1) * nb, dt, still)))
-                    return rc;
-                j += 2;
-            } else {
-                if ((rc = pairs && k0 + j >= 1
-                              ? rd_step1_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 1) * nb, dt, still)
-                              : rd_step_buffers(c, seg + (size_t)j * nb, seg + (size_t)(j + 1) * nb, dt)))
-                    return rc;
-                j += 1;
-            }
+    for (int64_t i = nseg - 1; i >= 0; --i) {
+        const int64_t k0 = start(i), k1 = i + 1 < nseg ? start(i + 1) : N;
+        if (i + 1 < nseg) {
+            GH_HIP_CHECK(hipMemcpyAsync(seg, ck + (size_t)i * nb, nb, hipMemcpyDeviceToDevice, c.stream));
+            if ((rc = run_on_tape(k0, k1 - 1, nullptr))) return rc;
         }
         for (int64_t k = k1 - 1; k >= k0; --k) {
             const Real* uk = (const Real*)(seg + (size_t)(k - k0) * nb);
@@ -132,7 +151,7 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     const unsigned igrid = 512;
     if ((rc = c.likPart.ensure(sizeof(double) * 4 * 1025))) return rc;
     hipLaunchKernelGGL(adj_ic_partials<Real>, dim3(igrid), dim3(256), 0, c.stream, nc, c.topo.uniform_bpd,
-                       c.adjLam[lc].as<double>(), (const Real*)ck, ic[0], ic[1], ic[2], 1.0 / (sigma * sigma),
+                       c.adjLam[lc].as<double>(), (const Real*)seg, ic[0], ic[1], ic[2], 1.0 / (sigma * sigma),
                        c.likPart.as<double>());
     GH_HIP_CHECK(hipGetLastError());
     std::vector<double> pp(ADJ_PART * (size_t)ns), ip(3 * igrid);

@@ -490,6 +490,25 @@ int set_adjoint_samples_t(Batch& b, const double* params, const int64_t* nsteps,
 // taken when no running sample ends after the first of them and (with
 // checkpoints every K) the state after the first is not a checkpoint.  A
 // sample's final state is in the buffer current when it ends.
+// the slots of full[f0 ..] and of the moving groups of grp[g0 ..] from one state to
+// another, an item per workgroup, nf of the first kind
+template <typename Real>
+__global__ __launch_bounds__(256) void copy_moving_kernel(int nf, const int32_t* __restrict__ full,
+                                                          const int2* __restrict__ grp,
+                                                          const unsigned char* __restrict__ still,
+                                                          const Real* __restrict__ src, Real* __restrict__ dst) {
+    const int i = blockIdx.x;
+    int s, n = 1;
+    if (i < nf) {
+        s = full[i];
+    } else {
+        if (still[i - nf]) return;
+        s = grp[i - nf].x;
+        n = grp[i - nf].y;
+    }
+    for (int c = threadIdx.x; c < n * BCELLS; c += 256) dst[(size_t)s * BCELLS + c] = src[(size_t)s * BCELLS + c];
+}
+
 template <typename Real>
 struct ForwardSweep {
     Batch& b;
@@ -518,12 +537,12 @@ struct ForwardSweep {
     void retire(int64_t k) {
         while (active > 0 && npos[active - 1] <= k) b.final_buf[--active] = cur;
     }
-    // one launch from step k; returns the steps taken.  From step 1 on every
+    // one launch from step k, up to step end; returns the steps taken.  From step 1 on every
     // running state was written by the fused update (clamped), so pairs take
     // rd_step2f_kernel when the anatomies allow it.
-    int launch(int64_t k, int K) {
+    int launch(int64_t k, int64_t end) {
         const int nsl = (int)b.slot0[active];
-        const bool two = npos[active - 1] >= k + 2 && (K <= 0 || (k + 1) % K != 0) && (k >= 1 || !b.fast_ok);
+        const bool two = std::min(npos[active - 1], end) >= k + 2 && (k >= 1 || !b.fast_ok);
         const Real* in = b.phi[cur].as<Real>();
         Real* out = b.phi[1 - cur].as<Real>();
         if (b.fast_ok && k >= 1) {
@@ -552,7 +571,7 @@ int run_t(Batch& b, double* elapsed_ms) {
     while (true) {
         fw.retire(k);
         if (k >= maxsteps) break;
-        k += fw.launch(k, 0);
+        k += fw.launch(k, maxsteps);
     }
     GH_HIP_CHECK(hipGetLastError());
     GH_HIP_CHECK(hipEventRecord(b.ev1, b.stream));
@@ -610,11 +629,13 @@ int likelihood_t(Batch& b, const double* lik, int stepPET, int stepTi, int use_r
 }
 
 
-// Forward sweep with checkpoints every K steps, loss, seed, reverse sweep
-// with per-segment recompute, initial-condition gradient -- gh_rd_adjoint for
-// every sample, the samples still running at a step forming a slot prefix in
-// both directions (the reverse of sample s starts at its own step N_s - 1,
-// with its seed placed in the adjoint buffer of parity N_s).
+// Forward sweep, loss, seed, reverse sweep, initial-condition gradient --
+// gh_rd_adjoint for every sample, the samples still running at a step forming a
+// slot prefix in both directions (the reverse of sample s starts at its own step
+// N_s - 1, with its seed placed in the adjoint buffer of parity N_s).  The tape
+// holds the states of the last segment of steps from the forward sweep on
+// (tape_ensure), each the slots of the samples that reached it; earlier segments
+// are recomputed from a checkpoint at their start.
 template <typename Real>
 int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int use_roi, double* loss, double* grad,
               double* elapsed_ms) {
@@ -627,37 +648,119 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
                      npos.begin());
     };
     const size_t slot_bytes = BCELLS * sizeof(Real);
-    const int64_t J = (Nmax + K - 1) / K;
-    std::vector<size_t> ckoff(J + 1, 0);
-    for (int64_t j = 0; j < J; ++j) ckoff[j + 1] = ckoff[j] + b.slot0[active(j * K)];
     const size_t nsl = b.nslots(), nc = nsl * BCELLS;
+    // slots of the states before state k: sample p has states 0 .. N_p
+    std::vector<size_t> ended(ns + 1, 0);
+    for (int p = ns - 1; p >= 0; --p)
+        ended[p] = ended[p + 1] + (b.slot0[p + 1] - b.slot0[p]) * (size_t)(npos[p] + 1);
+    auto cum = [&](int64_t k) {
+        const int p = active(k - 1);
+        return b.slot0[p] * (size_t)k + ended[p];
+    };
     constexpr int IC_GRID = 512;
     int rc;
-    if ((rc = b.ck.ensure(ckoff[J] * slot_bytes)) || (rc = b.tape.ensure((size_t)(K + 1) * nsl * slot_bytes)) ||
-        (rc = b.lam[0].ensure(nc * 8)) || (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
+    if ((rc = tape_ensure(b.tape, (size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes,
+                          cum(Nmax + 1) * slot_bytes)))
+        return rc;
+    // segments [start[i], start[i + 1]) of steps, as long as the tape takes
+    std::vector<int64_t> start{Nmax};
+    for (int64_t e = Nmax; e > 0;) {
+        int64_t lo = 0, hi = e - 1;  // (one step always fits)
+        while (lo < hi) {
+            const int64_t s = (lo + hi) / 2;
+            if ((cum(e + 1) - cum(s)) * slot_bytes <= b.tape.bytes) hi = s;
+            else lo = s + 1;
+        }
+        start.push_back(e = hi);
+    }
+    std::reverse(start.begin(), start.end());
+    const int nseg = (int)start.size() - 1;
+    std::vector<size_t> ckoff(nseg, 0);
+    for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
+    if ((rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes)) || (rc = b.lam[0].ensure(nc * 8)) ||
+        (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
         (rc = b.icpart.ensure((size_t)ns * 3 * IC_GRID * 8)) || (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
     const BatchStepParams<Real> fprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
-    auto step = [&](const void* in, void* out, int nslots) {  // one Euler step (tape recompute)
-        launch_step_kernel<Real, true, 2>(b.stream, nslots, b.zeroFlux, (const Real*)in, (Real*)out, b.statD.as<Stat4<Real>>(),
-                                          b.statSig.as<Real>(), fprm);
-    };
     char* ck = (char*)b.ck.p;
-    char* tape = (char*)b.tape.p;
+    auto state = [&](int seg, int64_t k) {
+        return (Real*)((char*)b.tape.p + (cum(k) - cum(start[seg])) * slot_bytes);
+    };
+    // the tape's zeros that no launch writes, over runs of states of one size
+    auto zero_still = [&](int seg) -> int {
+        for (int64_t k = start[seg] + 1; b.skip_still && k < start[seg + 1];) {
+            const int p = active(k - 1);
+            const int64_t end = std::min(start[seg + 1], npos[p - 1] + 1);
+            launch_still_zero<Real>(b.stream, b.nGrp[p - 1], b.grpList, b.stillGrp, b.zeroFlux, fprm, state(seg, k),
+                                    b.slot0[p] * BCELLS, end - k);
+            GH_HIP_CHECK(hipGetLastError());
+            k = end;
+        }
+        return GH_OK;
+    };
+    // states of the running samples on the tape from step k to end, two steps per
+    // launch from clamped states (k >= 1); done(k) is called with state k there
+    auto run_on_tape = [&](int seg, int64_t end, auto done) -> int {
+        for (int64_t k = start[seg];;) {
+            if (int e = done(k)) return e;
+            if (k >= end) return GH_OK;
+            const int p = active(k);
+            if (b.fast_ok && k >= 1) {
+                const bool two = std::min(npos[p - 1], end) >= k + 2;
+                launch_step2f_kernel<Real>(b.stream, b.work(p), b.plain_dom, two, (const Real*)state(seg, k),
+                                           state(seg, two ? k + 2 : k + 1), two ? state(seg, k + 1) : (Real*)nullptr,
+                                           b.statF.as<Stat4<Real>>(), fprm);
+                k += two ? 2 : 1;
+            } else {
+                launch_step_kernel<Real, true, 2>(b.stream, (int)b.slot0[p], b.zeroFlux, (const Real*)state(seg, k),
+                                                  state(seg, k + 1), b.statD.as<Stat4<Real>>(), b.statSig.as<Real>(),
+                                                  fprm);
+                k += 1;
+            }
+            GH_HIP_CHECK(hipGetLastError());
+        }
+    };
     GH_HIP_CHECK(hipEventRecord(b.ev0, b.stream));
-    // forward, with a checkpoint of the running samples every K steps
     ForwardSweep<Real> fw(b);
     if ((rc = fw.mark())) return rc;
-    for (int64_t k = 0;;) {
-        fw.retire(k);
-        if (k >= Nmax) break;
-        if (k % K == 0)
-            GH_HIP_CHECK(hipMemcpyAsync(ck + ckoff[k / K] * slot_bytes, b.phi[fw.cur].p, b.slot0[fw.active] * slot_bytes,
-                                        hipMemcpyDeviceToDevice, b.stream));
-        k += fw.launch(k, K);
+    int64_t k = 0;
+    for (int i = 0; i + 1 < nseg; ++i) {
+        for (; k < start[i + 1]; k += fw.launch(k, start[i + 1])) {
+            fw.retire(k);
+            if (k == start[i])
+                GH_HIP_CHECK(hipMemcpyAsync(ck + ckoff[i] * slot_bytes, b.phi[fw.cur].p,
+                                            b.slot0[fw.active] * slot_bytes, hipMemcpyDeviceToDevice, b.stream));
+        }
     }
-    GH_HIP_CHECK(hipGetLastError());
+    fw.retire(k);
+    const int last = nseg - 1;
+    GH_HIP_CHECK(hipMemcpyAsync(b.tape.p, b.phi[fw.cur].p, b.slot0[fw.active] * slot_bytes, hipMemcpyDeviceToDevice,
+                                b.stream));
+    if ((rc = zero_still(last))) return rc;
+    // the final states go where a solve leaves them (the still groups are there)
+    rc = run_on_tape(last, Nmax, [&](int64_t kk) -> int {
+        const int p1 = fw.active;
+        if (kk > start[last]) fw.retire(kk);
+        const int p0 = fw.active;
+        if (p0 == p1) return GH_OK;
+        const Real* from = state(last, kk);
+        Real* to = b.phi[fw.cur].template as<Real>();
+        if (b.skip_still) {
+            const int f0 = p0 ? b.nFull[p0 - 1] : 0, g0 = p0 ? b.nGrp[p0 - 1] : 0;
+            const int nf = b.nFull[p1 - 1] - f0, ng = b.nGrp[p1 - 1] - g0;
+            if (nf + ng > 0)
+                hipLaunchKernelGGL(copy_moving_kernel<Real>, dim3((unsigned)(nf + ng)), dim3(256), 0, b.stream, nf,
+                                   b.fullList.as<int32_t>() + f0, b.grpList.as<int2>() + g0,
+                                   b.stillGrp.as<unsigned char>() + g0, from, to);
+            GH_HIP_CHECK(hipGetLastError());
+        } else {
+            GH_HIP_CHECK(hipMemcpyAsync(to + b.slot0[p0] * BCELLS, from + b.slot0[p0] * BCELLS,
+                                        (b.slot0[p1] - b.slot0[p0]) * slot_bytes, hipMemcpyDeviceToDevice, b.stream));
+        }
+        return GH_OK;
+    });
+    if (rc) return rc;
     b.ran = true;
     // loss at every sample's final state
     std::vector<double> out((size_t)ns * 4);
@@ -699,37 +802,17 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     GH_HIP_CHECK(hipGetLastError());
     // reverse
     GH_HIP_CHECK(hipMemsetAsync(b.apart.p, 0, ADJ_PART * nsl * 8, b.stream));
-    if (b.skip_still) {  // the tape's zeros that no launch writes
-        hipLaunchKernelGGL(still_zero_kernel<Real>, dim3(b.nGrp.back(), K + 1), dim3(256), 0, b.stream, b.nGrp.back(),
-                           b.grpList.as<int2>(), b.stillGrp.as<unsigned char>(), b.tape.as<Real>(), nc);
-        GH_HIP_CHECK(hipGetLastError());
-    }
-    for (int64_t j = J - 1; j >= 0; --j) {
-        const int64_t k0 = j * K, k1 = std::min<int64_t>(Nmax, k0 + K);
-        GH_HIP_CHECK(hipMemcpyAsync(tape, ck + ckoff[j] * slot_bytes, b.slot0[active(k0)] * slot_bytes,
-                                    hipMemcpyDeviceToDevice, b.stream));
-        // recompute u_{k0+1} .. u_{k1} of the running samples, two steps per
-        // launch (both states written) where the input is a clamped state
-        // (k >= 1) and both fit the segment; a sample ending after the first of
-        // the two gets a second state past its end that no reverse step reads
-        for (int64_t k = k0; k < k1;) {
-            char* in = tape + (size_t)(k - k0) * nsl * slot_bytes;
-            if (b.fast_ok && k >= 1) {
-                const bool two = k + 2 <= k1;
-                Real* next = (Real*)(in + (size_t)nsl * slot_bytes);
-                launch_step2f_kernel<Real>(b.stream, b.work(active(k)), b.plain_dom, two, (const Real*)in,
-                                           two ? (Real*)(in + 2 * (size_t)nsl * slot_bytes) : next,
-                                           two ? next : (Real*)nullptr, b.statF.as<Stat4<Real>>(), fprm);
-                k += two ? 2 : 1;
-            } else {
-                step(in, in + (size_t)nsl * slot_bytes, (int)b.slot0[active(k)]);
-                k += 1;
-            }
+    for (int i = last; i >= 0; --i) {
+        const int64_t k0 = start[i], k1 = start[i + 1];
+        if (i < last) {
+            GH_HIP_CHECK(hipMemcpyAsync(b.tape.p, ck + ckoff[i] * slot_bytes, b.slot0[active(k0)] * slot_bytes,
+                                        hipMemcpyDeviceToDevice, b.stream));
+            if ((rc = zero_still(i)) || (rc = run_on_tape(i, k1 - 1, [](int64_t) { return GH_OK; }))) return rc;
         }
         for (int64_t k = k1 - 1; k >= k0; --k) {
             StepWork wk = b.work(active(k));
             if (k == 0) wk.still = nullptr;  // u_0 is the given state
-            const Real* uk = (const Real*)(tape + (size_t)(k - k0) * nsl * slot_bytes);
+            const Real* uk = state(i, k);
             const int mask_out = k >= 1;
             if (b.fast_ok && k >= 1)  // clamped states: the clamped-state records
                 launch_adj_step<true, Real>(b.stream, wk, uk, mask_out, b.lam[(k + 1) & 1].as<double>(),
@@ -742,10 +825,10 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         }
         GH_HIP_CHECK(hipGetLastError());
     }
-    // initial-condition gradient: lambda_0 (buffer 0) against u_0 (checkpoint 0)
+    // initial-condition gradient: lambda_0 (buffer 0) against u_0 (segment 0 came last)
     for (int p = 0; p < ns; ++p) {
         const BatchSample& q = b.smp[b.order[p]];
-        jobs[p].u = (const Real*)(ck) + b.slot0[p] * BCELLS;
+        jobs[p].u = state(0, 0) + b.slot0[p] * BCELLS;
         jobs[p].lam = b.lam[0].as<double>() + b.slot0[p] * BCELLS;
         jobs[p].x0 = q.ic[0];
         jobs[p].y0 = q.ic[1];

@@ -205,8 +205,9 @@ int rd_step1_buffers(Ctx& c, const void* in, void* out, double dt, bool skip_sti
 // marks the groups of blocks without diffusion that the clamped state `in`
 // leaves at zero for good, and writes their zeros into out
 int rd_mark_still(Ctx& c, const void* in, void* out);
-// the marked groups' zeros in n states, one after another from `states` on
-int rd_zero_still(Ctx& c, void* states, int n);
+// the marked groups' zeros in n states, one after another from `states` on, where
+// a block with diffusion reads them
+int rd_zero_still(Ctx& c, void* states, int64_t n);
 // the work list of the current constants
 struct StepWork;
 StepWork rd_step_work(const Ctx& c, bool skip_still);
@@ -244,6 +245,12 @@ int stage_send(int device, hipStream_t stream, void* field, size_t cells, int bp
 // a context (or batch) that may use them is created / destroyed
 void stage_retain();
 void stage_release();
+
+// A tape of a trajectory's states: at least `need` bytes, up to `want` (the whole
+// trajectory) while that stays within an eighth of the device's free memory; what
+// it already holds counts as free.  The states on it need no second solve on the
+// way back, a quarter of a gradient's launches.
+int tape_ensure(DevBuf& tape, size_t need, size_t want);
 
 // likelihood helpers (gh_lik.hip): -logL of the current phi; dJ/du of a state buffer
 int lik_eval_current(Ctx& c, const double* params, int stepPET, int stepTi, int use_roi, double* out,

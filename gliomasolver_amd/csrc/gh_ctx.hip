@@ -40,6 +40,24 @@ void DevBuf::release() {
     bytes = 0;
 }
 
+int tape_ensure(DevBuf& tape, size_t need, size_t want) {
+    if (tape.bytes >= want && tape.p) return GH_OK;
+    size_t room = 0, total = 0;
+    if (hipMemGetInfo(&room, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        room = 0;
+    }
+    const size_t held = tape.p ? tape.bytes : 0;
+    const size_t most = std::min(want, (room + held) / 8);
+    // (a tape short of the whole trajectory is not given up for one little longer)
+    if (held >= need && most < want && most <= held + held / 4) return GH_OK;
+    if (most > need) {
+        if (tape.ensure(most) == GH_OK) return GH_OK;
+        (void)hipGetLastError();
+    }
+    return tape.ensure(need);
+}
+
 int PinnedBuf::ensure_grow(size_t nbytes) {
     if (nbytes <= bytes && p) return GH_OK;
     release();

@@ -272,17 +272,17 @@ int rd_mark_still(Ctx& c, const void* in, void* out) {
                                       : mark_still<double>(c, (const double*)in, (double*)out);
 }
 
-int rd_zero_still(Ctx& c, void* states, int n) {
-    if (c.nGrp == 0 || n <= 0) return GH_OK;
-    const dim3 g((unsigned)c.nGrp, (unsigned)n);
-    if (c.real_kind == GH_REAL_F32)
-        hipLaunchKernelGGL(still_zero_kernel<float>, g, dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
-                           c.stillGrp.as<unsigned char>(), (float*)states, c.ncells());
-    else
-        hipLaunchKernelGGL(still_zero_kernel<double>, g, dim3(256), 0, c.stream, c.nGrp, c.grpList.as<int2>(),
-                           c.stillGrp.as<unsigned char>(), (double*)states, c.ncells());
+template <typename Real>
+static int zero_still(Ctx& c, Real* states, int64_t n) {
+    const int bpd = c.topo.uniform_bpd;
+    const UniformStepParams<Real> prm{0, 0, 0, bpd, bpd_magic(bpd)};  // (its pos)
+    launch_still_zero<Real>(c.stream, c.nGrp, c.grpList, c.stillGrp, c.zeroFlux, prm, states, c.ncells(), n);
     GH_HIP_CHECK(hipGetLastError());
     return GH_OK;
+}
+int rd_zero_still(Ctx& c, void* states, int64_t n) {
+    if (c.nGrp == 0 || n <= 0) return GH_OK;
+    return c.real_kind == GH_REAL_F32 ? zero_still(c, (float*)states, n) : zero_still(c, (double*)states, n);
 }
 
 static int step2f_buffers(Ctx& c, const void* in, void* out, void* mid, double dt, bool two, bool skip_still) {

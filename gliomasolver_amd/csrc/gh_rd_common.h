@@ -747,17 +747,48 @@ __global__ __launch_bounds__(256) void still_kernel(int ngrp, const int2* __rest
     if (!moves)
         for (int c = threadIdx.x; c < v.y * BCELLS; c += 256) out[c0 + c] = (Real)0;
 }
-// the zeros of the still groups in the state buffers out + k * stride, k <
-// gridDim.y (a segment's states, which no later launch writes there)
-template <typename Real>
+// The zeros of the still groups in the n state buffers out + k * stride (a
+// tape's states, which no later launch writes there), in the blocks that a block
+// with diffusion reads: those next to one, by a face, an edge or a corner: a
+// hull of 20 % of 128^3 instead of 62 %, 0.28 us a state at 5.8 TB/s.
+constexpr int STILL_ZERO_STATES = 8;  // per workgroup, which looks at a group's neighbours once
+template <typename Real, typename Params>
 __global__ __launch_bounds__(256) void still_zero_kernel(int ngrp, const int2* __restrict__ grp,
                                                          const unsigned char* __restrict__ still,
-                                                         Real* __restrict__ out, size_t stride) {
+                                                         const unsigned char* __restrict__ zflux, Params prm,
+                                                         Real* __restrict__ out, size_t stride, int n) {
     const int i = blockIdx.x;
     if (i >= ngrp || !still[i]) return;
     const int2 v = grp[i];
-    Real* o = out + (size_t)blockIdx.y * stride + (size_t)v.x * BCELLS;
-    for (int c = threadIdx.x; c < v.y * BCELLS; c += 256) o[c] = (Real)0;
+    __shared__ unsigned s_next;
+    const int t = threadIdx.x;
+    if (t == 0) s_next = 0;
+    __syncthreads();
+    const int blk = t >> 5, k = t & 31;  // neighbour k of block blk (27 of them, itself among them)
+    if (blk < v.y && k < 27) {
+        const BlockPos bp = prm.pos(v.x + blk);
+        if (zflux[bp.nb(k % 3 - 1, k / 3 % 3 - 1, k / 9 - 1)] == 0) atomicOr(&s_next, 1u << blk);
+    }
+    __syncthreads();
+    const unsigned next = s_next;
+    if (next == 0) return;
+    const int k0 = blockIdx.y * STILL_ZERO_STATES, k1 = min(n, k0 + STILL_ZERO_STATES);
+    for (int q = k0; q < k1; ++q)
+        for (int c = t; c < v.y * BCELLS; c += 256)
+            if ((next >> (c / BCELLS)) & 1) out[(size_t)q * stride + (size_t)v.x * BCELLS + c] = (Real)0;
+}
+template <typename Real, typename Params>
+void launch_still_zero(hipStream_t stream, int ngrp, const DevBuf& grp, const DevBuf& still, const DevBuf& zflux,
+                       const Params& prm, Real* out, size_t stride, int64_t n) {
+    static_assert(ZF_GROUP * 32 <= 256, "a lane per neighbour of a group's blocks");
+    constexpr int64_t PART = 32768 * STILL_ZERO_STATES;  // (gridDim.y limit)
+    for (int64_t q = 0; ngrp > 0 && q < n; q += PART) {
+        const int m = (int)std::min(PART, n - q);
+        hipLaunchKernelGGL((still_zero_kernel<Real, Params>),
+                           dim3((unsigned)ngrp, (unsigned)((m + STILL_ZERO_STATES - 1) / STILL_ZERO_STATES)), dim3(256),
+                           0, stream, ngrp, grp.as<int2>(), still.as<unsigned char>(), zflux.as<unsigned char>(), prm,
+                           out + (size_t)q * stride, stride, m);
+    }
 }
 // the work list of slots [0, cut.back()) from their zflux flags; nfull / ngrp (may be
 // null) receive the list lengths after each of the slot counts in cut

@@ -239,8 +239,10 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
 /* ---- adjoint (no reference counterpart: the reference has no derivatives) --
  * gh_rd_adjoint: forward solve of nsteps fused steps with dt = T/nsteps from
  * the current phi (the IC), J = -logL(u_N) as gh_likelihood, then the
- * hand-written discrete adjoint backwards with checkpoint/recompute every
- * ckpt_every steps.  The no-flux flags, the in-domain test and the upper clamp
+ * hand-written discrete adjoint backwards.  The states of the last steps stay on
+ * a tape of at least ckpt_every + 1 states, longer while it fits an eighth of
+ * the device's free memory; earlier ones are recomputed from checkpoints, a
+ * tape's length at a time.  The result does not depend on the length.  The no-flux flags, the in-domain test and the upper clamp
  * are frozen along the trajectory; the lower clamp is treated as inactive.
  * Requires gh_rd_prepare(Dw, Dg = Dw/10, rho) and gh_lik_set_data.  The IC is
  * taken to be a Gaussian of width ic_sigma (cells) centred at ic_center
@@ -304,12 +306,13 @@ int gh_batch_likelihood(gh_batch* b, const double* lik_params, int stepPET, int 
  *   (Gaussian centre in cells)}, nsteps[i] Euler steps of dt = T/N, initial
  *   state ic_peak*exp(-|x-x0|^2/(2 ic_sigma^2)) where p_w + p_g > 0
  *   (gh_gaussian_ic).
- * gh_batch_adjoint: forward with checkpoints every ckpt_every steps, loss,
- *   reverse sweep with recompute, for all samples at once; loss = 4 doubles
+ * gh_batch_adjoint: forward, loss and reverse sweep as gh_rd_adjoint, for all
+ *   samples at once; loss = 4 doubles
  *   and grad = 6 doubles {dJ/dDw, rho, T, x0, y0, z0} per sample, each equal
- *   to gh_rd_adjoint on that sample alone.  Memory: the checkpoints
- *   (sum over samples of ceil(N/K) states), a (K+1)-state tape and two FP64
- *   adjoint states per cell. */
+ *   to gh_rd_adjoint on that sample alone.  Memory: a tape of at
+ *   least ckpt_every + 1 states of all samples, at most every state of every
+ *   sample or an eighth of the free memory; a checkpoint for each tape's length
+ *   before the last; two FP64 adjoint states per cell. */
 int gh_batch_set_adjoint_samples(gh_batch* b, int nsamples, const int* anatomy_id, const double* params,
                                  const int64_t* nsteps, double ic_sigma, double ic_peak);
 int gh_batch_adjoint(gh_batch* b, int ckpt_every, const double* lik_params, int stepPET, int stepTi, int use_roi,
