@@ -242,8 +242,9 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
  * hand-written discrete adjoint backwards.  The states of the last steps stay on
  * a tape of at least ckpt_every + 1 states, longer while it fits an eighth of
  * the device's free memory; earlier ones are recomputed from checkpoints, a
- * tape's length at a time.  The result does not depend on the length.  The no-flux flags, the in-domain test and the upper clamp
- * are frozen along the trajectory; the lower clamp is treated as inactive.
+ * tape's length at a time.  The result does not depend on the length.  The
+ * no-flux flags, the in-domain test and the upper clamp are frozen along the
+ * trajectory; the lower clamp is treated as inactive.
  * Requires gh_rd_prepare(Dw, Dg = Dw/10, rho) and gh_lik_set_data.  The IC is
  * taken to be a Gaussian of width ic_sigma (cells) centred at ic_center
  * (cells), so dJ/dx0 = sum lambda_0 u_0 (i - x0)/sigma^2.
