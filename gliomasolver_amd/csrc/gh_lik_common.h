@@ -68,7 +68,8 @@ __device__ inline uint32_t pet_row(const LikParams& p, int base) {
 }
 
 // Cells of a wave whose Bernoulli term is one of four constants: u lost in u - uc
-// (in front of a tumour) or u above the threshold, with either label.
+// (in front of a tumour) or u above the threshold, with either label.  The constants
+// come from the function that makes the other terms, once per workgroup.
 struct BernoulliCount {
     int front = 0, front1 = 0, above = 0, above1 = 0;
     // counts the wave's cells and returns the others, whose terms take an exp and a
@@ -82,16 +83,6 @@ struct BernoulliCount {
         front += __popcll(f);
         front1 += __popcll(f & one);
         return all & ~(a | f);
-    }
-    // their terms' sum, in lane 0 of the wave; the terms come from the function
-    // that makes the rest
-    __device__ inline double sum(double uc, double is2) const {
-        const int l = threadIdx.x & 63;
-        const double v = log_bernoulli((l & 2) ? 1. : 0. - uc, l & 1, is2);
-        const int n = l == 0 ? front - front1 : l == 1 ? front1 : l == 2 ? above - above1 : above1;
-        const double s = n ? (double)n * v : 0.;  // (a label that no cell has may have no finite term)
-        const double t = (wave_get(s, 0) + wave_get(s, 1)) + (wave_get(s, 2) + wave_get(s, 3));
-        return l == 0 ? t : 0.;
     }
 };
 
@@ -175,8 +166,8 @@ __device__ inline void lik_cells(int wg, size_t base, size_t ncells, const Layou
 // counted by ballots on the scalar side, the others' terms are formed where a wave
 // has any, and a lane has four cells' loads in flight (eight do not help one state
 // and cost 24 samples of 96^3 a quarter: lanes without a cell).  128^3 FP32, PET on
-// every third cell, a quarter of the cells on the tumour's flank: 28 -> 17.5 us,
-// of which 11 remain without those; 24 samples of 96^3 230 -> 164 us.
+// every third cell, a quarter of the cells on the tumour's flank: 28 -> 15.8 us;
+// 24 samples of 96^3 230 -> 164 us.
 template <typename T>
 __device__ inline void lik_partials_body(int wg, size_t ncells, const Layout& lay, const T* __restrict__ u,
                                          const unsigned char* __restrict__ t1, const unsigned char* __restrict__ fl,
@@ -203,22 +194,34 @@ __device__ inline void lik_partials_body(int wg, size_t ncells, const Layout& la
             }
         }
     }
-    if (bern) {
-        l1 += b1.sum(p.uc1, p.is2);
-        l2 += b2.sum(p.uc2, p.is2);
-    }
     __shared__ double red[4][LIK_THREADS / 64];
+    __shared__ int cnt[LIK_THREADS / 64][8];
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
     const double a = wave_sum2(sse, npet), b = wave_sum2(l1, l2);
     if ((lane & 31) == 0) {
         red[lane >> 5][w] = a;
         red[2 + (lane >> 5)][w] = b;
     }
+    if (lane == 0) {
+        const int n[8] = {b1.front - b1.front1, b1.front1, b1.above - b1.above1, b1.above1,
+                          b2.front - b2.front1, b2.front1, b2.above - b2.above1, b2.above1};
+        for (int i = 0; i < 8; ++i) cnt[w][i] = n[i];
+    }
     __syncthreads();
-    if (threadIdx.x < 4) {
-        double s = 0;
-        for (int k = 0; k < LIK_THREADS / 64; ++k) s += red[threadIdx.x][k];
-        partials[threadIdx.x * LIK_GRID + wg] = s;
+    if (w != 0) return;
+    // lane l < 8: the counted terms of threshold l / 4, above it l & 2, label l & 1
+    const int l = lane & 7;
+    int n = 0;
+    for (int k = 0; k < LIK_THREADS / 64; ++k) n += cnt[k][l];
+    double v = log_bernoulli((l & 2) ? 1. : 0. - ((l & 4) ? p.uc2 : p.uc1), l & 1, p.is2);
+    v = n ? (double)n * v : 0.;  // (a label that no cell has may have no finite term)
+    v += __shfl_xor(v, 1, 64);
+    v += __shfl_xor(v, 2, 64);  // lanes 0..3: the sum of threshold 0, 4..7: of threshold 1
+    const double c1 = wave_get(v, 0), c2 = wave_get(v, 4);
+    if (lane < 4) {
+        double s = lane < 2 ? 0. : (lane == 2 ? c1 : c2);
+        for (int k = 0; k < LIK_THREADS / 64; ++k) s += red[lane][k];
+        partials[lane * LIK_GRID + wg] = s;
     }
 }
 
