@@ -51,7 +51,7 @@ struct AdjArgs {
     double rho, ih2, dt, invN, invDw;
     int bpd;
     uint32_t magic;
-    const int32_t* slot_pos;
+    const int4* slots;
     const void* range;
 };
 
@@ -61,10 +61,14 @@ struct UniformAdjParams {
     int bpd;
     uint32_t magic;  // bpd_magic(bpd)
     __host__ __device__ static inline UniformAdjParams make(double r, double i, double d, double n, double w, int b,
-                                                            uint32_t m, const int32_t*, const void*) {
+                                                            uint32_t m, const int4*, const void*) {
         return {r, i, d, n, w, b, m};
     }
     AdjArgs args() const { return {rho, ih2, dt, invN, invDw, bpd, magic, nullptr, nullptr}; }
+    using Item = int;
+    __device__ static inline Item item(const int32_t* full, int i) { return full ? full[i] : i; }
+    __device__ static inline Item item_of(int s) { return s; }
+    __device__ static inline int slot(Item it) { return it; }
     __device__ inline void get(int, double& r, double& i, double& d, double& n, double& w) const {
         r = rho;
         i = ih2;
@@ -192,18 +196,19 @@ __global__ __launch_bounds__(256) void adj_mask_kernel(size_t n, double* __restr
 template <typename Real, typename Params, bool CLAMPED = false>
 __global__ __launch_bounds__(512) void adj_step_kernel(
     int nfull, int fper, const int32_t* __restrict__ full, const Real* __restrict__ uk,
-    const Stat4<Real>* __restrict__ st, int bpd, uint32_t magic, const int32_t* __restrict__ slot_pos,
+    const Stat4<Real>* __restrict__ st, int bpd, uint32_t magic, const int4* __restrict__ slots,
     const void* __restrict__ range, const double* __restrict__ lam1, double* __restrict__ lam0,
     const Real* __restrict__ sig, double* __restrict__ partial, int mask_out, double rho_, double ih2_, double dt_,
     double invN_, double invDw_, int ngrp, int gper, const int2* __restrict__ grp,
     const unsigned char* __restrict__ still) {
     const StepWork wk{nfull, fper, ngrp, gper, full, grp, still};
-    const Params prm = Params::make(rho_, ih2_, dt_, invN_, invDw_, bpd, magic, slot_pos, range);
+    const Params prm = Params::make(rho_, ih2_, dt_, invN_, invDw_, bpd, magic, slots, range);
     int nzf;
-    const int s = wk.item(&nzf);
+    typename Params::Item it;
+    const int s = wk.item(prm, &nzf, it);
     if (s < 0) return;
     double rho, ih2, dt, invN, invDw;
-    prm.get(s, rho, ih2, dt, invN, invDw);  // a group's blocks belong to one solve
+    prm.get(it, rho, ih2, dt, invN, invDw);  // a group's blocks belong to one solve
     const int t = threadIdx.x;
     for (int b = 0; b < nzf; ++b) {  // uniform per workgroup
         const size_t g = (size_t)(s + b) * BCELLS + t;
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(512) void adj_step_kernel(
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const size_t base = (size_t)s * BCELLS;
     const unsigned ut = (unsigned)t;
-    const BlockPos bp = prm.pos(s);
+    const BlockPos bp = prm.pos(it);
     // halo roles: waves 0-5 the depth-1 cells of face wv (state, flags, w,
     // minus-face D), waves 6, 7 and 0-3 the depth-2 cells of faces 0-5 (state,
     // flags)
@@ -333,7 +338,7 @@ inline void launch_adj_step(hipStream_t stream, const StepWork& wk, const Real* 
                             double* lam0, const Stat4<Real>* st, const Real* sig, const Params& prm, double* partial) {
     const AdjArgs q = prm.args();
     hipLaunchKernelGGL((adj_step_kernel<Real, Params, CLAMPED>), dim3(wk.grid()), dim3(512), 0, stream, wk.nfull,
-                       wk.fper, wk.full, uk, st, q.bpd, q.magic, q.slot_pos, q.range, lam1, lam0, sig, partial,
+                       wk.fper, wk.full, uk, st, q.bpd, q.magic, q.slots, q.range, lam1, lam0, sig, partial,
                        mask_out, q.rho, q.ih2, q.dt, q.invN, q.invDw, wk.ngrp, wk.gper, wk.grp, wk.still);
 }
 

@@ -68,25 +68,20 @@ struct BatchSample {
 };
 
 template <typename Real>
-struct BatchAdjParams {
-    const int32_t* __restrict__ slot_pos;
+struct BatchAdjParams : PackedItems {
     const SlotRange<Real>* __restrict__ range;
     __host__ __device__ static inline BatchAdjParams make(double, double, double, double, double, int, uint32_t,
-                                                          const int32_t* sp, const void* r) {
-        return {sp, (const SlotRange<Real>*)r};
+                                                          const int4* sl, const void* r) {
+        return {{sl}, (const SlotRange<Real>*)r};
     }
-    AdjArgs args() const { return {0., 0., 0., 0., 0., 0, 0u, slot_pos, range}; }
-    __device__ inline void get(int s, double& r, double& i, double& d, double& n, double& w) const {
-        const SlotRange<Real>& q = range[slot_pos[s]];
+    AdjArgs args() const { return {0., 0., 0., 0., 0., 0, 0u, slots, range}; }
+    __device__ inline void get(const Item& it, double& r, double& i, double& d, double& n, double& w) const {
+        const SlotRange<Real>& q = range[it.w];
         r = q.rho_d;
         i = q.ih2;
         d = q.dt;
         n = q.invN;
         w = q.invDw;
-    }
-    __device__ inline BlockPos pos(int s) const {
-        const SlotRange<Real>& q = range[slot_pos[s]];
-        return block_pos(s, (int)q.slot0, q.bpd, q.magic);
     }
 };
 
@@ -133,26 +128,35 @@ __global__ __launch_bounds__(256) void batch_ic_partials(const AdjJob<Real>* __r
 }
 
 template <typename Real>
-struct BatchStepParams {
-    const int32_t* __restrict__ slot_pos;
+struct BatchStepParams : PackedItems {
     const SlotRange<Real>* __restrict__ range;
     static constexpr bool kPow2 = false;  // any number of blocks per side
-    __host__ __device__ static inline BatchStepParams make(Real, double, double, int, uint32_t, const int32_t* sp,
+    __host__ __device__ static inline BatchStepParams make(Real, double, double, int, uint32_t, const int4* sl,
                                                            const void* r) {
-        return {sp, (const SlotRange<Real>*)r};
+        return {{sl}, (const SlotRange<Real>*)r};
     }
-    StepArgs<Real> args() const { return {(Real)0, 0., 0., 0, 0u, slot_pos, range}; }
-    __device__ inline void get(int s, Real& r, double& i, double& d) const {
-        const SlotRange<Real>& q = range[slot_pos[s]];
+    StepArgs<Real> args() const { return {(Real)0, 0., 0., 0, 0u, slots, range}; }
+    __device__ inline void get(const Item& it, Real& r, double& i, double& d) const {
+        const SlotRange<Real>& q = range[it.w];
         r = q.rho;
         i = q.ih2;
         d = q.dt;
     }
-    __device__ inline BlockPos pos(int s) const {
-        const SlotRange<Real>& q = range[slot_pos[s]];
-        return block_pos(s, (int)q.slot0, q.bpd, q.magic);
-    }
+    __device__ inline void get(int s, Real& r, double& i, double& d) const { get(slots[s], r, i, d); }
 };
+// the items (PackedItems) of the slots full[0 .. n), or of slots 0 .. n without a list
+template <typename Real>
+__global__ __launch_bounds__(256) void items_kernel(int n, const int32_t* __restrict__ full,
+                                                    const int32_t* __restrict__ slot_pos,
+                                                    const SlotRange<Real>* __restrict__ range,
+                                                    int4* __restrict__ items) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int s = full ? full[i] : i, p = slot_pos[s];
+    const SlotRange<Real>& q = range[p];
+    const BlockPos b = block_pos(s, (int)q.slot0, q.bpd, q.magic);
+    items[i] = make_int4(s, b.slot0, b.bpd | b.bx << 8 | b.by << 16 | b.bz << 24, p);
+}
 
 // constants_kernel's source: the anatomy, Dw and Dg of the slot's sample
 template <typename Real>
@@ -235,13 +239,14 @@ struct Batch {
     DevBuf zeroFlux;                 // per slot: != 0 a block without diffusion (constants_kernel)
     // StepWork lists of all slots and their lengths per count of positions (index p: positions 0..p)
     DevBuf fullList, grpList, stillGrp;
+    DevBuf slotItem, fullItem;  // PackedItems of every slot, of fullList's
     std::vector<int> nFull, nGrp;
     bool skip_still = false;  // stillGrp holds the marks of the current states
     // the work of the slots of positions [0, active)
     StepWork work(int active) const {
         const int p = active - 1;
         if (nGrp.empty() || nGrp.back() == 0) return step_work((int)slot0[active], nullptr, 0, nullptr, nullptr);
-        return step_work(nFull[p], fullList.as<int32_t>(), nGrp[p], grpList.as<int2>(),
+        return step_work(nFull[p], fullItem.as<int32_t>(), nGrp[p], grpList.as<int2>(),
                          skip_still ? stillGrp.as<unsigned char>() : nullptr);
     }
     DevBuf ck, tape, lam[2], apart, icpart, adjJobs;  // adjoint
@@ -341,6 +346,11 @@ int build_layout_t(Batch& b) {
     b.skip_still = false;
     std::vector<unsigned char> z(nsl);
     if (nsl > 0) {
+        if ((rc = b.slotItem.ensure_grow(nsl * sizeof(int4)))) return rc;
+        hipLaunchKernelGGL(items_kernel<Real>, dim3((unsigned)((nsl + 255) / 256)), dim3(256), 0, b.stream, (int)nsl,
+                           (const int32_t*)nullptr, b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>(),
+                           b.slotItem.as<int4>());
+        GH_HIP_CHECK(hipGetLastError());
         const BatchAnatomySrc<Real> src{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>(),
                                         b.apw.as<const Real* const>(), b.apg.as<const Real* const>()};
         hipLaunchKernelGGL((constants_kernel<Real, BatchAnatomySrc<Real>>), dim3((unsigned)nsl), dim3(512), 0,
@@ -369,6 +379,12 @@ int build_layout_t(Batch& b) {
                                             hipMemcpyHostToDevice, b.stream));
             GH_HIP_CHECK(hipMemcpyAsync(b.grpList.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice,
                                         b.stream));
+            if ((rc = b.fullItem.ensure_grow(std::max<size_t>(1, full.size()) * sizeof(int4)))) return rc;
+            if (!full.empty())
+                hipLaunchKernelGGL(items_kernel<Real>, dim3((unsigned)((full.size() + 255) / 256)), dim3(256), 0,
+                                   b.stream, (int)full.size(), b.fullList.as<int32_t>(), b.slotPos.as<int32_t>(),
+                                   b.range.as<SlotRange<Real>>(), b.fullItem.as<int4>());
+            GH_HIP_CHECK(hipGetLastError());
             GH_HIP_CHECK(hipStreamSynchronize(b.stream));  // the lists are read by the copies
         }
     }
@@ -516,7 +532,7 @@ struct ForwardSweep {
     BatchStepParams<Real> prm;
     int cur = 0, active = 0;
     explicit ForwardSweep(Batch& bb)
-        : b(bb), prm{bb.slotPos.as<int32_t>(), bb.range.as<SlotRange<Real>>()} {
+        : b(bb), prm{{bb.slotItem.as<int4>()}, bb.range.as<SlotRange<Real>>()} {
         const int ns = (int)b.smp.size();
         npos.resize(ns);
         for (int p = 0; p < ns; ++p) npos[p] = b.smp[b.order[p]].nsteps;
@@ -681,8 +697,8 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
         (rc = b.icpart.ensure((size_t)ns * 3 * IC_GRID * 8)) || (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
-    const BatchStepParams<Real> fprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
-    const BatchAdjParams<Real> aprm{b.slotPos.as<int32_t>(), b.range.as<SlotRange<Real>>()};
+    const BatchStepParams<Real> fprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
+    const BatchAdjParams<Real> aprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     char* ck = (char*)b.ck.p;
     auto state = [&](int seg, int64_t k) {
         return (Real*)((char*)b.tape.p + (cum(k) - cum(start[seg])) * slot_bytes);
@@ -903,7 +919,7 @@ int gh_batch_destroy(gh_batch* bh) {
         a->pet.release();
         a->roi.release();
     }
-    DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->slotPos, &b->range,
+    DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->slotPos, &b->slotItem, &b->fullItem, &b->range,
                       &b->apw,    &b->apg,    &b->likPart, &b->likOut, &b->likJobs, &b->ck,     &b->tape,
                       &b->lam[0], &b->lam[1], &b->apart,   &b->icpart, &b->adjJobs, &b->statF,  &b->flag,
                       &b->zeroFlux, &b->fullList, &b->grpList, &b->stillGrp};

@@ -259,7 +259,7 @@ struct StepArgs {
     double ih2, dt;
     int bpd;
     uint32_t magic;
-    const int32_t* slot_pos;  // packed solves: the solve of a slot and its SlotRange
+    const int4* slots;  // packed solves: where a slot lies, and its solve's SlotRange
     const void* range;
 };
 
@@ -273,16 +273,38 @@ struct UniformStepParams {
     uint32_t magic;  // bpd_magic(bpd)
     static constexpr bool kPow2 = true;  // h = 2^-level / 8
     __host__ __device__ static inline UniformStepParams make(Real r, double i, double d, int b, uint32_t m,
-                                                             const int32_t*, const void*) {
+                                                             const int4*, const void*) {
         return {r, i, d, b, m};
     }
     StepArgs<Real> args() const { return {rho, ih2, dt, bpd, magic, nullptr, nullptr}; }
+    // what a work list's entry, or a slot alone, tells of a block
+    using Item = int;
+    __device__ static inline Item item(const int32_t* full, int i) { return full ? full[i] : i; }
+    __device__ static inline Item item_of(int s) { return s; }
+    __device__ static inline int slot(Item it) { return it; }
     __device__ inline void get(int, Real& r, double& i, double& d) const {
         r = rho;
         i = ih2;
         d = dt;
     }
     __device__ inline BlockPos pos(int s) const { return block_pos(s, 0, bpd, magic); }
+};
+// Packed solves: {slot, the solve's first slot, blocks per side | x << 8 | y << 16 |
+// z << 24, the solve}, 16 B in one scalar load.  (The slot, its solve, the solve's
+// first slot and a division were three loads in a row before a workgroup's first
+// load of a cell: 24 samples of 96^3, a pair of steps 21.1 -> 20.5 us.)
+struct PackedItems {
+    using Item = int4;
+    const int4* __restrict__ slots;
+    __device__ inline Item item(const int32_t* full, int i) const {
+        return (full ? reinterpret_cast<const int4*>(full) : slots)[i];
+    }
+    __device__ inline Item item_of(int s) const { return slots[s]; }
+    __device__ static inline int slot(const Item& it) { return it.x; }
+    __device__ static inline BlockPos pos(const Item& it) {
+        return BlockPos{it.y, it.z & 0xff, (it.z >> 8) & 0xff, (it.z >> 16) & 0xff, (it.z >> 24) & 0xff};
+    }
+    __device__ inline BlockPos pos(int s) const { return pos(slots[s]); }
 };
 
 // Two fused Euler steps per launch (temporal blocking): one workgroup per 8^3
@@ -591,8 +613,8 @@ __device__ inline Real rd_rhs_reaction_only(Real pc, bool dom, Real rho) {
 }
 
 // Work list of the two-step and the reverse-step kernels.  Blocks with
-// diffusion are one item each (full: their slots, ascending; null: item i is
-// slot i), runs of up to ZF_GROUP consecutive blocks without diffusion one item
+// diffusion are one item each (full: their items, ascending -- slots, or the
+// int4 of packed solves; null: item i is slot i), runs of up to ZF_GROUP consecutive blocks without diffusion one item
 // of grp {slot, blocks}.  Workgroup w runs on XCD w % 8 and takes item w / 8 of
 // that XCD's contiguous share of full (fper items) -- neighbours' halos stay in
 // one L2 -- and after these its share of grp (gper), which fill the tail.
@@ -602,20 +624,23 @@ struct StepWork {
     const int32_t* __restrict__ full;
     const int2* __restrict__ grp;
     const unsigned char* __restrict__ still;
-    // this workgroup's item: its first slot, *nzf = 0 for a block with
+    // this workgroup's item and its first slot, *nzf = 0 for a block with
     // diffusion, else the blocks without diffusion; -1: nothing to do
-    __device__ inline int item(int* nzf) const {
+    template <typename Params>
+    __device__ inline int item(const Params& prm, int* nzf, typename Params::Item& it) const {
         const int x = (int)(blockIdx.x % 8), j = (int)(blockIdx.x / 8);
         *nzf = 0;
         if (j < fper) {
             const int i = x * fper + j;
             if (i >= nfull) return -1;
-            return full ? full[i] : i;
+            it = prm.item(full, i);
+            return prm.slot(it);
         }
         const int i = x * gper + j - fper;
         if (i >= ngrp || (still && still[i])) return -1;
         const int2 v = grp[i];
         *nzf = v.y;
+        it = prm.item_of(v.x);
         return v.x;
     }
     unsigned grid() const { return 8u * (unsigned)(fper + gper); }
@@ -841,14 +866,15 @@ __device__ inline int mad24(int a, int b, int c) { return (int)__umul24((unsigne
 template <typename Real, typename Params, bool DOM, bool TWO>
 __global__ __launch_bounds__(512) void rd_step2f_kernel(
     int nfull, int fper, const int32_t* __restrict__ full, const Real* __restrict__ phi,
-    const Stat4<Real>* __restrict__ stf, int bpd, uint32_t magic, const int32_t* __restrict__ slot_pos,
+    const Stat4<Real>* __restrict__ stf, int bpd, uint32_t magic, const int4* __restrict__ slots,
     const void* __restrict__ range, Real* __restrict__ out, Real* __restrict__ mid, Real rho_, double ih2_, double dt_,
     int ngrp, int gper, const int2* __restrict__ grp, const unsigned char* __restrict__ still) {
     const StepWork wk{nfull, fper, ngrp, gper, full, grp, still};
-    const Params prm = Params::make(rho_, ih2_, dt_, bpd, magic, slot_pos, range);
+    const Params prm = Params::make(rho_, ih2_, dt_, bpd, magic, slots, range);
     constexpr bool POW2 = Params::kPow2;
     int nzf;
-    const int s = wk.item(&nzf);
+    typename Params::Item it;
+    const int s = wk.item(prm, &nzf, it);
     if (s < 0) return;
     __shared__ Real s_uu[UU_SIZE];
     __shared__ Real s_dmx[1000], s_dmy[1000], s_dmz[1000];
@@ -857,7 +883,7 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(
     const size_t base = (size_t)s * BCELLS;
     Real rho;
     double ih2, dt;
-    prm.get(s, rho, ih2, dt);  // a group's blocks belong to one solve
+    prm.get(it, rho, ih2, dt);  // a group's blocks belong to one solve
     if (nzf > 0) {             // uniform per workgroup
         for (int i = t; i < nzf * BCELLS; i += 512) {
             const size_t bc = base + (unsigned)i;
@@ -871,7 +897,7 @@ __global__ __launch_bounds__(512) void rd_step2f_kernel(
     }
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // wave = interior plane z; halo role
     const int a = t & 7, b = (t >> 3) & 7;
-    const BlockPos bp = prm.pos(s);
+    const BlockPos bp = prm.pos(it);
     const unsigned ut = (unsigned)t;
 
     // ---- loads: (waves 0-5) the depth-1 and depth-2 cells of face w, (waves
@@ -987,7 +1013,7 @@ inline void launch_step2f_kernel(hipStream_t stream, const StepWork& wk, bool pl
     const auto q = prm.args();
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(wk.grid()), dim3(512), 0, stream, wk.nfull, wk.fper, wk.full, in, stf, q.bpd,
-                           q.magic, q.slot_pos, q.range, out, mid, q.rho, q.ih2, q.dt, wk.ngrp, wk.gper, wk.grp,
+                           q.magic, q.slots, q.range, out, mid, q.rho, q.ih2, q.dt, wk.ngrp, wk.gper, wk.grp,
                            wk.still);
     };
     if (two) {
