@@ -148,7 +148,7 @@ struct Ctx {
     bool plain_dom = false;  // no cell has p_w = -p_g != 0: rd_step2f_kernel needs no domain test
     DevBuf zeroFlux;       // per slot: != 0 a block without diffusion (constants_kernel), uniform grids
     int nZeroFlux = 0;     // blocks without diffusion
-    // work list of the two-step and reverse-step kernels (StepWork, plan_step2f):
+    // work list of the two-step and reverse-step kernels (StepWork):
     // slots of the blocks with diffusion, groups of blocks without (nGrp = 0:
     // every slot an item), and per group whether a solve leaves it at zero
     DevBuf fullList, grpList, stillGrp;
