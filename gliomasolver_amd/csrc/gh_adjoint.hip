@@ -36,6 +36,11 @@
 namespace gh {
 namespace {
 
+__global__ __launch_bounds__(512) void adj_reduce_kernel(const double* __restrict__ part, size_t n,
+                                                         const double* __restrict__ ic, double* __restrict__ out) {
+    adj_reduce_body(part, n, ic, out);
+}
+
 template <typename Real>
 int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET, int stepTi, int use_roi,
               const double* ic, double sigma, double* loss, double* grad) {
@@ -148,22 +153,19 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
         }
     }
     // initial-condition gradient from lambda_0 and u_0
-    const unsigned igrid = 512;
-    if ((rc = c.likPart.ensure(sizeof(double) * 4 * 1025))) return rc;
-    hipLaunchKernelGGL(adj_ic_partials<Real>, dim3(igrid), dim3(256), 0, c.stream, nc, c.topo.uniform_bpd,
+    if ((rc = c.likPart.ensure(sizeof(double) * 4 * 1025)) || (rc = c.pinLik.ensure_grow(ADJ_SUMS * sizeof(double))))
+        return rc;
+    hipLaunchKernelGGL(adj_ic_partials<Real>, dim3(ADJ_IC_GRID), dim3(256), 0, c.stream, nc, c.topo.uniform_bpd,
                        c.adjLam[lc].as<double>(), (const Real*)seg, ic[0], ic[1], ic[2], 1.0 / (sigma * sigma),
                        c.likPart.as<double>());
     GH_HIP_CHECK(hipGetLastError());
-    std::vector<double> pp(ADJ_PART * (size_t)ns), ip(3 * igrid);
-    GH_HIP_CHECK(hipMemcpyAsync(pp.data(), c.adjPart.p, pp.size() * 8, hipMemcpyDeviceToHost, c.stream));
-    GH_HIP_CHECK(hipMemcpyAsync(ip.data(), c.likPart.p, ip.size() * 8, hipMemcpyDeviceToHost, c.stream));
+    double* const sums = c.pinLik.as<double>();
+    hipLaunchKernelGGL(adj_reduce_kernel, dim3(1), dim3(512), 0, c.stream, c.adjPart.as<double>(), (size_t)ns,
+                       c.likPart.as<double>(), sums);
+    GH_HIP_CHECK(hipGetLastError());
     GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    for (int q = 0; q < 6; ++q) grad[q] = 0;
-    double ab[2];
-    sum_slot_partials(pp.data(), ns, ab);
-    adj_param_grads(ab, prm.dt, prm.invDw, prm.invN, prm.rho, grad);
-    for (unsigned w = 0; w < igrid; ++w)
-        for (int q = 0; q < 3; ++q) grad[3 + q] += ip[3 * w + q];
+    adj_param_grads(sums, prm.dt, prm.invDw, prm.invN, prm.rho, grad);
+    for (int q = 0; q < 3; ++q) grad[3 + q] = sums[2 + q];
     return GH_OK;
 }
 

@@ -372,16 +372,38 @@ __global__ __launch_bounds__(256) void adj_ic_partials(size_t nc, int bpd, const
     adj_ic_body<Real>((int)blockIdx.x, (int)gridDim.x, nc, bpd, lam, u0, x0, y0, z0, is2, partial);
 }
 
-// The host's summation of the per-wave partials: workgroup order g = 0..8*per_xcd-1
-// of the step kernel's grid, slot = (g % 8) * per_xcd + g / 8, then wave order.
-inline void sum_slot_partials(const double* part, int nslots, double ab[2]) {
-    const int per_xcd = (nslots + 7) / 8;
-    ab[0] = ab[1] = 0;
-    for (int g = 0; g < 8 * per_xcd; ++g) {
-        const int s = (g % 8) * per_xcd + g / 8;
-        if (s >= nslots) continue;
-        for (int w = 0; w < 8; ++w)
-            for (int q = 0; q < 2; ++q) ab[q] += part[ADJ_PART * (size_t)s + 2 * w + q];
+// A solve's sums A, B over its n slots and the three initial-condition sums over
+// ADJ_IC_GRID partials, by one workgroup of 512 lanes in a fixed order.  (The
+// partials of twelve mixed samples were 3 MB copied to pageable memory and added
+// one after another on the host: 0.4 of 20.7 ms; of 64^3 FP64 0.1 of 2.7 ms.)
+constexpr int ADJ_IC_GRID = 512;
+constexpr int ADJ_SUMS = 5;
+__device__ inline void adj_reduce_body(const double* __restrict__ part, size_t n, const double* __restrict__ ic,
+                                       double* __restrict__ out) {
+    static_assert(ADJ_PART % 2 == 0 && ADJ_IC_GRID == 512, "even words are A's, odd ones B's; a lane per partial");
+    __shared__ double red[ADJ_SUMS][8];
+    const int t = threadIdx.x;
+    double a[4] = {0, 0, 0, 0};
+    const size_t m = n * ADJ_PART;  // a multiple of 16
+    size_t i = t;
+    for (; i + 3 * 512 < m; i += 4 * 512)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] += part[i + 512 * k];
+    for (int k = 0; i < m; i += 512, ++k) a[k] += part[i];
+    double v = (a[0] + a[1]) + (a[2] + a[3]), g[3];
+    for (int q = 0; q < 3; ++q) g[q] = ic[3 * t + q];
+    for (int o = 32; o > 1; o >>= 1) v += __shfl_xor(v, o, 64);  // lane 0: A's, lane 1: B's
+    for (int o = 32; o > 0; o >>= 1)
+        for (int q = 0; q < 3; ++q) g[q] += __shfl_xor(g[q], o, 64);
+    const int w = t >> 6, lane = t & 63;
+    if (lane < 2) red[lane][w] = v;
+    if (lane == 0)
+        for (int q = 0; q < 3; ++q) red[2 + q][w] = g[q];
+    __syncthreads();
+    if (t < ADJ_SUMS) {
+        double s = 0;
+        for (int k = 0; k < 8; ++k) s += red[t][k];
+        out[t] = s;
     }
 }
 

@@ -127,6 +127,17 @@ __global__ __launch_bounds__(256) void batch_ic_partials(const AdjJob<Real>* __r
                       partial + (size_t)blockIdx.y * 3 * gridDim.x);
 }
 
+// a sample's sums (adj_reduce_body), a workgroup each
+template <typename Real>
+__global__ __launch_bounds__(512) void batch_reduce_kernel(const double* __restrict__ part,
+                                                           const AdjJob<Real>* __restrict__ jobs,
+                                                           const SlotRange<Real>* __restrict__ range,
+                                                           const double* __restrict__ ic, double* __restrict__ out) {
+    const size_t p = blockIdx.x;
+    adj_reduce_body(part + ADJ_PART * range[p].slot0, jobs[p].ncells / BCELLS, ic + p * 3 * ADJ_IC_GRID,
+                    out + p * ADJ_SUMS);
+}
+
 template <typename Real>
 struct BatchStepParams : PackedItems {
     const SlotRange<Real>* __restrict__ range;
@@ -673,7 +684,6 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         const int p = active(k - 1);
         return b.slot0[p] * (size_t)k + ended[p];
     };
-    constexpr int IC_GRID = 512;
     int rc;
     if ((rc = tape_ensure(b.tape, (size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes,
                           cum(Nmax + 1) * slot_bytes)))
@@ -695,7 +705,7 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
     if ((rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes)) || (rc = b.lam[0].ensure(nc * 8)) ||
         (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
-        (rc = b.icpart.ensure((size_t)ns * 3 * IC_GRID * 8)) || (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
+        (rc = b.icpart.ensure((size_t)ns * (3 * ADJ_IC_GRID + ADJ_SUMS) * 8)) || (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
     const BatchStepParams<Real> fprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
@@ -853,13 +863,16 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     }
     GH_HIP_CHECK(hipMemcpyAsync(b.adjJobs.p, jobs.data(), ns * sizeof(AdjJob<Real>), hipMemcpyHostToDevice, b.stream));
     for (int p0 = 0; p0 < ns; p0 += 65535)
-        hipLaunchKernelGGL(batch_ic_partials<Real>, dim3(IC_GRID, std::min(65535, ns - p0)), dim3(256), 0, b.stream,
-                           b.adjJobs.as<AdjJob<Real>>() + p0, b.icpart.as<double>() + (size_t)p0 * 3 * IC_GRID);
+        hipLaunchKernelGGL(batch_ic_partials<Real>, dim3(ADJ_IC_GRID, std::min(65535, ns - p0)), dim3(256), 0, b.stream,
+                           b.adjJobs.as<AdjJob<Real>>() + p0, b.icpart.as<double>() + (size_t)p0 * 3 * ADJ_IC_GRID);
+    GH_HIP_CHECK(hipGetLastError());
+    double* const dsums = b.icpart.as<double>() + (size_t)ns * 3 * ADJ_IC_GRID;
+    hipLaunchKernelGGL(batch_reduce_kernel<Real>, dim3((unsigned)ns), dim3(512), 0, b.stream, b.apart.as<double>(),
+                       b.adjJobs.as<AdjJob<Real>>(), b.range.as<SlotRange<Real>>(), b.icpart.as<double>(), dsums);
     GH_HIP_CHECK(hipGetLastError());
     GH_HIP_CHECK(hipEventRecord(b.ev1, b.stream));
-    std::vector<double> ap(ADJ_PART * nsl), ip((size_t)ns * 3 * IC_GRID);
-    GH_HIP_CHECK(hipMemcpyAsync(ap.data(), b.apart.p, ap.size() * 8, hipMemcpyDeviceToHost, b.stream));
-    GH_HIP_CHECK(hipMemcpyAsync(ip.data(), b.icpart.p, ip.size() * 8, hipMemcpyDeviceToHost, b.stream));
+    std::vector<double> sums((size_t)ns * ADJ_SUMS);
+    GH_HIP_CHECK(hipMemcpyAsync(sums.data(), dsums, sums.size() * 8, hipMemcpyDeviceToHost, b.stream));
     GH_HIP_CHECK(hipStreamSynchronize(b.stream));
     float ms = 0;
     GH_HIP_CHECK(hipEventElapsedTime(&ms, b.ev0, b.ev1));
@@ -868,12 +881,9 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         const int i = b.order[p];
         double* gi = grad + 6 * (size_t)i;
         const BatchSample& q = b.smp[i];
-        double ab[2];
-        sum_slot_partials(ap.data() + ADJ_PART * b.slot0[p], (int)(b.slot0[p + 1] - b.slot0[p]), ab);
-        adj_param_grads(ab, q.dt, 1.0 / q.Dw, 1.0 / (double)q.nsteps, q.rho, gi);
-        gi[3] = gi[4] = gi[5] = 0;
-        for (int w = 0; w < IC_GRID; ++w)
-            for (int qd = 0; qd < 3; ++qd) gi[3 + qd] += ip[((size_t)p * IC_GRID + w) * 3 + qd];
+        const double* const sp = &sums[(size_t)p * ADJ_SUMS];
+        adj_param_grads(sp, q.dt, 1.0 / q.Dw, 1.0 / (double)q.nsteps, q.rho, gi);
+        for (int qd = 0; qd < 3; ++qd) gi[3 + qd] = sp[2 + qd];
         for (int qd = 0; qd < 4; ++qd) loss[4 * (size_t)i + qd] = out[4 * (size_t)i + qd];
     }
     return GH_OK;
