@@ -2781,7 +2781,9 @@ int gh_set_field_blocks(gh_ctx* ctx, int field, const void* values) {
               : field == GH_FIELD_DPHIDT ? &c->dphidt : nullptr;
     if (!b) return set_error(GH_EINVAL, "gh_set_field_blocks: bad field");
     GH_HIP_CHECK(hipSetDevice(c->device));
-    if (int rc = stage_send(c->device, c->stream, b->p, c->ncells(), 0, c->real_size, values)) return rc;
+    // (block-major already: the runtime's copy, 300 us for 8 MB, 350 through the slabs)
+    GH_HIP_CHECK(hipMemcpyAsync(b->p, values, c->ncells() * c->real_size, hipMemcpyHostToDevice, c->stream));
+    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
     if (field == GH_FIELD_PW || field == GH_FIELD_PG) c->prepared = false;
     return GH_OK;
 }

@@ -276,7 +276,7 @@ int add_anatomy_t(Batch& b, BatchAnatomy& a, int nx, int ny, int nz, const doubl
                   const double* csf) {
     const int n = BS * a.bpd;
     const size_t nc = (size_t)n * n * n;
-    std::vector<Real> pw(nc), pg(nc), pc(nc), tis(nc), bm(nc);
+    std::vector<Real> pw(nc), pg(nc), pc(nc), tis(nc);
     anatomy_from_data<Real>(a.bpd, nx, ny, nz, gm, wm, csf, pw.data(), pg.data(), pc.data(), tis.data());
     a.tissue.resize(nc * sizeof(Real));
     std::memcpy(a.tissue.data(), tis.data(), nc * sizeof(Real));
@@ -288,11 +288,8 @@ int add_anatomy_t(Batch& b, BatchAnatomy& a, int nx, int ny, int nz, const doubl
     if ((rc = a.pw.ensure(nc * sizeof(Real))) || (rc = a.pg.ensure(nc * sizeof(Real)))) return rc;
     const std::vector<Real>* src[2] = {&pw, &pg};
     DevBuf* dst[2] = {&a.pw, &a.pg};
-    for (int f = 0; f < 2; ++f) {
-        for (size_t c = 0; c < nc; ++c) bm[block_index(a.bpd, c)] = (*src[f])[c];
-        GH_HIP_CHECK(hipMemcpyAsync(dst[f]->p, bm.data(), nc * sizeof(Real), hipMemcpyHostToDevice, b.stream));
-        GH_HIP_CHECK(hipStreamSynchronize(b.stream));
-    }
+    for (int f = 0; f < 2; ++f)
+        if ((rc = stage_send(b.device, b.stream, dst[f]->p, nc, a.bpd, sizeof(Real), src[f]->data()))) return rc;
     return GH_OK;
 }
 
@@ -512,11 +509,6 @@ int set_adjoint_samples_t(Batch& b, const double* params, const int64_t* nsteps,
     return GH_OK;
 }
 
-// Launches of the forward sweep: one or two Euler steps over the prefix of
-// running samples, reading phi[cur] and writing phi[1 - cur].  Two steps are
-// taken when no running sample ends after the first of them and (with
-// checkpoints every K) the state after the first is not a checkpoint.  A
-// sample's final state is in the buffer current when it ends.
 // the slots of full[f0 ..] and of the moving groups of grp[g0 ..] from one state to
 // another, an item per workgroup, nf of the first kind
 template <typename Real>
@@ -536,6 +528,10 @@ __global__ __launch_bounds__(256) void copy_moving_kernel(int nf, const int32_t*
     for (int c = threadIdx.x; c < n * BCELLS; c += 256) dst[(size_t)s * BCELLS + c] = src[(size_t)s * BCELLS + c];
 }
 
+// Launches of the forward sweep: one or two Euler steps over the prefix of
+// running samples, reading phi[cur] and writing phi[1 - cur].  Two steps are
+// taken when no running sample and no segment ends after the first of them.  A
+// sample's final state is in the buffer current when it ends.
 template <typename Real>
 struct ForwardSweep {
     Batch& b;
@@ -705,7 +701,8 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
     if ((rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes)) || (rc = b.lam[0].ensure(nc * 8)) ||
         (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
-        (rc = b.icpart.ensure((size_t)ns * (3 * ADJ_IC_GRID + ADJ_SUMS) * 8)) || (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
+        (rc = b.icpart.ensure((size_t)ns * (3 * ADJ_IC_GRID + ADJ_SUMS) * 8)) ||
+        (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
     const BatchStepParams<Real> fprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};

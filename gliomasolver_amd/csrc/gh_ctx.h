@@ -121,7 +121,8 @@ struct Ctx {
     // adaptation scratch kept across epochs: spare field arrays swapped with
     // the live ones by apply_new_tree, split labs, remap list, FWT details
     DevBuf spare[4], labSplit[4], remapBuf, detBuf;
-    PinnedBuf pinRemap, pinDense, pinBlk, pinSplit, pinSlots, pinDet, pinLik;  // staging of the adaptation's host<->device tables
+    PinnedBuf pinRemap, pinDense, pinBlk, pinSplit, pinSlots, pinDet;  // staging of the adaptation's host<->device tables
+    PinnedBuf pinLik;  // sums of the likelihood and of a gradient, written by their last kernel
     // adaptation profile (gh_adapt_profile), host wall time in ms per phase
     double prof[8] = {0};
     // how ghosts were built (gh_adapt_counters): lab batches on the device,
@@ -238,8 +239,8 @@ int grid_compress(Ctx& c, const std::vector<char>& flagged, int* ncollapsed,
 
 // fields to and from the caller's memory (gh_stage.hip), in stream order; each
 // returns when the caller's memory has been read or written.  The caller's array
-// is block-major like the field for bpd 0, dense x-fastest otherwise (a uniform
-// grid of bpd blocks per dimension).
+// is dense x-fastest (a uniform grid of bpd blocks per dimension); for bpd 0, which
+// a fetch takes, it is block-major like the field.
 int stage_fetch(int device, hipStream_t stream, const void* field, size_t cells, int bpd, size_t real_size, void* dst);
 int stage_send(int device, hipStream_t stream, void* field, size_t cells, int bpd, size_t real_size, const void* src);
 // a context (or batch) that may use them is created / destroyed

@@ -112,22 +112,6 @@ void Ctx::release_all() {
     labPermOrder = 0;
 }
 
-// dense x-fastest n^3 -> block-major [slot][z][y][x] for a uniform grid in
-// slot order bx + bpd*(by + bpd*bz)
-template <typename T>
-static void dense_to_blocks(int n, const T* dense, T* bm) {
-    const int bpd = n / BS;
-    for (int bz = 0; bz < bpd; ++bz)
-        for (int by = 0; by < bpd; ++by)
-            for (int bx = 0; bx < bpd; ++bx) {
-                T* dst = bm + ((size_t)bx + (size_t)bpd * (by + (size_t)bpd * bz)) * BCELLS;
-                for (int z = 0; z < BS; ++z)
-                    for (int y = 0; y < BS; ++y)
-                        std::memcpy(dst + BS * (y + BS * z),
-                                    dense + (size_t)BS * bx + (size_t)n * ((size_t)BS * by + y + (size_t)n * (BS * bz + z)),
-                                    BS * sizeof(T));
-            }
-}
 static int check_dense(Ctx* c, int n) {
     if (!c) return set_error(GH_EINVAL, "null context");
     if (c->topo.uniform_bpd <= 0) return set_error(GH_ESTATE, "dense transfer needs a uniform grid");
@@ -168,15 +152,13 @@ static void anatomy(size_t nc, const double* gm, const double* wm, const double*
 template <typename Real>
 static int set_anatomy_t(Ctx* c, int n, const double* gm, const double* wm, const double* csf) {
     const size_t nc = (size_t)n * n * n;
-    std::vector<Real> a(nc), b(nc), d(nc), bm(nc);
+    std::vector<Real> a(nc), b(nc), d(nc);
     anatomy<Real>(nc, gm, wm, csf, a.data(), b.data(), d.data());
     const std::vector<Real>* src[3] = {&a, &b, &d};
     DevBuf* dst[3] = {&c->pw, &c->pg, &c->pcsf};
-    for (int f = 0; f < 3; ++f) {
-        dense_to_blocks<Real>(n, src[f]->data(), bm.data());
-        GH_HIP_CHECK(hipMemcpyAsync(dst[f]->p, bm.data(), nc * sizeof(Real), hipMemcpyHostToDevice, c->stream));
-        GH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    }
+    for (int f = 0; f < 3; ++f)
+        if (int rc = stage_send(c->device, c->stream, dst[f]->p, nc, c->topo.uniform_bpd, sizeof(Real), src[f]->data()))
+            return rc;
     c->prepared = false;
     return GH_OK;
 }
@@ -191,7 +173,6 @@ static int ic_from_anatomy_t(Ctx* c, int nx, int ny, int nz, const double* gm, c
                              const double* tumor_ic) {
     const int bpd = c->topo.uniform_bpd;
     const size_t nc = c->ncells();
-    const int n = BS * bpd;
     std::vector<Real> pw(nc), pg(nc), pc(nc), tis(nc), phi(nc, (Real)0);
     anatomy_from_data<Real>(bpd, nx, ny, nz, gm, wm, csf, pw.data(), pg.data(), pc.data(), tis.data());
     if (tumor_ic) {
@@ -199,14 +180,10 @@ static int ic_from_anatomy_t(Ctx* c, int nx, int ny, int nz, const double* gm, c
         tumour_cells<Real>(bpd, tis.data(), tumor_ic, cells);
         for (const auto& e : cells) phi[e.first] = e.second;
     }
-    std::vector<Real> bm(nc);
     const std::vector<Real>* src[4] = {&pw, &pg, &pc, &phi};
     DevBuf* dst[4] = {&c->pw, &c->pg, &c->pcsf, &c->phi[c->cur]};
-    for (int f = 0; f < (tumor_ic ? 4 : 3); ++f) {
-        dense_to_blocks<Real>(n, src[f]->data(), bm.data());
-        GH_HIP_CHECK(hipMemcpyAsync(dst[f]->p, bm.data(), nc * sizeof(Real), hipMemcpyHostToDevice, c->stream));
-        GH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    }
+    for (int f = 0; f < (tumor_ic ? 4 : 3); ++f)
+        if (int rc = stage_send(c->device, c->stream, dst[f]->p, nc, bpd, sizeof(Real), src[f]->data())) return rc;
     c->prepared = false;
     return GH_OK;
 }

@@ -104,12 +104,22 @@ struct Pair {
     }
 };
 
+// Threads for a transfer of n chunks: one, and one more for each pair of slabs that
+// lies ready.  So a transfer pins two slabs at most (0.5 ms), a program that moves
+// one field pays for no more, and the fourth transfer has its four threads.
+int threads_for(int device, size_t n) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    size_t ready = 0;
+    for (const Slab& f : g_free) ready += f.device == device && f.bytes == kSlabBytes;
+    return (int)std::min<size_t>({(size_t)kStageThreads, n, 1 + ready / 2});
+}
+
 // Runs part(first, last) over the chunks of `bytes` on up to kStageThreads
 // threads; the first failure's code and message.
 template <typename F>
-int in_parts(size_t bytes, F part) {
+int in_parts(int device, size_t bytes, F part) {
     const size_t n = (bytes + kSlabBytes - 1) / kSlabBytes;
-    const int nt = bytes < kThreadedBytes ? 1 : (int)std::min<size_t>(kStageThreads, n);
+    const int nt = bytes < kThreadedBytes ? 1 : threads_for(device, n);
     if (nt <= 1) return part((size_t)0, n);
     int rc[kStageThreads] = {};
     std::string msg[kStageThreads];
@@ -137,7 +147,7 @@ int in_parts(size_t bytes, F part) {
 // device -> dst: fill(offset, bytes, slab) enqueues a chunk of the result
 template <typename Fill>
 int fetch(int device, hipStream_t stream, size_t bytes, void* dst, Fill fill) {
-    return in_parts(bytes, [&](size_t c0, size_t c1) -> int {
+    return in_parts(device, bytes, [&](size_t c0, size_t c1) -> int {
         GH_HIP_CHECK(hipSetDevice(device));
         auto size = [&](size_t c) { return std::min(kSlabBytes, bytes - c * kSlabBytes); };
         Pair p;
@@ -162,7 +172,7 @@ int fetch(int device, hipStream_t stream, size_t bytes, void* dst, Fill fill) {
 // src -> device: drain(offset, bytes, slab) enqueues a chunk's use
 template <typename Drain>
 int send(int device, hipStream_t stream, size_t bytes, const void* src, Drain drain) {
-    return in_parts(bytes, [&](size_t c0, size_t c1) -> int {
+    return in_parts(device, bytes, [&](size_t c0, size_t c1) -> int {
         GH_HIP_CHECK(hipSetDevice(device));
         Pair p;
         int rc;
@@ -208,11 +218,13 @@ __global__ __launch_bounds__(256) void units_kernel(int bpd, size_t first, unsig
         *b = slab[i];
 }
 
-// bpd 0: block-major
+// bpd 0: block-major (a fetch only)
 template <bool FETCH>
 int units(hipStream_t stream, int bpd, size_t real_size, void* f, size_t offset, size_t bytes, void* slab) {
     const unsigned n = (unsigned)(bytes / 16);
-    auto* k = bpd == 0 ? units_kernel<0, FETCH> : real_size == 4 ? units_kernel<2, FETCH> : units_kernel<4, FETCH>;
+    auto* k = real_size == 4 ? units_kernel<2, FETCH> : units_kernel<4, FETCH>;
+    if constexpr (FETCH)
+        if (bpd == 0) k = units_kernel<0, true>;
     hipLaunchKernelGGL(k, dim3((n + 255) / 256), dim3(256), 0, stream, bpd, offset / 16, n, (Unit*)f, (Unit*)slab);
     GH_HIP_CHECK(hipGetLastError());
     return GH_OK;
