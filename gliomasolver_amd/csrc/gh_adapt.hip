@@ -1549,6 +1549,7 @@ int device_face_table(Ctx& c, bool& done) {
     }
     if (!bad) {
         c.nFacePatch = nf;
+        c.facePatchOrder = order;
         done = true;
         return GH_OK;
     }
@@ -1750,7 +1751,7 @@ int prepare_ghosted_t(Ctx& c, double Dw, double Dg) {
                                c.faceList.as<int32_t>(), c.faceCode.as<int32_t>(), c.faceSrc.as<int32_t>(),
                                c.pw.as<Real>(), c.pg.as<Real>(), c.fgPw.as<Real>(), c.fgPg.as<Real>());
         };
-        if (c.tree.order == 4) go(face_patch_kernel<Real, 4>);
+        if (c.facePatchOrder == 4) go(face_patch_kernel<Real, 4>);
         else go(face_patch_kernel<Real, 2>);
         GH_HIP_CHECK(hipGetLastError());
     } else if ((rc = face_ghosts<Real>(c, c.pw.as<Real>(), c.fgPw.as<Real>())) ||
@@ -1808,7 +1809,7 @@ int step_ghosted_t(Ctx& c, const Real* in, Real* out, double dt) {
         };
         constexpr int MANY = sizeof(Real) == 4 ? 256 : 512;
         const bool few = ns <= kPatchedFewBlocks;
-        if (c.tree.order == 4) {
+        if (c.facePatchOrder == 4) {
             if (few) go(rd_step_patched_kernel<Real, FUSED, 4, 512>, 512);
             else go(rd_step_patched_kernel<Real, FUSED, 4, MANY>, MANY);
         } else {
@@ -2291,7 +2292,11 @@ int gh_grid_configure(gh_ctx* ctx, int wavelet_order, int max_level, int min_lev
     if ((wavelet_order != 2 && wavelet_order != 4) || max_level < 0 || max_level > 9 || min_level < 0 ||
         min_level > max_level)
         return set_error(GH_EINVAL, "gh_grid_configure: order 2|4, 0 <= min_level <= max_level <= 9");
-    if (c->tree.order != wavelet_order) c->labAllVersion = ~(uint64_t)0;  // labs are sized by the order
+    if (c->tree.order != wavelet_order) {
+        c->labAllVersion = ~(uint64_t)0;  // labs are sized by the order
+        c->faces_stale = true;            // so are the face ghosts' patches, and the ghosts' taps are its
+        if (c->prepared && c->topo.uniform_bpd <= 0) c->constants_stale = true;  // made from the ghosts' p_w, p_g
+    }
     c->tree.order = wavelet_order;
     c->tree.max_level = max_level;
     c->tree.min_level = min_level;

@@ -97,8 +97,9 @@ struct Ctx {
     int nFacePk = 0;                 // faces in packets (0: the GhostEntry table is used)
     // device-built face table in patches (every ghost of the grid from single
     // cells of its face's patch): cells in faceSrc, a face's neighbour
-    // or patch in faceCode; 0: packets or the GhostEntry table
-    int nFacePatch = 0;
+    // or patch in faceCode; 0: packets or the GhostEntry table.  Rows are laid
+    // out, and must be read, for the wavelet order of the time they were built
+    int nFacePatch = 0, facePatchOrder = 0;
     DevBuf fgPhi, fgTau, fgDm;       // per slot: 6*64 ghost phi, 6*64 ghost tau, 3*64 minus-face D
     DevBuf fgPw, fgPg;               // per slot: 6*64 ghost p_w, p_g (statics)
     // FWT / split labs (compact, one per listed slot)
