@@ -232,6 +232,13 @@ class Context:
         check(self.lib.gh_adapt_counters(self.h, _ptr(n), int(reset)))
         return dict(zip(("labs_device", "labs_host", "faces_device", "faces_host"), n.tolist()))
 
+    def face_ghost_info(self) -> dict:
+        """The form of the multi-level step's face ghosts: jump faces in patches,
+        in packets, ghosts of a host-built table."""
+        v = [C.c_int() for _ in range(3)]
+        check(self.lib.gh_face_ghost_info(self.h, *[C.byref(x) for x in v]))
+        return dict(zip(("patches", "packets", "entries"), [x.value for x in v]))
+
     def set_field_blocks(self, field: int, values: np.ndarray):
         v = np.ascontiguousarray(values, self.dtype).reshape(self.nblocks(), 8, 8, 8)
         check(self.lib.gh_set_field_blocks(self.h, field, _ptr(v)))

@@ -45,6 +45,7 @@ SIGNATURES = {
     "gh_grid_compress_blocks": (_i, [_vp, _i, _vp, _pi]),
     "gh_adapt_profile": (_i, [_vp, _vp, _i]),
     "gh_adapt_counters": (_i, [_vp, _vp, _i]),
+    "gh_face_ghost_info": (_i, [_vp, _pi, _pi, _pi]),
     "gh_set_field_blocks": (_i, [_vp, _i, _vp]),
     "gh_get_field_blocks": (_i, [_vp, _i, _vp]),
     "gh_uq_resample": (_i, [_vp, _i, _vp]),

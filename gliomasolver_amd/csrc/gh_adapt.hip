@@ -2766,6 +2766,16 @@ int gh_adapt_counters(gh_ctx* ctx, int64_t* counts, int reset) {
     return GH_OK;
 }
 
+int gh_face_ghost_info(gh_ctx* ctx, int* patches, int* packets, int* entries) {
+    Ctx* c = as_ctx(ctx);
+    if (!c || !patches || !packets || !entries) return set_error(GH_EINVAL, "gh_face_ghost_info: NULL argument");
+    const bool built = c->topo.uniform_bpd <= 0 && !c->faces_stale;
+    *patches = built ? c->nFacePatch : 0;
+    *packets = built ? c->nFacePk : 0;
+    *entries = built ? c->nFaceEnt : 0;
+    return GH_OK;
+}
+
 int gh_adapt_profile(gh_ctx* ctx, double* ms, int reset) {
     Ctx* c = as_ctx(ctx);
     if (!c) return set_error(GH_EINVAL, "null context");

@@ -110,6 +110,12 @@ int gh_adapt_profile(gh_ctx* ctx, double* ms, int reset);
  * Host tables are used only for ghosts that need more than two synthesis
  * levels; any depth of the tree is served on the device otherwise. */
 int gh_adapt_counters(gh_ctx* ctx, int64_t* counts, int reset);
+/* gh_face_ghost_info: which form the face ghosts of the multi-level RD step have
+ * (no reference counterpart; for tuning and tests): jump faces in patches, jump
+ * faces in term packets, single ghosts of a host-built table -- at most one of
+ * them not 0.  All 0 on a uniform grid, and from a change of the grid or of the
+ * wavelet order to the next RD call. */
+int gh_face_ghost_info(gh_ctx* ctx, int* patches, int* packets, int* entries);
 int gh_set_field_blocks(gh_ctx* ctx, int field, const void* values);
 int gh_get_field_blocks(gh_ctx* ctx, int field, void* values);
 int gh_uq_resample(gh_ctx* ctx, int gpd, double* out);
