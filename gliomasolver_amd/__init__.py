@@ -356,6 +356,10 @@ class Context:
                                      loss, grad))
         return np.array(loss[:]), np.array(grad[:])
 
+    def adjoint_release(self):
+        """Frees the tape and the checkpoints that rd_adjoint keeps."""
+        check(self.lib.gh_adjoint_release(self.h))
+
     def checkpoint_save(self, slot: int):
         check(self.lib.gh_checkpoint_save(self.h, slot))
 
@@ -452,6 +456,10 @@ class Batch:
         check(self.lib.gh_batch_adjoint(self.h, ckpt_every, _ptr(lp), stepPET, stepTi, int(use_roi), _ptr(loss),
                                         _ptr(grad), C.byref(ms)))
         return loss, grad, ms.value
+
+    def adjoint_release(self):
+        """Frees the tape and the checkpoints that adjoint keeps."""
+        check(self.lib.gh_batch_adjoint_release(self.h))
 
     def likelihood(self, lik_params, stepPET=1, stepTi=1, use_roi=False) -> np.ndarray:
         """(N, 4) rows {-logL, L_PET, L_T1, L_T2}; lik_params (N, 5) or one row for all."""

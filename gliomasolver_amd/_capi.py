@@ -71,6 +71,7 @@ SIGNATURES = {
     "gh_likelihood_dense": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _pd, _i, _i, _pd, _pi64]),
     "gh_likelihood_noalloc": (_i, [_vp, _pd, _i, _i, _i, _pd, _pi64]),
     "gh_rd_adjoint": (_i, [_vp, _i64, _d, _i, _pd, _i, _i, _i, _pd, _d, _pd, _pd]),
+    "gh_adjoint_release": (_i, [_vp]),
     "gh_checkpoint_save": (_i, [_vp, _i]),
     "gh_checkpoint_load": (_i, [_vp, _i]),
     "gh_batch_create": (_i, [_i, _i, C.POINTER(_vp)]),
@@ -82,6 +83,7 @@ SIGNATURES = {
     "gh_batch_likelihood": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "gh_batch_set_adjoint_samples": (_i, [_vp, _i, _vp, _vp, _vp, _d, _d]),
     "gh_batch_adjoint": (_i, [_vp, _i, _vp, _i, _i, _i, _vp, _vp, _pd]),
+    "gh_batch_adjoint_release": (_i, [_vp]),
     "gh_batch_sample_info": (_i, [_vp, _i, _pd, _pd, _pd, _pi64]),
     "gh_batch_get_phi": (_i, [_vp, _i, _vp]),
     "gh_batch_get_anatomy": (_i, [_vp, _i, _vp, _vp]),

@@ -23,7 +23,7 @@
 // FP64 per wave (dt, rho, N and Dw are constant over the solve and applied
 // once at the end); every wave owns the same cells in every step, so the
 // accumulation order is fixed.  The states that fit the tape
-// (tape_ensure) stay on it from the forward sweep, which writes them there; the
+// (TapeBuf) stay on it from the forward sweep, which writes them there; the
 // steps before them are cut into segments of the tape's length, recomputed from
 // checkpoints taken in the forward sweep.  With every segment recomputed, 343
 // steps of 64^3 FP64 took 3.3 ms (2.7 with none), 1,000 of 128^3 FP32 12.8 (11.0).
@@ -46,18 +46,27 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
               const double* ic, double sigma, double* loss, double* grad) {
     const size_t nc = c.ncells();
     const size_t nb = nc * sizeof(Real);
+    const int ns = c.topo.nblocks();
     int rc;
-    if ((rc = tape_ensure(c.adjSeg, ((size_t)std::min<int64_t>(K, N) + 1) * nb, ((size_t)N + 1) * nb))) return rc;
-    // segments of `len` steps, the first one shorter; the last stays on the tape
-    const int64_t len = std::min<int64_t>(N, (int64_t)(c.adjSeg.bytes / nb) - 1);
-    const int64_t nseg = (N + len - 1) / len;
-    auto start = [&](int64_t i) { return i == 0 ? (int64_t)0 : N - (nseg - i) * len; };
-    if ((rc = c.adjCk.ensure(std::max<size_t>(1, (size_t)(nseg - 1)) * nb)) || (rc = c.adjLam[0].ensure(nc * 8)) ||
-        (rc = c.adjLam[1].ensure(nc * 8)))
+    if ((rc = c.adjLam[0].ensure(nc * 8)) || (rc = c.adjLam[1].ensure(nc * 8)) ||
+        (rc = c.adjPart.ensure(sizeof(double) * ADJ_PART * ns)))
         return rc;
+    // segments of `len` steps, the first one shorter; the last stays on the tape.  Where
+    // its length beyond K leaves no room for the checkpoints, K it is
+    const size_t need = ((size_t)std::min<int64_t>(K, N) + 1) * nb;
+    int64_t len = 0, nseg = 0;
+    for (size_t want = ((size_t)N + 1) * nb;; want = need) {
+        if ((rc = c.adjSeg.ensure(c.device, need, want))) return rc;
+        len = std::min<int64_t>(N, (int64_t)(c.adjSeg.buf.bytes / nb) - 1);
+        nseg = (N + len - 1) / len;
+        rc = c.adjCk.ensure(std::max<size_t>(1, (size_t)(nseg - 1)) * nb);
+        if (rc == GH_OK) break;
+        if (want == need) return rc;
+    }
+    auto start = [&](int64_t i) { return i == 0 ? (int64_t)0 : N - (nseg - i) * len; };
     const double dt = T / (double)N;
     char* ck = (char*)c.adjCk.p;
-    char* seg = (char*)c.adjSeg.p;
+    char* seg = (char*)c.adjSeg.buf.p;
     // two steps per launch from a clamped state (k >= 1) within a segment
     const bool pairs = c.fast_ok && c.topo.uniform_bpd > 0;
     // the two-step schedule (tile 0) leaves out the groups of blocks without
@@ -118,8 +127,6 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     if (still)  // the launches leave out the seed in the still groups: it stands in both adjoint buffers
         GH_HIP_CHECK(hipMemcpyAsync(c.adjLam[1 - lc].p, c.adjLam[lc].p, nc * 8, hipMemcpyDeviceToDevice, c.stream));
     // reverse sweep
-    const int ns = c.topo.nblocks();
-    if ((rc = c.adjPart.ensure(sizeof(double) * ADJ_PART * ns))) return rc;
     GH_HIP_CHECK(hipMemsetAsync(c.adjPart.p, 0, sizeof(double) * ADJ_PART * ns, c.stream));
     const double h = block_h_of(c);
     const double ih2 = 1. / (h * h);
@@ -192,4 +199,14 @@ extern "C" int gh_rd_adjoint(gh_ctx* ctx, int64_t nsteps, double T, int ckpt_eve
                                   ic_sigma, loss, grad)
                : adjoint_t<double>(*c, nsteps, T, ckpt_every, lik_params, stepPET, stepTi, use_roi, ic_center,
                                    ic_sigma, loss, grad);
+}
+
+extern "C" int gh_adjoint_release(gh_ctx* ctx) {
+    Ctx* c = as_ctx(ctx);
+    if (!c) return set_error(GH_EINVAL, "null context");
+    GH_HIP_CHECK(hipSetDevice(c->device));
+    GH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    c->adjSeg.release();
+    c->adjCk.release();
+    return GH_OK;
 }

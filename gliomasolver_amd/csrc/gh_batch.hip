@@ -260,7 +260,8 @@ struct Batch {
         return step_work(nFull[p], fullItem.as<int32_t>(), nGrp[p], grpList.as<int2>(),
                          skip_still ? stillGrp.as<unsigned char>() : nullptr);
     }
-    DevBuf ck, tape, lam[2], apart, icpart, adjJobs;  // adjoint
+    DevBuf ck, lam[2], apart, icpart, adjJobs;  // adjoint
+    TapeBuf tape;
     double ic_is2 = 1.0;                                 // adjoint: 1 / sigma^2 of the Gaussian IC
     std::vector<int> final_buf;                          // per position: phi buffer of the final state
     bool ran = false, adjoint = false;
@@ -657,7 +658,7 @@ int likelihood_t(Batch& b, const double* lik, int stepPET, int stepTi, int use_r
 // slot prefix in both directions (the reverse of sample s starts at its own step
 // N_s - 1, with its seed placed in the adjoint buffer of parity N_s).  The tape
 // holds the states of the last segment of steps from the forward sweep on
-// (tape_ensure), each the slots of the samples that reached it; earlier segments
+// (TapeBuf), each the slots of the samples that reached it; earlier segments
 // are recomputed from a checkpoint at their start.
 template <typename Real>
 int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int use_roi, double* loss, double* grad,
@@ -681,34 +682,42 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         return b.slot0[p] * (size_t)k + ended[p];
     };
     int rc;
-    if ((rc = tape_ensure(b.tape, (size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes,
-                          cum(Nmax + 1) * slot_bytes)))
-        return rc;
-    // segments [start[i], start[i + 1]) of steps, as long as the tape takes
-    std::vector<int64_t> start{Nmax};
-    for (int64_t e = Nmax; e > 0;) {
-        int64_t lo = 0, hi = e - 1;  // (one step always fits)
-        while (lo < hi) {
-            const int64_t s = (lo + hi) / 2;
-            if ((cum(e + 1) - cum(s)) * slot_bytes <= b.tape.bytes) hi = s;
-            else lo = s + 1;
-        }
-        start.push_back(e = hi);
-    }
-    std::reverse(start.begin(), start.end());
-    const int nseg = (int)start.size() - 1;
-    std::vector<size_t> ckoff(nseg, 0);
-    for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
-    if ((rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes)) || (rc = b.lam[0].ensure(nc * 8)) ||
-        (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
+    if ((rc = b.lam[0].ensure(nc * 8)) || (rc = b.lam[1].ensure(nc * 8)) || (rc = b.apart.ensure(ADJ_PART * nsl * 8)) ||
         (rc = b.icpart.ensure((size_t)ns * (3 * ADJ_IC_GRID + ADJ_SUMS) * 8)) ||
         (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
+    // segments [start[i], start[i + 1]) of steps, as long as the tape takes; where its
+    // length beyond K leaves no room for the checkpoints, K it is
+    const size_t all = cum(Nmax + 1) * slot_bytes,
+                 need = std::min((size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes, all);
+    std::vector<int64_t> start;
+    std::vector<size_t> ckoff;
+    int nseg = 0;
+    for (size_t want = all;; want = need) {
+        if ((rc = b.tape.ensure(b.device, need, want))) return rc;
+        start.assign(1, Nmax);
+        for (int64_t e = Nmax; e > 0;) {
+            int64_t lo = 0, hi = e - 1;  // (one step always fits)
+            while (lo < hi) {
+                const int64_t s = (lo + hi) / 2;
+                if ((cum(e + 1) - cum(s)) * slot_bytes <= b.tape.buf.bytes) hi = s;
+                else lo = s + 1;
+            }
+            start.push_back(e = hi);
+        }
+        std::reverse(start.begin(), start.end());
+        nseg = (int)start.size() - 1;
+        ckoff.assign(nseg, 0);
+        for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
+        rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes);
+        if (rc == GH_OK) break;
+        if (want == need) return rc;
+    }
     const BatchStepParams<Real> fprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     char* ck = (char*)b.ck.p;
     auto state = [&](int seg, int64_t k) {
-        return (Real*)((char*)b.tape.p + (cum(k) - cum(start[seg])) * slot_bytes);
+        return (Real*)((char*)b.tape.buf.p + (cum(k) - cum(start[seg])) * slot_bytes);
     };
     // the tape's zeros that no launch writes, over runs of states of one size
     auto zero_still = [&](int seg) -> int {
@@ -758,7 +767,7 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     }
     fw.retire(k);
     const int last = nseg - 1;
-    GH_HIP_CHECK(hipMemcpyAsync(b.tape.p, b.phi[fw.cur].p, b.slot0[fw.active] * slot_bytes, hipMemcpyDeviceToDevice,
+    GH_HIP_CHECK(hipMemcpyAsync(b.tape.buf.p, b.phi[fw.cur].p, b.slot0[fw.active] * slot_bytes, hipMemcpyDeviceToDevice,
                                 b.stream));
     if ((rc = zero_still(last))) return rc;
     // the final states go where a solve leaves them (the still groups are there)
@@ -828,7 +837,7 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
     for (int i = last; i >= 0; --i) {
         const int64_t k0 = start[i], k1 = start[i + 1];
         if (i < last) {
-            GH_HIP_CHECK(hipMemcpyAsync(b.tape.p, ck + ckoff[i] * slot_bytes, b.slot0[active(k0)] * slot_bytes,
+            GH_HIP_CHECK(hipMemcpyAsync(b.tape.buf.p, ck + ckoff[i] * slot_bytes, b.slot0[active(k0)] * slot_bytes,
                                         hipMemcpyDeviceToDevice, b.stream));
             if ((rc = zero_still(i)) || (rc = run_on_tape(i, k1 - 1, [](int64_t) { return GH_OK; }))) return rc;
         }
@@ -927,10 +936,11 @@ int gh_batch_destroy(gh_batch* bh) {
         a->roi.release();
     }
     DevBuf* bufs[] = {&b->phi[0], &b->phi[1], &b->statD,  &b->statSig, &b->slotPos, &b->slotItem, &b->fullItem, &b->range,
-                      &b->apw,    &b->apg,    &b->likPart, &b->likOut, &b->likJobs, &b->ck,     &b->tape,
+                      &b->apw,    &b->apg,    &b->likPart, &b->likOut, &b->likJobs, &b->ck,
                       &b->lam[0], &b->lam[1], &b->apart,   &b->icpart, &b->adjJobs, &b->statF,  &b->flag,
                       &b->zeroFlux, &b->fullList, &b->grpList, &b->stillGrp};
     for (DevBuf* d : bufs) d->release();
+    b->tape.release();
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -1076,6 +1086,16 @@ int gh_batch_adjoint(gh_batch* bh, int ckpt_every, const double* lik_params, int
     return b->real_kind == GH_REAL_F32
                ? adjoint_t<float>(*b, ckpt_every, lik_params, stepPET, stepTi, use_roi, loss, grad, elapsed_ms)
                : adjoint_t<double>(*b, ckpt_every, lik_params, stepPET, stepTi, use_roi, loss, grad, elapsed_ms);
+}
+
+int gh_batch_adjoint_release(gh_batch* bh) {
+    Batch* b = as_batch(bh);
+    if (!b) return set_error(GH_EINVAL, "null batch");
+    GH_HIP_CHECK(hipSetDevice(b->device));
+    GH_HIP_CHECK(hipStreamSynchronize(b->stream));
+    b->tape.release();
+    b->ck.release();
+    return GH_OK;
 }
 
 int gh_batch_sample_info(gh_batch* bh, int sample, double* Dw, double* Dg, double* dt, int64_t* nsteps) {

@@ -47,6 +47,25 @@ struct DevBuf {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// The tape of a trajectory's states of a gradient.  The caller's checkpoint
+// interval asks for `need` bytes; up to `want` (the whole trajectory) are taken
+// beyond it, since the states on the tape need no second solve on the way back, a
+// quarter of a gradient's launches.  What is taken beyond `need` is at most an
+// eighth of what is free, and over all contexts and batches of the process an eighth
+// of the device's memory: more of them do with shorter tapes.  It is kept between
+// calls (taking freed memory again waits until it has been cleared: a gradient of
+// 1,001 steps of 128^3 FP32 took 127 instead of 11 ms) until release().
+struct TapeBuf {
+    DevBuf buf;
+    int ensure(int device, size_t need, size_t want);
+    void release();
+    ~TapeBuf() { release(); }
+
+private:
+    int dev = 0;
+    size_t extra = 0;  // bytes beyond the last need
+};
+
 // Pinned host staging buffer (hipHostMalloc), move-only, freed by the
 // destructor.  The adaptation's per-epoch tables go to and from the device
 // through these, so each hipMemcpyAsync is one DMA (from pageable memory the
@@ -161,7 +180,8 @@ struct Ctx {
     // likelihood data (block-major): y == 1 flags of T1c/FLAIR, PET values, ROI {cell, ix, iy, iz}
     DevBuf obsT1, obsFl, obsPet, obsRoi, likPart;
     // adjoint: forward checkpoints, segment tape, adjoint ping-pong (FP64), parameter partials
-    DevBuf adjCk, adjSeg, adjLam[2], adjPart;
+    DevBuf adjCk, adjLam[2], adjPart;
+    TapeBuf adjSeg;
     int nroi = 0;
     bool lik_ready = false;
     uint64_t lik_version = 0;  // tree_version the likelihood data was laid out for
@@ -248,11 +268,6 @@ int stage_send(int device, hipStream_t stream, void* field, size_t cells, int bp
 void stage_retain();
 void stage_release();
 
-// A tape of a trajectory's states: at least `need` bytes, up to `want` (the whole
-// trajectory) while that stays within an eighth of the device's free memory; what
-// it already holds counts as free.  The states on it need no second solve on the
-// way back, a quarter of a gradient's launches.
-int tape_ensure(DevBuf& tape, size_t need, size_t want);
 
 // likelihood helpers (gh_lik.hip): -logL of the current phi; dJ/du of a state buffer
 int lik_eval_current(Ctx& c, const double* params, int stepPET, int stepTi, int use_roi, double* out,

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 
 #include "gh_anatomy.h"
@@ -24,6 +25,7 @@ int DevBuf::ensure(size_t nbytes) {
     if (nbytes == 0) return GH_OK;
     hipError_t e = hipMalloc(&p, nbytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // (reported here: not by the next launch's check too)
         p = nullptr;
         return set_error(GH_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     }
@@ -40,22 +42,52 @@ void DevBuf::release() {
     bytes = 0;
 }
 
-int tape_ensure(DevBuf& tape, size_t need, size_t want) {
-    if (tape.bytes >= want && tape.p) return GH_OK;
-    size_t room = 0, total = 0;
-    if (hipMemGetInfo(&room, &total) != hipSuccess) {
+namespace {
+constexpr int kTapeShare = 8;  // of the device's memory (TapeBuf)
+struct TapeSum {
+    size_t total = 0;  // the device's memory
+    size_t extra = 0;  // the sum over its tapes
+};
+std::mutex g_tape_mu;
+TapeSum g_tapes[64];  // per device
+TapeSum& tape_sum(int device) { return g_tapes[device % 64]; }
+}  // namespace
+
+int TapeBuf::ensure(int device, size_t need, size_t want) {
+    need = std::min(need, want);
+    size_t room = 0, total = 0, take = 0;
+    const size_t held = buf.p ? buf.bytes : 0;  // counts as free
+    if (held < want && hipMemGetInfo(&room, &total) != hipSuccess) {
         (void)hipGetLastError();
-        room = 0;
+        room = total = 0;
     }
-    const size_t held = tape.p ? tape.bytes : 0;
-    const size_t most = std::min(want, (room + held) / 8);
-    // (a tape short of the whole trajectory is not given up for one little longer)
-    if (held >= need && most < want && most <= held + held / 4) return GH_OK;
-    if (most > need) {
-        if (tape.ensure(most) == GH_OK) return GH_OK;
-        (void)hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lock(g_tape_mu);
+        TapeSum& sum = tape_sum(device);
+        if (total) sum.total = total;
+        if (held >= want) room = sum.total;  // (nothing more is taken)
+        dev = device;
+        sum.extra -= extra;
+        const size_t share = sum.total / kTapeShare, left = share > sum.extra ? share - sum.extra : 0;
+        take = std::min({want, need + left, std::max(need, (room + held) / kTapeShare)});
+        // (a tape short of the whole trajectory is not given up for one little longer)
+        if (held >= need && held <= need + left && (held >= want || take <= held + held / 4)) take = held;
+        extra = take - need;
+        sum.extra += extra;
     }
-    return tape.ensure(need);
+    if (take == held) return GH_OK;
+    buf.release();
+    if (buf.ensure(take) == GH_OK) return GH_OK;
+    release();
+    return buf.ensure(need);
+}
+
+void TapeBuf::release() {
+    buf.release();
+    if (extra == 0) return;
+    std::lock_guard<std::mutex> lock(g_tape_mu);
+    tape_sum(dev).extra -= extra;
+    extra = 0;
 }
 
 int PinnedBuf::ensure_grow(size_t nbytes) {
@@ -102,8 +134,9 @@ void Ctx::release_all() {
                       &labAllSrc, &labAllW, &labAllSlots, &dDense, &dBlk, &dBad, &spare[0], &spare[1], &spare[2], &spare[3],
                       &labSplit[0], &labSplit[1], &labSplit[2], &labSplit[3], &remapBuf, &detBuf, &phi[0],  &phi[1],    &dphidt,      &pw,      &pg,
                       &pcsf,     &statD,   &statSig,    &statF,     &flag,      &zeroFlux,   &fullList, &grpList, &stillGrp,      &nbr,         &obsT1,   &obsFl,
-                      &obsPet,   &obsRoi,  &likPart,    &adjCk,     &adjSeg,    &adjLam[0],   &adjLam[1], &adjPart};
+                      &obsPet,   &obsRoi,  &likPart,    &adjCk,     &adjLam[0],   &adjLam[1], &adjPart};
     for (DevBuf* b : bufs) b->release();
+    adjSeg.release();
     for (DevBuf& b : ckpt) b.release();
     faceScan.release();
     dHashKey.release();

@@ -246,10 +246,13 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
  * gh_rd_adjoint: forward solve of nsteps fused steps with dt = T/nsteps from
  * the current phi (the IC), J = -logL(u_N) as gh_likelihood, then the
  * hand-written discrete adjoint backwards.  The states of the last steps stay on
- * a tape of at least ckpt_every + 1 states, longer while it fits an eighth of
- * the device's free memory; earlier ones are recomputed from checkpoints, a
- * tape's length at a time.  The result does not depend on the length.  The
- * no-flux flags, the in-domain test and the upper clamp are frozen along the
+ * a tape of at least ckpt_every + 1 states; earlier ones are recomputed from
+ * checkpoints, a tape's length at a time.  The tape is longer, up to the whole
+ * trajectory, while what it takes beyond ckpt_every + 1 states is within an
+ * eighth of the device's free memory and, over all contexts and batches of the
+ * process, within an eighth of the device's memory.  The result does not depend
+ * on the length.  The context keeps it until gh_adjoint_release or
+ * gh_ctx_destroy.  The no-flux flags, the in-domain test and the upper clamp are frozen along the
  * trajectory; the lower clamp is treated as inactive.
  * Requires gh_rd_prepare(Dw, Dg = Dw/10, rho) and gh_lik_set_data.  The IC is
  * taken to be a Gaussian of width ic_sigma (cells) centred at ic_center
@@ -260,6 +263,10 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
 int gh_rd_adjoint(gh_ctx* ctx, int64_t nsteps, double T, int ckpt_every, const double* lik_params,
                   int stepPET, int stepTi, int use_roi, const double* ic_center, double ic_sigma,
                   double* loss, double* grad);
+/* gh_adjoint_release (and gh_batch_adjoint_release below): waits for the
+ * context's work and frees its tape and its checkpoints; the next gradient takes
+ * them anew. */
+int gh_adjoint_release(gh_ctx* ctx);
 
 /* ---- checkpoints (no reference counterpart: the reference keeps one copy of
  * the state) -- device-side copies of phi, used to restart solves from one
@@ -317,13 +324,14 @@ int gh_batch_likelihood(gh_batch* b, const double* lik_params, int stepPET, int 
  *   samples at once; loss = 4 doubles
  *   and grad = 6 doubles {dJ/dDw, rho, T, x0, y0, z0} per sample, each equal
  *   to gh_rd_adjoint on that sample alone.  Memory: a tape of at
- *   least ckpt_every + 1 states of all samples, at most every state of every
- *   sample or an eighth of the free memory; a checkpoint for each tape's length
+ *   least ckpt_every + 1 states of all samples, longer as gh_rd_adjoint's, at
+ *   most every state of every sample; a checkpoint for each tape's length
  *   before the last; two FP64 adjoint states per cell. */
 int gh_batch_set_adjoint_samples(gh_batch* b, int nsamples, const int* anatomy_id, const double* params,
                                  const int64_t* nsteps, double ic_sigma, double ic_peak);
 int gh_batch_adjoint(gh_batch* b, int ckpt_every, const double* lik_params, int stepPET, int stepTi, int use_roi,
                      double* loss, double* grad, double* elapsed_ms);
+int gh_batch_adjoint_release(gh_batch* b);
 int gh_batch_sample_info(gh_batch* b, int sample, double* Dw, double* Dg, double* dt, int64_t* nsteps);
 int gh_batch_get_phi(gh_batch* b, int sample, void* dense);
 int gh_batch_get_anatomy(gh_batch* b, int anatomy_id, void* p_w, void* p_g);

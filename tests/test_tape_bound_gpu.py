@@ -1,0 +1,104 @@
+"""What gradients keep of the device's memory: beyond the states that the
+checkpoint interval asks for, at most an eighth of it over all contexts of the
+process, and nothing once released or closed; and the same results from a whole
+tape, one cut short beside other contexts' tapes, and one taken anew."""
+import threading
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import gliomasolver_amd as gh
+from test_batch_gpu import LIK, anatomy, observations
+from test_still_gpu import N, context
+
+pytestmark = pytest.mark.gpu
+STEPS, K, CONTEXTS = 12000, 16, 5  # a trajectory of 64^3 FP32: 12.6 GB
+OWN = 256 << 20                    # a context's fields, constants and tape of K + 1 states: under 100 MB
+
+
+def opened():
+    ctx, dt = context("f32", "moving")
+    rng = np.random.default_rng(1)
+    t1, fl = (rng.random((2, N, N, N)) < 0.3).astype(np.float64)
+    ctx.lik_set_data(t1, fl, np.where(t1 > 0, 0.5, 0.0))
+    return ctx, dt
+
+
+def gradient(ctx, dt):
+    ctx.checkpoint_load(0)
+    return np.concatenate(ctx.rd_adjoint(STEPS, STEPS * dt, (30.0, 33.0, 29.0), ckpt_every=K)).view(np.uint64)
+
+
+def free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()
+
+
+def given_back(before, most):
+    """Whether all but `most` bytes are free again; the driver takes them back a
+    few milliseconds after the library has freed them."""
+    for _ in range(50):
+        if before - free()[0] <= most:
+            return True
+        time.sleep(0.02)
+    return False
+
+
+def test_kept_memory_is_bounded():
+    opened()[0].close()  # the library's and the runtime's own first allocations
+    before, total = free()
+    if CONTEXTS * STEPS * N ** 3 * 4 <= total // 8 + CONTEXTS * OWN or before < 2 * total // 3:
+        pytest.skip("another size of device, or one in use")
+    ctxs = [opened() for _ in range(CONTEXTS)]
+    first = [gradient(*c) for c in ctxs]
+    kept = before - free()[0]
+    assert kept <= total // 8 + CONTEXTS * OWN, "%.2f GB kept" % (kept / 1e9)
+    ctxs[0][0].adjoint_release()
+    again = [gradient(*c) for c in ctxs]
+    assert given_back(before, total // 8 + CONTEXTS * OWN)
+    for r in first[1:] + again:
+        assert np.array_equal(first[0], r)
+    for c, _ in ctxs:
+        c.adjoint_release()
+    assert given_back(before, CONTEXTS * OWN)
+    for c, _ in ctxs:
+        c.close()
+    assert given_back(before, OWN)
+
+
+def test_batch_release():
+    b = gh.Batch(0, "f32")
+    b.set_observations(b.add_anatomy(8, *anatomy((70, 60, 64), 3)), *observations(64, 3))
+    rows = [(0.0004, 0.2, 30.0, 28.6, 32.0, 27.4)] * 3
+    out = []
+    for _ in range(2):
+        b.set_adjoint_samples([0] * 3, rows, [3000, 2000, 40], 1.0, 0.1)
+        before = free()[0]
+        out.append(np.concatenate(b.adjoint(LIK, ckpt_every=K, stepPET=2)[:2], axis=1).view(np.uint64))
+        assert before - free()[0] >= 5000 * N ** 3 * 4
+        b.adjoint_release()
+        assert given_back(before, OWN)
+    assert np.array_equal(*out)
+    b.close()
+
+
+def test_gradients_side_by_side():
+    ctxs = [opened() for _ in range(3)]
+    want = gradient(*ctxs[0])
+    got = [None] * len(ctxs)
+
+    def run(i):
+        for _ in range(2):
+            got[i] = gradient(*ctxs[i])
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(ctxs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g in got:
+        assert np.array_equal(want, g)
+    for c, _ in ctxs:
+        c.close()
