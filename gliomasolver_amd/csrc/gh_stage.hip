@@ -8,8 +8,9 @@
 // that one is filled while the other is emptied.  A field of 256^3 FP32 cells
 // arrives in 2.4 ms (21 before), 128^3 in 0.3 ms (0.75), 32^3 in 25 us (60).
 //
-// The slabs outlive a call: kPoolSlabs of 512 KiB at most per device, shared by
-// every context and thread under a mutex, freed with the last context.  Pinning
+// The slabs outlive a call: eight of 512 KiB and eight of 128 KiB at most per
+// device, shared by every context and thread under a mutex, freed with the last
+// context.  Pinning
 // costs 0.5 ms a MiB, which a program that moves one field must win back, so the
 // slabs are small (of 2 MiB they save another 0.4 ms at 256^3 and cost 6 ms
 // once), and transfers within 128 KiB take smaller ones.
@@ -21,13 +22,13 @@
 #include <vector>
 
 #include "gh_ctx.h"
+#include "gh_slab_pool.h"
 
 namespace gh {
 namespace {
 
 constexpr size_t kSlabBytes = 512u << 10;
 constexpr size_t kSmallSlab = 128u << 10;
-constexpr size_t kPoolSlabs = 8;
 constexpr int kStageThreads = 4;
 constexpr size_t kThreadedBytes = 1u << 20;  // 60 us of copying; starting three threads takes 30
 
@@ -39,7 +40,7 @@ struct Slab {
 };
 
 std::mutex g_mu;
-std::vector<Slab> g_free;
+SlabPool<Slab> g_free;
 int g_users = 0;
 
 void drop(Slab& s) {
@@ -52,12 +53,7 @@ void drop(Slab& s) {
 int take(int device, size_t need, Slab& s) {
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        for (size_t i = 0; i < g_free.size(); ++i)
-            if (g_free[i].device == device && g_free[i].bytes >= need) {
-                s = g_free[i];
-                g_free.erase(g_free.begin() + i);
-                return GH_OK;
-            }
+        if (g_free.take(device, need, s)) return GH_OK;
     }
     s.device = device;
     s.bytes = need <= kSmallSlab ? kSmallSlab : kSlabBytes;
@@ -71,10 +67,7 @@ void give(Slab& s) {
     if (!s.p && !s.ev) return;
     try {
         std::lock_guard<std::mutex> lock(g_mu);
-        size_t mine = 0;
-        for (const Slab& f : g_free) mine += f.device == s.device;
-        if (s.p && s.ev && g_users > 0 && mine < kPoolSlabs) {
-            g_free.push_back(s);
+        if (s.p && s.ev && g_users > 0 && g_free.give(s)) {
             s = Slab{};
             return;
         }
@@ -109,9 +102,7 @@ struct Pair {
 // one field pays for no more, and the fourth transfer has its four threads.
 int threads_for(int device, size_t n) {
     std::lock_guard<std::mutex> lock(g_mu);
-    size_t ready = 0;
-    for (const Slab& f : g_free) ready += f.device == device && f.bytes == kSlabBytes;
-    return (int)std::min<size_t>({(size_t)kStageThreads, n, 1 + ready / 2});
+    return (int)std::min<size_t>({(size_t)kStageThreads, n, 1 + g_free.ready(device, kSlabBytes) / 2});
 }
 
 // Runs part(first, last) over the chunks of `bytes` on up to kStageThreads
@@ -240,7 +231,7 @@ void stage_release() {
     std::vector<Slab> gone;
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        if (--g_users == 0) gone.swap(g_free);
+        if (--g_users == 0) gone.swap(g_free.slabs);
     }
     for (Slab& s : gone) drop(s);
 }
