@@ -471,6 +471,14 @@ __global__ __launch_bounds__(256) void face_patch_table_kernel(const int32_t* __
     tab[(size_t)k * PATCH_STRIDE + patch_word(n, e)] = src;
 }
 
+// LDS from lane to lane of one wave, whose LDS operations are in order: the fences
+// keep the compiler from moving stores and loads across (they make no instruction)
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // the ghost (u, v) = (lane & 7, lane >> 3) of face f from its patch p of n
 // values: the taps z-major, then y, then x (ghost_visit's order); wave-uniform
 // f; a coarser neighbour's face
@@ -545,7 +553,7 @@ __global__ __launch_bounds__(256) void face_patch_kernel(int nf, const int32_t* 
         s_p[w][0][lane] = f0[src];
         s_p[w][1][lane] = f1[src];
     }
-    __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations are in order
+    wave_lds_order();
     out0[(size_t)sf * 64 + lane] = patch_ghost<Real, ORDER>(s_p[w][0], f, lane);
     out1[(size_t)sf * 64 + lane] = patch_ghost<Real, ORDER>(s_p[w][1], f, lane);
 }
@@ -1289,9 +1297,9 @@ __global__ __launch_bounds__(NT) void rd_step_patched_kernel(
             } else {
                 p[lane] = pv[c][0];  // (lanes past the patch: not used)
             }
-            __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations are in order
+            wave_lds_order();
             const Real g = patch_ghost<Real, ORDER>(p, f, lane);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();  // (the next face's patch goes to the same place)
             put(g, gt[c], gd[c], gd[c], gd[c]);
         }
     }
