@@ -400,6 +400,16 @@ int build_layout_t(Batch& b) {
     return GH_OK;
 }
 
+// the result of setting samples: after a failure there are none, for their buffers and
+// lists may be missing or of another layout
+int checked(Batch& b, int rc) {
+    if (rc) {
+        b.smp.clear();
+        b.ran = b.adjoint = false;
+    }
+    return rc;
+}
+
 // phi[0][idx] = val for the nonzero initial cells of every sample
 template <typename Real>
 int scatter_ic(Batch& b, const std::vector<uint64_t>& idx, const std::vector<Real>& val) {
@@ -1029,8 +1039,8 @@ int gh_batch_set_samples(gh_batch* bh, int nsamples, const int* anatomy_id, cons
     GH_HIP_CHECK(hipSetDevice(b->device));
     b->smp.assign(nsamples, BatchSample{});
     for (int i = 0; i < nsamples; ++i) b->smp[i].anat = anatomy_id[i];
-    return b->real_kind == GH_REAL_F32 ? set_samples_t<float>(*b, params, cfl)
-                                       : set_samples_t<double>(*b, params, cfl);
+    return checked(*b, b->real_kind == GH_REAL_F32 ? set_samples_t<float>(*b, params, cfl)
+                                                   : set_samples_t<double>(*b, params, cfl));
 }
 
 int gh_batch_run(gh_batch* bh, double* elapsed_ms) {
@@ -1071,8 +1081,8 @@ int gh_batch_set_adjoint_samples(gh_batch* bh, int nsamples, const int* anatomy_
     b->smp.assign(nsamples, BatchSample{});
     for (int i = 0; i < nsamples; ++i) b->smp[i].anat = anatomy_id[i];
     b->ic_is2 = 1.0 / (ic_sigma * ic_sigma);
-    return b->real_kind == GH_REAL_F32 ? set_adjoint_samples_t<float>(*b, params, nsteps, ic_sigma, ic_peak)
-                                       : set_adjoint_samples_t<double>(*b, params, nsteps, ic_sigma, ic_peak);
+    return checked(*b, b->real_kind == GH_REAL_F32 ? set_adjoint_samples_t<float>(*b, params, nsteps, ic_sigma, ic_peak)
+                                                   : set_adjoint_samples_t<double>(*b, params, nsteps, ic_sigma, ic_peak));
 }
 
 int gh_batch_adjoint(gh_batch* bh, int ckpt_every, const double* lik_params, int stepPET, int stepTi, int use_roi,
