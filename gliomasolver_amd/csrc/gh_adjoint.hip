@@ -130,8 +130,7 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     GH_HIP_CHECK(hipMemsetAsync(c.adjPart.p, 0, sizeof(double) * ADJ_PART * ns, c.stream));
     const double h = block_h_of(c);
     const double ih2 = 1. / (h * h);
-    const UniformAdjParams prm{c.rho, ih2, dt, 1.0 / (double)N, 1.0 / c.Dw, c.topo.uniform_bpd,
-                                bpd_magic(c.topo.uniform_bpd)};
+    const UniformAdjParams prm{c.rho, ih2, dt, c.topo.uniform_bpd, bpd_magic(c.topo.uniform_bpd)};
     // blocks without diffusion take the reverse step's short path under the
     // two-step schedule (tile 0); step 0 reads the caller's state and leaves
     // nothing out
@@ -171,7 +170,7 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
                        c.likPart.as<double>(), sums);
     GH_HIP_CHECK(hipGetLastError());
     GH_HIP_CHECK(hipStreamSynchronize(c.stream));
-    adj_param_grads(sums, prm.dt, prm.invDw, prm.invN, prm.rho, grad);
+    adj_param_grads(sums, dt, 1.0 / c.Dw, 1.0 / (double)N, c.rho, grad);
     for (int q = 0; q < 3; ++q) grad[3 + q] = sums[2 + q];
     return GH_OK;
 }

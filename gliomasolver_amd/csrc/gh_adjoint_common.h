@@ -48,7 +48,7 @@ __device__ inline double block_sum(double v, double* red) {
 
 // adj_step_kernel's parameters as plain arguments (StepArgs)
 struct AdjArgs {
-    double rho, ih2, dt, invN, invDw;
+    double rho, ih2, dt;
     int bpd;
     uint32_t magic;
     const int4* slots;
@@ -57,24 +57,22 @@ struct AdjArgs {
 
 // Per-slot parameters of the reverse step: one solve, or packed solves.
 struct UniformAdjParams {
-    double rho, ih2, dt, invN, invDw;
+    double rho, ih2, dt;
     int bpd;
     uint32_t magic;  // bpd_magic(bpd)
-    __host__ __device__ static inline UniformAdjParams make(double r, double i, double d, double n, double w, int b,
-                                                            uint32_t m, const int4*, const void*) {
-        return {r, i, d, n, w, b, m};
+    __host__ __device__ static inline UniformAdjParams make(double r, double i, double d, int b, uint32_t m, const int4*,
+                                                            const void*) {
+        return {r, i, d, b, m};
     }
-    AdjArgs args() const { return {rho, ih2, dt, invN, invDw, bpd, magic, nullptr, nullptr}; }
+    AdjArgs args() const { return {rho, ih2, dt, bpd, magic, nullptr, nullptr}; }
     using Item = int;
     __device__ static inline Item item(const int32_t* full, int i) { return full ? full[i] : i; }
     __device__ static inline Item item_of(int s) { return s; }
     __device__ static inline int slot(Item it) { return it; }
-    __device__ inline void get(int, double& r, double& i, double& d, double& n, double& w) const {
+    __device__ inline void get(int, double& r, double& i, double& d) const {
         r = rho;
         i = ih2;
         d = dt;
-        n = invN;
-        w = invDw;
     }
     __device__ inline BlockPos pos(int s) const { return block_pos(s, 0, bpd, magic); }
 };
@@ -89,11 +87,6 @@ template <bool CLAMPED, typename Real>
 __device__ inline bool adj_in_domain(Real u, const Stat4<Real>& r, const Real* sig, size_t g) {
     if (CLAMPED) return sign_of(r.tau) || u > (Real)0;
     return u > sig[g];
-}
-template <bool CLAMPED, typename Real>
-__device__ inline bool adj_outside(Real u, const Stat4<Real>& r) {
-    if (CLAMPED) return u < fabs(r.tau);
-    return u < r.tau;
 }
 
 // Face halo cell (a, b) of face f at depth d (1 or 2): the cell index in the
@@ -199,16 +192,15 @@ __global__ __launch_bounds__(512) void adj_step_kernel(
     const Stat4<Real>* __restrict__ st, int bpd, uint32_t magic, const int4* __restrict__ slots,
     const void* __restrict__ range, const double* __restrict__ lam1, double* __restrict__ lam0,
     const Real* __restrict__ sig, double* __restrict__ partial, int mask_out, double rho_, double ih2_, double dt_,
-    double invN_, double invDw_, int ngrp, int gper, const int2* __restrict__ grp,
-    const unsigned char* __restrict__ still) {
+    int ngrp, int gper, const int2* __restrict__ grp, const unsigned char* __restrict__ still) {
     const StepWork wk{nfull, fper, ngrp, gper, full, grp, still};
-    const Params prm = Params::make(rho_, ih2_, dt_, invN_, invDw_, bpd, magic, slots, range);
+    const Params prm = Params::make(rho_, ih2_, dt_, bpd, magic, slots, range);
     int nzf;
     typename Params::Item it;
     const int s = wk.item(prm, &nzf, it);
     if (s < 0) return;
-    double rho, ih2, dt, invN, invDw;
-    prm.get(it, rho, ih2, dt, invN, invDw);  // a group's blocks belong to one solve
+    double rho, ih2, dt;
+    prm.get(it, rho, ih2, dt);  // a group's blocks belong to one solve
     const int t = threadIdx.x;
     for (int b = 0; b < nzf; ++b) {  // uniform per workgroup
         const size_t g = (size_t)(s + b) * BCELLS + t;
@@ -339,7 +331,7 @@ inline void launch_adj_step(hipStream_t stream, const StepWork& wk, const Real* 
     const AdjArgs q = prm.args();
     hipLaunchKernelGGL((adj_step_kernel<Real, Params, CLAMPED>), dim3(wk.grid()), dim3(512), 0, stream, wk.nfull,
                        wk.fper, wk.full, uk, st, q.bpd, q.magic, q.slots, q.range, lam1, lam0, sig, partial,
-                       mask_out, q.rho, q.ih2, q.dt, q.invN, q.invDw, wk.ngrp, wk.gper, wk.grp, wk.still);
+                       mask_out, q.rho, q.ih2, q.dt, wk.ngrp, wk.gper, wk.grp, wk.still);
 }
 
 // sum over cells of lam0 * u0 * (X - x0) / sigma^2 for X = ix, iy, iz, by

@@ -54,7 +54,7 @@ struct SlotRange {
     size_t aslot0;   // the anatomy's first slot is at aslot0 in its own arrays (always 0)
     Real rho, Dw, Dg;
     double ih2, dt;
-    double rho_d, invN, invDw;  // adjoint: rho and 1/Dw as given, 1/N
+    double rho_d;               // adjoint: rho as given
     int bpd;                    // blocks per side of the sample's grid
     uint32_t magic;             // bpd_magic(bpd)
 };
@@ -70,18 +70,16 @@ struct BatchSample {
 template <typename Real>
 struct BatchAdjParams : PackedItems {
     const SlotRange<Real>* __restrict__ range;
-    __host__ __device__ static inline BatchAdjParams make(double, double, double, double, double, int, uint32_t,
-                                                          const int4* sl, const void* r) {
+    __host__ __device__ static inline BatchAdjParams make(double, double, double, int, uint32_t, const int4* sl,
+                                                          const void* r) {
         return {{sl}, (const SlotRange<Real>*)r};
     }
-    AdjArgs args() const { return {0., 0., 0., 0., 0., 0, 0u, slots, range}; }
-    __device__ inline void get(const Item& it, double& r, double& i, double& d, double& n, double& w) const {
+    AdjArgs args() const { return {0., 0., 0., 0, 0u, slots, range}; }
+    __device__ inline void get(const Item& it, double& r, double& i, double& d) const {
         const SlotRange<Real>& q = range[it.w];
         r = q.rho_d;
         i = q.ih2;
         d = q.dt;
-        n = q.invN;
-        w = q.invDw;
     }
 };
 
@@ -336,8 +334,6 @@ int build_layout_t(Batch& b) {
         rng[p].ih2 = 1. / ((double)hr * (double)hr);
         rng[p].dt = q.dt;
         rng[p].rho_d = q.rho;
-        rng[p].invN = 1.0 / (double)q.nsteps;
-        rng[p].invDw = 1.0 / q.Dw;
         rng[p].bpd = a.bpd;
         rng[p].magic = bpd_magic(a.bpd);
         apw[p] = a.pw.p;
