@@ -51,8 +51,9 @@ struct DevBuf {
 // interval asks for `need` bytes; up to `want` (the whole trajectory) are taken
 // beyond it, since the states on the tape need no second solve on the way back, a
 // quarter of a gradient's launches.  What is taken beyond `need` is at most an
-// eighth of what is free, and over all contexts and batches of the process an eighth
-// of the device's memory: more of them do with shorter tapes.  It is kept between
+// eighth of what is free, and over all contexts and batches of the process a quarter
+// of the device's memory; past it they do with shorter tapes (with an eighth in all,
+// the third of three batches of 17 GB each recomputed, 5 % of the three).  It is kept between
 // calls (taking freed memory again waits until it has been cleared: a gradient of
 // 1,001 steps of 128^3 FP32 took 127 instead of 11 ms) until release().
 struct TapeBuf {

@@ -43,7 +43,7 @@ void DevBuf::release() {
 }
 
 namespace {
-constexpr int kTapeShare = 8;  // of the device's memory (TapeBuf)
+constexpr int kTapeFree = 8, kTapeAll = 4;  // a tape's share of free memory, all tapes' of the device's (TapeBuf)
 struct TapeSum {
     size_t total = 0;  // the device's memory
     size_t extra = 0;  // the sum over its tapes
@@ -68,8 +68,8 @@ int TapeBuf::ensure(int device, size_t need, size_t want) {
         if (held >= want) room = sum.total;  // (nothing more is taken)
         dev = device;
         sum.extra -= extra;
-        const size_t share = sum.total / kTapeShare, left = share > sum.extra ? share - sum.extra : 0;
-        take = std::min({want, need + left, std::max(need, (room + held) / kTapeShare)});
+        const size_t share = sum.total / kTapeAll, left = share > sum.extra ? share - sum.extra : 0;
+        take = std::min({want, need + left, std::max(need, (room + held) / kTapeFree)});
         // (a tape short of the whole trajectory is not given up for one little longer)
         if (held >= need && held <= need + left && (held >= want || take <= held + held / 4)) take = held;
         extra = take - need;

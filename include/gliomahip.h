@@ -250,7 +250,7 @@ int gh_likelihood_noalloc(gh_ctx* ctx, const double* params, int stepPET, int st
  * checkpoints, a tape's length at a time.  The tape is longer, up to the whole
  * trajectory, while what it takes beyond ckpt_every + 1 states is within an
  * eighth of the device's free memory and, over all contexts and batches of the
- * process, within an eighth of the device's memory.  The result does not depend
+ * process, within a quarter of the device's memory.  The result does not depend
  * on the length.  The context keeps it until gh_adjoint_release or
  * gh_ctx_destroy.  The no-flux flags, the in-domain test and the upper clamp are frozen along the
  * trajectory; the lower clamp is treated as inactive.
