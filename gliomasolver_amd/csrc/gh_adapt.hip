@@ -1777,10 +1777,11 @@ int prepare_ghosted_t(Ctx& c, double Dw, double Dg) {
 }
 
 // Largest FP32 grid whose patched step has 512 lanes a block; above it 256 lanes
-// of two cells (more blocks in flight a CU): 500 / 3,816 / 9,500 blocks 5.4 /
-// 14.8 / 32.1 us with 512, 6.2 / 14.2 / 28.6 us with 256.  In FP64 512 is the
+// of two cells (more blocks in flight a CU).  us a step with 512 / with 256 lanes:
+// 477 blocks 4.8 / 6.2, 960 5.6 / 6.8, 1,408 7.1 / 7.2, 1,912 9.0 / 8.8, 2,248 10.9 /
+// 10.5, 3,816 14.4 / 13.9, 6,336 21.8 / 19.4, 9,136 27.8 / 24.3.  In FP64 512 is the
 // faster at every size measured (3,816 blocks: 21.2 and 22.9 us).
-constexpr int kPatchedFewBlocks = 2500;
+constexpr int kPatchedFewBlocks = 1600;
 constexpr int kFusedGhostMaxBlocks = 1450;  // largest grid whose step kernel gathers its own ghosts
 
 // The step kernel with 512 lanes per block when it gathers the face ghosts
