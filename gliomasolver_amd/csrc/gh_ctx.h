@@ -197,9 +197,13 @@ struct Ctx {
     double Dw = 0, Dg = 0, rho = 0;
     double dt_last = 0;  // dt of the running gh_rd_steps call
     // schedule of gh_rd_set_tile: blocks per workgroup of the step kernel (1, 2
-    // or 4, one step per launch) or 0, two steps per launch -- the faster one at
-    // every size (us per step, 2 vs 0: 32^3 FP32 4.1 / 2.3, 64^3 FP64 4.7 / 2.8,
-    // 128^3 FP32 12.7 / 3.2)
+    // or 4, one step per launch) or 0, two steps per launch -- on clamped states the
+    // faster one at every size (us per step, one and two a launch: 32^3 FP32 3.8 /
+    // 1.8, 64^3 FP64 4.8 / 2.2, 128^3 FP32 10.1 / 4.1, 256^3 FP32 76 / 20).  Calls of
+    // exactly two steps, and anatomies with p_w + p_g < 0, take rd_step2_kernel under
+    // 0: faster on small grids (two steps at 32^3 4.4 / 7.1 us) and where most blocks
+    // hold tissue (256^3 FP32 177 / 209), slower on large ones that are mostly empty
+    // (153 against 177, FP64 297 against 355)
     int rd_bpw = 0;
 
     size_t ncells() const { return (size_t)topo.nblocks() * BCELLS; }

@@ -862,7 +862,10 @@ __device__ inline int mad24(int a, int b, int c) { return (int)__umul24((unsigne
 // planes and two roles each, 14 % fewer vector instructions per block, a pair of
 // steps takes as long at 256^3 (27.5 us) and longer at 128^3 (6.6 -> 7.3 us):
 // the loads and barriers of a block bound it.  TWO = false: one step only (no
-// edges, no depth-2 halo), 18 instead of 73 us for 41,000 slots.
+// edges, no depth-2 halo); FP32 with still groups left out, against
+// rd_step_kernel, which runs every block: 128^3 (1,572 of 4,096 blocks move) 5.4
+// and 11.8 us, 256^3 (11,635 of 32,768) 29.5 and 82.9, 24 samples of 96^3 29.6
+// and 104.8.
 template <typename Real, typename Params, bool DOM, bool TWO>
 __global__ __launch_bounds__(512) void rd_step2f_kernel(
     int nfull, int fper, const int32_t* __restrict__ full, const Real* __restrict__ phi,

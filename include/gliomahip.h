@@ -233,8 +233,8 @@ int gh_likelihood_dense(gh_ctx* ctx, int nx, int ny, int nz, const double* model
  *   callers that cannot allocate device memory (code under HIP graph capture,
  *   tight sampling loops, harnesses that forbid hipMalloc): same arguments,
  *   same result bit for bit, but the per-workgroup partials live in a
- *   file-scope device array of 4 * (1024 + 1) doubles (32.8 KB per GPU, held
- *   until the process ends) instead of a context buffer, and the call makes no
+ *   file-scope device array of 4 * 1024 doubles (32.8 KB per GPU, held until
+ *   the process ends) instead of a context buffer, and the call makes no
  *   hipMalloc/hipFree.  The partition is fixed at 1,024 workgroups for every
  *   grid size, so no input exceeds the array.  The array is shared by every
  *   context on a GPU: calls that overlap on one GPU (two threads, two
