@@ -51,18 +51,11 @@ int adjoint_t(Ctx& c, int64_t N, double T, int K, const double* lik, int stepPET
     if ((rc = c.adjLam[0].ensure(nc * 8)) || (rc = c.adjLam[1].ensure(nc * 8)) ||
         (rc = c.adjPart.ensure(sizeof(double) * ADJ_PART * ns)))
         return rc;
-    // segments of `len` steps, the first one shorter; the last stays on the tape.  Where
-    // its length beyond K leaves no room for the checkpoints, K it is
-    const size_t need = ((size_t)std::min<int64_t>(K, N) + 1) * nb;
-    int64_t len = 0, nseg = 0;
-    for (size_t want = ((size_t)N + 1) * nb;; want = need) {
-        if ((rc = c.adjSeg.ensure(c.device, need, want))) return rc;
-        len = std::min<int64_t>(N, (int64_t)(c.adjSeg.buf.bytes / nb) - 1);
-        nseg = (N + len - 1) / len;
-        rc = c.adjCk.ensure(std::max<size_t>(1, (size_t)(nseg - 1)) * nb);
-        if (rc == GH_OK) break;
-        if (want == need) return rc;
-    }
+    if ((rc = c.adjSeg.ensure(c.device, ((size_t)std::min<int64_t>(K, N) + 1) * nb, ((size_t)N + 1) * nb))) return rc;
+    // segments of `len` steps, the first one shorter; the last stays on the tape
+    const int64_t len = std::min<int64_t>(N, (int64_t)(c.adjSeg.buf.bytes / nb) - 1);
+    const int64_t nseg = (N + len - 1) / len;
+    if ((rc = c.adjCk.ensure(std::max<size_t>(1, (size_t)(nseg - 1)) * nb))) return rc;
     auto start = [&](int64_t i) { return i == 0 ? (int64_t)0 : N - (nseg - i) * len; };
     const double dt = T / (double)N;
     char* ck = (char*)c.adjCk.p;

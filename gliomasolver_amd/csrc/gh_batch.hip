@@ -692,33 +692,24 @@ int adjoint_t(Batch& b, int K, const double* lik, int stepPET, int stepTi, int u
         (rc = b.icpart.ensure((size_t)ns * (3 * ADJ_IC_GRID + ADJ_SUMS) * 8)) ||
         (rc = b.adjJobs.ensure(ns * sizeof(AdjJob<Real>))))
         return rc;
-    // segments [start[i], start[i + 1]) of steps, as long as the tape takes; where its
-    // length beyond K leaves no room for the checkpoints, K it is
-    const size_t all = cum(Nmax + 1) * slot_bytes,
-                 need = std::min((size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes, all);
-    std::vector<int64_t> start;
-    std::vector<size_t> ckoff;
-    int nseg = 0;
-    for (size_t want = all;; want = need) {
-        if ((rc = b.tape.ensure(b.device, need, want))) return rc;
-        start.assign(1, Nmax);
-        for (int64_t e = Nmax; e > 0;) {
-            int64_t lo = 0, hi = e - 1;  // (one step always fits)
-            while (lo < hi) {
-                const int64_t s = (lo + hi) / 2;
-                if ((cum(e + 1) - cum(s)) * slot_bytes <= b.tape.buf.bytes) hi = s;
-                else lo = s + 1;
-            }
-            start.push_back(e = hi);
+    const size_t all = cum(Nmax + 1) * slot_bytes;
+    if ((rc = b.tape.ensure(b.device, (size_t)(std::min<int64_t>(K, Nmax) + 1) * nsl * slot_bytes, all))) return rc;
+    // segments [start[i], start[i + 1]) of steps, as long as the tape takes
+    std::vector<int64_t> start{Nmax};
+    for (int64_t e = Nmax; e > 0;) {
+        int64_t lo = 0, hi = e - 1;  // (one step always fits)
+        while (lo < hi) {
+            const int64_t s = (lo + hi) / 2;
+            if ((cum(e + 1) - cum(s)) * slot_bytes <= b.tape.buf.bytes) hi = s;
+            else lo = s + 1;
         }
-        std::reverse(start.begin(), start.end());
-        nseg = (int)start.size() - 1;
-        ckoff.assign(nseg, 0);
-        for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
-        rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes);
-        if (rc == GH_OK) break;
-        if (want == need) return rc;
+        start.push_back(e = hi);
     }
+    std::reverse(start.begin(), start.end());
+    const int nseg = (int)start.size() - 1;
+    std::vector<size_t> ckoff(nseg, 0);
+    for (int i = 1; i < nseg; ++i) ckoff[i] = ckoff[i - 1] + b.slot0[active(start[i - 1])];
+    if ((rc = b.ck.ensure(std::max<size_t>(1, ckoff[nseg - 1]) * slot_bytes))) return rc;
     const BatchStepParams<Real> fprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     const BatchAdjParams<Real> aprm{{b.slotItem.as<int4>()}, b.range.as<SlotRange<Real>>()};
     char* ck = (char*)b.ck.p;
